@@ -2,7 +2,8 @@
 // the 2D cloud map (RG8: Perlin-FBM coverage, Worley-FBM type), the 3D detail
 // volume (R8 Perlin-Worley), the 3D Worley detail volume (R8 Worley-FBM) and the 2D
 // displacement map (RGBA8 Perlin-FBM),
-// plus the box-filter mip chain builder.  One lane per texel.  Hashes are
+// plus the box-filter mip chain builder.  One lane per texel, workgroups over tiles of texels that
+// share their octaves' hashes.  Hashes are
 // exact uint32 arithmetic; FBM sums run in FP32 as in the shader.
 #include <hip/hip_fp16.h>
 
@@ -19,68 +20,196 @@ __device__ __forceinline__ uint32_t wang_hash(uint32_t seed) {
     return seed;
 }
 
-// Gradient table of Noise.glsl:17-22, packed as 2-bit signed triples.
-__device__ __forceinline__ float perlin_grad_dot(uint32_t h, float x, float y, float z) {
-    constexpr int8_t g[16][3] = {{1, 1, 0},  {-1, 1, 0}, {1, -1, 0}, {-1, -1, 0}, {1, 0, 1},  {-1, 0, 1},
-                                 {1, 0, -1}, {-1, 0, -1}, {0, 1, 1}, {0, -1, 1},  {0, 1, -1}, {0, -1, -1},
-                                 {1, 1, 0},  {-1, 1, 0},  {0, -1, 1}, {0, -1, -1}};
-    int i = int(h & 15u);
-    return float(g[i][0]) * x + float(g[i][1]) * y + float(g[i][2]) * z;
+// A gradient of Noise.glsl:17-22 dotted with (x, y, z).  The table's 16 entries are 12 distinct
+// gradients, +-u +-v with (u, v) = (x, y) for 0..3, (x, z) for 4..7 and (y, z) for 8..11, the signs
+// in bits 0 and 1; entries 12..15 repeat 0, 1, 9 and 11 (perlin_gradient).
+__device__ __forceinline__ uint32_t perlin_gradient(uint32_t h) {
+    const uint32_t i = h & 15u;
+    return i < 12u ? i : (0xb910u >> (4u * (i - 12u))) & 15u;
+}
+__device__ __forceinline__ float perlin_grad_dot(uint32_t g, float x, float y, float z) {
+    const float u = g < 8u ? x : y, v = g < 4u ? y : z;
+    return __uint_as_float(__float_as_uint(u) ^ (g << 31)) + __uint_as_float(__float_as_uint(v) ^ ((g & 2u) << 30));
 }
 
 __device__ __forceinline__ float gmixf(float a, float b, float t) { return a * (1.0f - t) + b * t; }
 
-// PerlinNoise, Noise.glsl:28-60 (p >= 0 here: texture coordinates in [0, 1)).
-__device__ inline float perlin_noise(float px, float py, float pz, uint32_t freq, uint32_t seed) {
-    px *= float(freq);
-    py *= float(freq);
-    pz *= float(freq);
-    float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
-    uint32_t i0 = uint32_t(int(fx)) % freq, j0 = uint32_t(int(fy)) % freq, k0 = uint32_t(int(fz)) % freq;
-    uint32_t i1 = uint32_t(int(ceilf(px))) % freq, j1 = uint32_t(int(ceilf(py))) % freq,
-             k1 = uint32_t(int(ceilf(pz))) % freq;
-    float tx = px - fx, ty = py - fy, tz = pz - fz;
-    float u = tx * tx * tx * (tx * (tx * 6.0f - 15.0f) + 10.0f);
-    float v = ty * ty * ty * (ty * (ty * 6.0f - 15.0f) + 10.0f);
-    float w = tz * tz * tz * (tz * (tz * 6.0f - 15.0f) + 10.0f);
-    // GetPerlinGradients(i, j, k) = table[WangHash(seed + WangHash(i + WangHash(j + WangHash(k))))]
-    uint32_t hk0 = wang_hash(k0), hk1 = wang_hash(k1);
-    uint32_t hj0k0 = wang_hash(j0 + hk0), hj1k0 = wang_hash(j1 + hk0), hj0k1 = wang_hash(j0 + hk1),
-             hj1k1 = wang_hash(j1 + hk1);
-    auto G = [&](uint32_t i, uint32_t hjk) { return wang_hash(seed + wang_hash(i + hjk)); };
-    float x1 = tx - 1.0f, y1 = ty - 1.0f, z1 = tz - 1.0f;
-    float n000 = perlin_grad_dot(G(i0, hj0k0), tx, ty, tz), n100 = perlin_grad_dot(G(i1, hj0k0), x1, ty, tz);
-    float n010 = perlin_grad_dot(G(i0, hj1k0), tx, y1, tz), n110 = perlin_grad_dot(G(i1, hj1k0), x1, y1, tz);
-    float n001 = perlin_grad_dot(G(i0, hj0k1), tx, ty, z1), n101 = perlin_grad_dot(G(i1, hj0k1), x1, ty, z1);
-    float n011 = perlin_grad_dot(G(i0, hj1k1), tx, y1, z1), n111 = perlin_grad_dot(G(i1, hj1k1), x1, y1, z1);
+// ---------------------------------------------------------------------------
+// Octaves by tile.  A workgroup covers a TX x TY x TZ tile of texels, and an octave's hashes depend
+// on lattice cells, which neighbouring texels share: the tile's cells are hashed once into LDS and
+// the texels read them there.  The reference's chains are H(seed + H(x + H(y + H(z)))), so their
+// (y, z) parts are a table of their own (`hash`), filled first; where the whole cell table does not
+// fit (an octave finer than the texels, whose texels share no cells) the texels finish the chain from
+// the (y, z) table, and where that does not fit either they hash for themselves.
+// Bound by the integer hashes (a 3D Worley octave is 198 per texel without sharing, each about 10
+// instructions with a quarter-rate multiply).  Same hashes and float operations as the reference's
+// texel-by-texel form, so the same bytes.  Measured: detail 128^3 1,090 -> 520 us (its two finest
+// octaves, whose texels share no cells, are half of what is left), cloud map 512^2 130 -> 59 us,
+// Worley 32^3 35 -> 28 us; all textures of the default material 1,331 -> 665 us.
+// The tables hold 1,024 columns and 1,536 cells (30 KiB, five workgroups per CU): a 256-texel tile
+// of a 128^3 volume fits them up to one octave beyond the texels' own density, past which filling the
+// table would hash as many cells as the texels do themselves.
+// ---------------------------------------------------------------------------
+constexpr int kMaxPairs = 1024;   // (y, z) columns of a tile's cells
+constexpr int kMaxCells = 1536;
+struct NoiseLds {
+    uint32_t hash[3][kMaxPairs];
+    float cell[3][kMaxCells];  // Worley feature points; Perlin keeps its gradients in cell[0]
+};
+
+// One octave's cells over the tile along each axis: base[a] + [0, n[a]), from the cell coordinates
+// of the tile's first and last texels (the texels' own float operations, monotonic in the texel).
+struct CellRange {
+    uint32_t base[3], n[3];
+    bool pairs, cells;
+};
+struct NoiseTile {
+    float lo[3], hi[3];  // coordinates of the tile's first and last texel
+    float p[3];          // this thread's texel
+};
+
+__device__ __forceinline__ CellRange cell_range(const NoiseTile& t, uint32_t freq, uint32_t extra) {
+    CellRange r;
+    for (int a = 0; a < 3; ++a) {
+        r.base[a] = uint32_t(floorf(t.lo[a] * float(freq)));
+        r.n[a] = uint32_t(floorf(t.hi[a] * float(freq))) - r.base[a] + extra;
+    }
+    r.pairs = r.n[1] <= uint32_t(kMaxPairs) && r.n[2] <= uint32_t(kMaxPairs) && r.n[1] * r.n[2] <= uint32_t(kMaxPairs);
+    r.cells = r.pairs && r.n[0] <= uint32_t(kMaxCells) && r.n[0] * r.n[1] * r.n[2] <= uint32_t(kMaxCells);
+    return r;
+}
+
+// v % freq for v < 3 freq (a division below frequency 4, where v can be larger).
+__device__ __forceinline__ uint32_t wrap_cell(uint32_t v, uint32_t freq) {
+    if (freq < 4u) return v % freq;
+    if (v >= freq) v -= freq;
+    return v >= freq ? v - freq : v;
+}
+
+// PerlinNoise, Noise.glsl:28-60 (p >= 0 here: texture coordinates in [0, 1)).  The far corner is
+// cell + 1 where the reference takes ceil: they differ only at integer coordinates, where the
+// corner's weight is 0.
+template <int kThreads>
+__device__ inline float perlin_octave(NoiseLds& s, const NoiseTile& t, uint32_t freq, uint32_t seed) {
+    const CellRange r = cell_range(t, freq, 2u);
+    uint8_t* grad = reinterpret_cast<uint8_t*>(s.cell[0]);
+    if (r.pairs) {
+        __syncthreads();  // the previous octave's reads
+        for (uint32_t k = threadIdx.x; k < r.n[1] * r.n[2]; k += kThreads) {
+            const uint32_t cz = k / r.n[1], cy = k - cz * r.n[1];
+            s.hash[0][k] = wang_hash(wrap_cell(r.base[1] + cy, freq) + wang_hash(wrap_cell(r.base[2] + cz, freq)));
+        }
+        __syncthreads();
+    }
+    if (r.cells) {
+        for (uint32_t k = threadIdx.x; k < r.n[0] * r.n[1] * r.n[2]; k += kThreads) {
+            const uint32_t pair = k / r.n[0], cx = k - pair * r.n[0];
+            grad[k] = uint8_t(perlin_gradient(
+                wang_hash(seed + wang_hash(wrap_cell(r.base[0] + cx, freq) + s.hash[0][pair]))));
+        }
+        __syncthreads();
+    }
+    const float px = t.p[0] * float(freq), py = t.p[1] * float(freq), pz = t.p[2] * float(freq);
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const float tx = px - fx, ty = py - fy, tz = pz - fz;
+    uint32_t g[8];  // corner x + 2 y + 4 z
+    const uint32_t ix = uint32_t(int(fx)), iy = uint32_t(int(fy)), iz = uint32_t(int(fz));
+    if (r.cells) {
+        const uint32_t at = ((iz - r.base[2]) * r.n[1] + (iy - r.base[1])) * r.n[0] + (ix - r.base[0]);
+        const uint32_t sy = r.n[0], sz = r.n[0] * r.n[1];
+        for (uint32_t c = 0; c < 8; ++c) g[c] = grad[at + (c & 1u) + ((c >> 1) & 1u) * sy + (c >> 2) * sz];
+    } else {
+        const uint32_t x0 = wrap_cell(ix, freq), x1 = wrap_cell(ix + 1u, freq);
+        const uint32_t at = (iz - r.base[2]) * r.n[1] + (iy - r.base[1]);
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint32_t hjk = r.pairs ? s.hash[0][at + (c & 1u) + (c >> 1) * r.n[1]]
+                                         : wang_hash(wrap_cell(iy + (c & 1u), freq) +
+                                                     wang_hash(wrap_cell(iz + (c >> 1), freq)));
+            g[2 * c] = perlin_gradient(wang_hash(seed + wang_hash(x0 + hjk)));
+            g[2 * c + 1] = perlin_gradient(wang_hash(seed + wang_hash(x1 + hjk)));
+        }
+    }
+    const float u = tx * tx * tx * (tx * (tx * 6.0f - 15.0f) + 10.0f);
+    const float v = ty * ty * ty * (ty * (ty * 6.0f - 15.0f) + 10.0f);
+    const float w = tz * tz * tz * (tz * (tz * 6.0f - 15.0f) + 10.0f);
+    const float x1 = tx - 1.0f, y1 = ty - 1.0f, z1 = tz - 1.0f;
+    const float n000 = perlin_grad_dot(g[0], tx, ty, tz), n100 = perlin_grad_dot(g[1], x1, ty, tz);
+    const float n010 = perlin_grad_dot(g[2], tx, y1, tz), n110 = perlin_grad_dot(g[3], x1, y1, tz);
+    const float n001 = perlin_grad_dot(g[4], tx, ty, z1), n101 = perlin_grad_dot(g[5], x1, ty, z1);
+    const float n011 = perlin_grad_dot(g[6], tx, y1, z1), n111 = perlin_grad_dot(g[7], x1, y1, z1);
     return gmixf(gmixf(gmixf(n000, n100, u), gmixf(n010, n110, u), v),
                  gmixf(gmixf(n001, n101, u), gmixf(n011, n111, u), v), w);
 }
 
-// WorleyNoise (3D), Noise.glsl:81-101.
-__device__ inline float worley_noise(float px, float py, float pz, uint32_t freq, uint32_t seed) {
-    px *= float(freq);
-    py *= float(freq);
-    pz *= float(freq);
-    uint32_t ix = uint32_t(floorf(px)), iy = uint32_t(floorf(py)), iz = uint32_t(floorf(pz));
+// The reference's random float of a hash.
+__device__ __forceinline__ float hash_to_unit(uint32_t h) { return float(h) * 2.3283064365386963e-10f; }
+
+// WorleyNoise (3D), Noise.glsl:81-101: the nearest feature point of the 27 cells around p, shifted
+// up by one period as the reference shifts it (the feature point of cell g is g + a fraction).
+template <int kThreads>
+__device__ inline float worley_octave(NoiseLds& s, const NoiseTile& t, uint32_t freq, uint32_t seed) {
+    const CellRange r = cell_range(t, freq, 3u);  // cells base - 1 .. of the shifted coordinates
+    const uint32_t off = freq - 1u;
+    if (r.pairs) {
+        __syncthreads();  // the previous octave's reads
+        for (uint32_t k = threadIdx.x; k < r.n[1] * r.n[2]; k += kThreads) {
+            const uint32_t cz = k / r.n[1], cy = k - cz * r.n[1];
+            const uint32_t sz = wrap_cell(r.base[2] + off + cz, freq), sy = wrap_cell(r.base[1] + off + cy, freq);
+            for (uint32_t c = 0; c < 3; ++c) s.hash[c][k] = wang_hash(sy + wang_hash(sz + c));
+        }
+        __syncthreads();
+    }
+    if (r.cells) {
+        for (uint32_t k = threadIdx.x; k < r.n[0] * r.n[1] * r.n[2]; k += kThreads) {
+            const uint32_t pair = k / r.n[0], cx = k - pair * r.n[0];
+            const uint32_t sx = wrap_cell(r.base[0] + off + cx, freq);
+            for (uint32_t c = 0; c < 3; ++c)
+                s.cell[c][k] = hash_to_unit(wang_hash(seed + wang_hash(sx + s.hash[c][pair])));
+        }
+        __syncthreads();
+    }
+    float px = t.p[0] * float(freq), py = t.p[1] * float(freq), pz = t.p[2] * float(freq);
+    const uint32_t ix = uint32_t(floorf(px)), iy = uint32_t(floorf(py)), iz = uint32_t(floorf(pz));
     px += float(freq);
     py += float(freq);
     pz += float(freq);
+    const uint32_t lx = ix - r.base[0], ly = iy - r.base[1], lz = iz - r.base[2];
     float min_d2 = 1e20f;
+    if (r.cells) {
+        const uint32_t at0 = (lz * r.n[1] + ly) * r.n[0] + lx;
+#pragma unroll
+        for (uint32_t dk = 0; dk < 3; ++dk)
+#pragma unroll
+            for (uint32_t dj = 0; dj < 3; ++dj) {
+                const uint32_t at = at0 + (dk * r.n[1] + dj) * r.n[0];
+#pragma unroll
+                for (uint32_t di = 0; di < 3; ++di) {
+                    const float dx = px - (float(ix + off + di) + s.cell[0][at + di]);
+                    const float dy = py - (float(iy + off + dj) + s.cell[1][at + di]);
+                    const float dz = pz - (float(iz + off + dk) + s.cell[2][at + di]);
+                    min_d2 = fminf(min_d2, dx * dx + dy * dy + dz * dz);
+                }
+            }
+        return sqrtf(min_d2);
+    }
+    uint32_t sx[3];
+    for (uint32_t di = 0; di < 3; ++di) sx[di] = wrap_cell(ix + off + di, freq);
     for (uint32_t dk = 0; dk < 3; ++dk) {
-        uint32_t gz = iz + freq - 1 + dk, sz = gz % freq;
-        uint32_t hz0 = wang_hash(sz), hz1 = wang_hash(sz + 1), hz2 = wang_hash(sz + 2);
+        const uint32_t sz = wrap_cell(iz + off + dk, freq);
         for (uint32_t dj = 0; dj < 3; ++dj) {
-            uint32_t gy = iy + freq - 1 + dj, sy = gy % freq;
-            uint32_t hy0 = wang_hash(sy + hz0), hy1 = wang_hash(sy + hz1), hy2 = wang_hash(sy + hz2);
+            uint32_t hy[3];
+            if (r.pairs) {
+                const uint32_t at = (lz + dk) * r.n[1] + ly + dj;
+                for (int c = 0; c < 3; ++c) hy[c] = s.hash[c][at];
+            } else {
+                const uint32_t sy = wrap_cell(iy + off + dj, freq);
+                for (uint32_t c = 0; c < 3; ++c) hy[c] = wang_hash(sy + wang_hash(sz + c));
+            }
+#pragma unroll
             for (uint32_t di = 0; di < 3; ++di) {
-                uint32_t gx = ix + freq - 1 + di, sx = gx % freq;
-                uint32_t r0 = wang_hash(seed + wang_hash(sx + hy0));
-                uint32_t r1 = wang_hash(seed + wang_hash(sx + hy1));
-                uint32_t r2 = wang_hash(seed + wang_hash(sx + hy2));
-                float dx = px - (float(gx) + float(r0) * 2.3283064365386963e-10f);
-                float dy = py - (float(gy) + float(r1) * 2.3283064365386963e-10f);
-                float dz = pz - (float(gz) + float(r2) * 2.3283064365386963e-10f);
+                const float dx = px - (float(ix + off + di) + hash_to_unit(wang_hash(seed + wang_hash(sx[di] + hy[0]))));
+                const float dy = py - (float(iy + off + dj) + hash_to_unit(wang_hash(seed + wang_hash(sx[di] + hy[1]))));
+                const float dz = pz - (float(iz + off + dk) + hash_to_unit(wang_hash(seed + wang_hash(sx[di] + hy[2]))));
                 min_d2 = fminf(min_d2, dx * dx + dy * dy + dz * dz);
             }
         }
@@ -92,12 +221,13 @@ __device__ __forceinline__ float remap_to01(float x, float x0, float x1) {
     return fminf(fmaxf((x - x0) / (x1 - x0), 0.0f), 1.0f);
 }
 
-// PerlinFBM / WorleyFBM, NoiseGen.comp:20-50 (8 octaves).
-__device__ inline float perlin_fbm(float x, float y, float z, SkyhipNoiseCreateInfo ci) {
+// PerlinFBM / WorleyFBM, NoiseGen.comp:20-50 (8 octaves).  Every thread of the workgroup calls them.
+template <int kThreads>
+__device__ inline float perlin_fbm(NoiseLds& s, const NoiseTile& t, const SkyhipNoiseCreateInfo& ci) {
     float res = 0.0f, a = 0.5f, sum_a = 0.0f;
     uint32_t f = ci.base_frequency;
     for (int c = 0; c < 8; ++c) {
-        float n = perlin_noise(x, y, z, f, ci.seed) * 0.5f + 0.5f;
+        float n = perlin_octave<kThreads>(s, t, f, ci.seed) * 0.5f + 0.5f;
         res += remap_to01(n, ci.remap_min, ci.remap_max) * a;
         sum_a += a;
         f *= 2u;
@@ -105,11 +235,12 @@ __device__ inline float perlin_fbm(float x, float y, float z, SkyhipNoiseCreateI
     }
     return res / sum_a;
 }
-__device__ inline float worley_fbm(float x, float y, float z, SkyhipNoiseCreateInfo ci) {
+template <int kThreads>
+__device__ inline float worley_fbm(NoiseLds& s, const NoiseTile& t, const SkyhipNoiseCreateInfo& ci) {
     float res = 0.0f, a = 0.5f, sum_a = 0.0f;
     uint32_t f = ci.base_frequency;
     for (int c = 0; c < 8; ++c) {
-        float n = worley_noise(x, y, z, f, ci.seed);
+        float n = worley_octave<kThreads>(s, t, f, ci.seed);
         res += remap_to01(n, ci.remap_min, ci.remap_max) * a;
         sum_a += a;
         f *= 2u;
@@ -122,53 +253,86 @@ __device__ __forceinline__ uint8_t to_unorm8(float f) {
     return uint8_t(floorf(fminf(fmaxf(f, 0.0f), 1.0f) * 255.0f + 0.5f));
 }
 
+// The tile of a workgroup of TX x TY x TZ threads, x fastest, at `tile` tiles of a dims-sized texture,
+// and this thread's texel.  Threads past the edge take the coordinates of the last texel (they still
+// hash and synchronise) and store nothing.  Coordinates are texel centres; an axis of size 0 is the
+// plane 0 of a 2D texture.
+struct TexelPos {
+    int x, y, z;
+    bool in;
+};
+template <int TX, int TY, int TZ>
+__device__ inline TexelPos noise_tile(int tx, int ty, int tz, const int dims[3], NoiseTile& t) {
+    const int id = threadIdx.x;
+    const int first[3] = {tx * TX, ty * TY, tz * TZ}, edge[3] = {TX, TY, TZ};
+    const int at[3] = {first[0] + id % TX, first[1] + (id / TX) % TY, first[2] + id / (TX * TY)};
+    TexelPos p{at[0], at[1], at[2], true};
+    for (int a = 0; a < 3; ++a) {
+        if (dims[a] == 0) {
+            t.lo[a] = t.hi[a] = t.p[a] = 0.0f;
+            continue;
+        }
+        const int last = min(first[a] + edge[a], dims[a]) - 1;
+        t.lo[a] = (float(first[a]) + 0.5f) / float(dims[a]);
+        t.hi[a] = (float(last) + 0.5f) / float(dims[a]);
+        t.p[a] = (float(min(at[a], last)) + 0.5f) / float(dims[a]);
+        p.in = p.in && at[a] < dims[a];
+    }
+    return p;
+}
+
+// Tiles of 256 texels: 16 x 16 of an image, 8 x 8 x 4 of a volume.
+constexpr int kImageTile = 16, kVolumeTileXY = 8, kVolumeTileZ = 4;
+__device__ inline TexelPos image_tile(int size, NoiseTile& t) {
+    const int dims[3] = {size, size, 0};
+    return noise_tile<kImageTile, kImageTile, 1>(blockIdx.x, blockIdx.y, 0, dims, t);
+}
+__device__ inline TexelPos volume_tile(int nx, int ny, int nz, NoiseTile& t) {
+    const int dims[3] = {nx, ny, nz};
+    return noise_tile<kVolumeTileXY, kVolumeTileXY, kVolumeTileZ>(blockIdx.x, blockIdx.y, blockIdx.z, dims, t);
+}
+
+// The image kernels give each channel its own workgroups (blockIdx.z): an image has few tiles, and a
+// tile's octaves follow one another through barriers.  128^2 displacement: 13.6 us, 47.8 with a tile's
+// four channels in one workgroup (17.5 with every texel hashing for itself).
 __global__ __launch_bounds__(256) void cloud_map_kernel(SkyhipNoiseCreateInfo density, SkyhipNoiseCreateInfo height,
                                                         uint8_t* __restrict__ out, int size) {
-    int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= size * size) return;
-    float x = (float(t % size) + 0.5f) / float(size), y = (float(t / size) + 0.5f) / float(size);
-    uchar2 v;
-    v.x = to_unorm8(perlin_fbm(x, y, 0.0f, density));
-    v.y = to_unorm8(worley_fbm(x, y, 0.0f, height));
-    reinterpret_cast<uchar2*>(out)[t] = v;
+    __shared__ NoiseLds s;
+    NoiseTile t;
+    const TexelPos p = image_tile(size, t);
+    const float v = blockIdx.z == 0 ? perlin_fbm<256>(s, t, density) : worley_fbm<256>(s, t, height);
+    if (p.in) out[2ll * (p.y * size + p.x) + blockIdx.z] = to_unorm8(v);
 }
 
 __global__ __launch_bounds__(256) void detail_kernel(SkyhipNoiseCreateInfo perlin, SkyhipNoiseCreateInfo worley,
                                                      uint8_t* __restrict__ out, int size) {
-    long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (long long)size * size * size) return;
-    int ix = int(t % size), iy = int((t / size) % size), iz = int(t / ((long long)size * size));
-    float x = (float(ix) + 0.5f) / float(size), y = (float(iy) + 0.5f) / float(size),
-          z = (float(iz) + 0.5f) / float(size);
-    float p = perlin_fbm(x, y, z, perlin);
-    float w = worley_fbm(x, y, z, worley);
-    out[t] = to_unorm8(fminf(fmaxf(w + p * (1.0f - w), 0.0f), 1.0f));  // RemapFrom01(p, w, 1)
+    __shared__ NoiseLds s;
+    NoiseTile t;
+    const TexelPos at = volume_tile(size, size, size, t);
+    float p = perlin_fbm<256>(s, t, perlin);
+    float w = worley_fbm<256>(s, t, worley);
+    if (at.in)  // RemapFrom01(p, w, 1)
+        out[((long long)at.z * size + at.y) * size + at.x] = to_unorm8(fminf(fmaxf(w + p * (1.0f - w), 0.0f), 1.0f));
 }
 
 // The Worley detail volume: WorleyFBM alone at texel centres, UNORM8.
 __global__ __launch_bounds__(256) void worley_kernel(SkyhipNoiseCreateInfo worley, uint8_t* __restrict__ out,
                                                      int size) {
-    long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (long long)size * size * size) return;
-    int ix = int(t % size), iy = int((t / size) % size), iz = int(t / ((long long)size * size));
-    float x = (float(ix) + 0.5f) / float(size), y = (float(iy) + 0.5f) / float(size),
-          z = (float(iz) + 0.5f) / float(size);
-    out[t] = to_unorm8(worley_fbm(x, y, z, worley));
+    __shared__ NoiseLds s;
+    NoiseTile t;
+    const TexelPos at = volume_tile(size, size, size, t);
+    const uint8_t v = to_unorm8(worley_fbm<256>(s, t, worley));
+    if (at.in) out[((long long)at.z * size + at.y) * size + at.x] = v;
 }
 
 __global__ __launch_bounds__(256) void displacement_kernel(SkyhipNoiseCreateInfo perlin, uint8_t* __restrict__ out,
                                                            int size) {
-    int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= size * size) return;
-    float x = (float(t % size) + 0.5f) / float(size), y = (float(t / size) + 0.5f) / float(size);
-    uchar4 v;
-    uint8_t* c = &v.x;
-    for (int i = 0; i < 4; ++i) {
-        SkyhipNoiseCreateInfo ci = perlin;
-        ci.seed += uint32_t(i);
-        c[i] = to_unorm8(perlin_fbm(x, y, 0.0f, ci));
-    }
-    reinterpret_cast<uchar4*>(out)[t] = v;
+    __shared__ NoiseLds s;
+    NoiseTile t;
+    const TexelPos p = image_tile(size, t);
+    perlin.seed += blockIdx.z;
+    const uint8_t v = to_unorm8(perlin_fbm<256>(s, t, perlin));
+    if (p.in) out[4ll * (p.y * size + p.x) + blockIdx.z] = v;
 }
 
 // One mip step of a UNORM8 texture: box over 2x2(x2) source texels (indices
@@ -196,14 +360,13 @@ __global__ __launch_bounds__(256) void downsample_kernel(const uint8_t* __restri
 // threshold, FP16 round-to-nearest-even.  One lane per texel.
 __global__ __launch_bounds__(256) void voxel_grid_kernel(SkyhipVoxelGridCreateInfo ci, uint16_t* __restrict__ out,
                                                          int nx, int ny, int nz) {
-    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (long long)nx * ny * nz) return;
-    int x = int(i % nx), y = int((i / nx) % ny), z = int(i / ((long long)nx * ny));
-    float p[3] = {(float(x) + 0.5f) / float(nx), (float(y) + 0.5f) / float(ny), (float(z) + 0.5f) / float(nz)};
+    __shared__ NoiseLds s;
+    NoiseTile t;
+    const TexelPos at = volume_tile(nx, ny, nz, t);
     float res = 0.0f, a = 1.0f, sum_a = 0.0f;
     uint32_t f = ci.base_frequency;
     for (int o = 0; o < ci.octaves; ++o) {
-        res += perlin_noise(p[0], p[1], p[2], f, ci.seed) * a;
+        res += perlin_octave<256>(s, t, f, ci.seed) * a;
         sum_a += a;
         f *= 2u;
         a *= 0.5f;
@@ -211,12 +374,20 @@ __global__ __launch_bounds__(256) void voxel_grid_kernel(SkyhipVoxelGridCreateIn
     float fbm = res / sum_a;
     float e = 0.0f;
     for (int k = 0; k < 3; ++k) {
-        float q = (p[k] - ci.ellipsoid_center[k]) / ci.ellipsoid_radii[k];
+        float q = (t.p[k] - ci.ellipsoid_center[k]) / ci.ellipsoid_radii[k];
         e += q * q;
     }
     float falloff = fmaxf(1.0f - e, 0.0f);
     float density = fmaxf(expf(ci.lognormal_sigma * ci.fbm_inv_std * fbm) * falloff - ci.threshold, 0.0f);
-    out[i] = __builtin_bit_cast(uint16_t, __float2half_rn(density));
+    if (at.in)
+        out[((long long)at.z * ny + at.y) * nx + at.x] = __builtin_bit_cast(uint16_t, __float2half_rn(density));
+}
+
+dim3 image_grid(int size, int channels) {
+    return dim3(div_up(size, kImageTile), div_up(size, kImageTile), unsigned(channels));
+}
+dim3 volume_grid(int nx, int ny, int nz) {
+    return dim3(div_up(nx, kVolumeTileXY), div_up(ny, kVolumeTileXY), div_up(nz, kVolumeTileZ));
 }
 
 int validate_noise(const SkyhipNoiseCreateInfo* ci) {
@@ -259,7 +430,7 @@ extern "C" int skyhip_noise_cloud_map(SkyhipContext* ctx, const SkyhipNoiseCreat
     SKYHIP_CHECK(validate_noise(height));
     if (out_rg8 == nullptr) return fail(SKYHIP_ERR_INVALID_ARGUMENT, "output is NULL");
     if (size < 1 || size > 16384) return fail(SKYHIP_ERR_INVALID_SIZE, "cloud map size %d outside [1, 16384]", size);
-    hipLaunchKernelGGL(cloud_map_kernel, dim3(div_up((long long)size * size, 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(cloud_map_kernel, image_grid(size, 2), dim3(256), 0, ctx->stream,
                        *density, *height, out_rg8, size);
     SKYHIP_LAUNCH_CHECK("cloud_map_kernel");
     return SKYHIP_OK;
@@ -272,7 +443,7 @@ extern "C" int skyhip_noise_detail(SkyhipContext* ctx, const SkyhipNoiseCreateIn
     SKYHIP_CHECK(validate_noise(worley));
     if (out_r8 == nullptr) return fail(SKYHIP_ERR_INVALID_ARGUMENT, "output is NULL");
     if (size < 1 || size > 1024) return fail(SKYHIP_ERR_INVALID_SIZE, "detail size %d outside [1, 1024]", size);
-    hipLaunchKernelGGL(detail_kernel, dim3(div_up((long long)size * size * size, 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(detail_kernel, volume_grid(size, size, size), dim3(256), 0, ctx->stream,
                        *perlin, *worley, out_r8, size);
     SKYHIP_LAUNCH_CHECK("detail_kernel");
     return SKYHIP_OK;
@@ -284,7 +455,7 @@ extern "C" int skyhip_noise_displacement(SkyhipContext* ctx, const SkyhipNoiseCr
     SKYHIP_CHECK(validate_noise(perlin));
     if (out_rgba8 == nullptr) return fail(SKYHIP_ERR_INVALID_ARGUMENT, "output is NULL");
     if (size < 1 || size > 16384) return fail(SKYHIP_ERR_INVALID_SIZE, "displacement size %d outside [1, 16384]", size);
-    hipLaunchKernelGGL(displacement_kernel, dim3(div_up((long long)size * size, 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(displacement_kernel, image_grid(size, 4), dim3(256), 0, ctx->stream,
                        *perlin, out_rgba8, size);
     SKYHIP_LAUNCH_CHECK("displacement_kernel");
     return SKYHIP_OK;
@@ -296,7 +467,7 @@ extern "C" int skyhip_noise_worley(SkyhipContext* ctx, const SkyhipNoiseCreateIn
     SKYHIP_CHECK(validate_noise(worley));
     if (out_r8 == nullptr) return fail(SKYHIP_ERR_INVALID_ARGUMENT, "output is NULL");
     if (size < 1 || size > 1024) return fail(SKYHIP_ERR_INVALID_SIZE, "Worley volume size %d outside [1, 1024]", size);
-    hipLaunchKernelGGL(worley_kernel, dim3(div_up((long long)size * size * size, 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(worley_kernel, volume_grid(size, size, size), dim3(256), 0, ctx->stream,
                        *worley, out_r8, size);
     SKYHIP_LAUNCH_CHECK("worley_kernel");
     return SKYHIP_OK;
@@ -397,8 +568,7 @@ extern "C" int skyhip_voxel_grid_generate(SkyhipContext* ctx, const SkyhipVoxelG
     if (!finite_block(&info->fbm_inv_std, 9)) return fail(SKYHIP_ERR_NON_FINITE, "non-finite grid parameter");
     for (int k = 0; k < 3; ++k)
         if (!(info->ellipsoid_radii[k] > 0.0f)) return fail(SKYHIP_ERR_INVALID_ARGUMENT, "ellipsoid radii must be > 0");
-    long long n = (long long)dim_x * dim_y * dim_z;
-    hipLaunchKernelGGL(voxel_grid_kernel, dim3(unsigned(div_up(n, 256))), dim3(256), 0, ctx->stream, *info, out_grid,
+    hipLaunchKernelGGL(voxel_grid_kernel, volume_grid(dim_x, dim_y, dim_z), dim3(256), 0, ctx->stream, *info, out_grid,
                        dim_x, dim_y, dim_z);
     SKYHIP_LAUNCH_CHECK("voxel_grid_kernel");
     return SKYHIP_OK;
