@@ -4,7 +4,7 @@
 // Layout: every LUT is RGBA32F in GL texel order, one lane per texel (one
 // wave64 per texel for multiple scattering, whose 64 sphere directions map to
 // the 64 lanes), 256-lane workgroups, 1D grids over texels so stores coalesce.
-#include "lut_texels.h"
+#include "sky_rows.h"
 
 #include <cmath>
 
@@ -21,17 +21,34 @@ __global__ __launch_bounds__(256) void transmittance_kernel(SkyhipAtmosphereBuff
 }
 
 // ---------------------------------------------------------------------------
-// Multiple scattering (Atmosphere.glsl:344-438): one wave64 per texel.
+// Multiple scattering (Atmosphere.glsl:344-438): one wave64 per texel, whose step tables (sky_rows.h)
+// its workgroup's texels, of one row, share; marches of more than kMsMaxSteps steps integrate
+// direction by direction.  32 x 32, 30 steps: 13.1 us, 21.3 with every direction evaluating its own
+// densities and exponentials.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void multiscattering_kernel(SkyhipAtmosphereBufferData b,
-                                                              const float4* __restrict__ T, int tw, int th,
-                                                              float4* __restrict__ out, int w, int h) {
+constexpr int kMsTexels = 4;  // texels (waves) of a workgroup
+__global__ __launch_bounds__(64 * kMsTexels) void multiscattering_kernel(SkyhipAtmosphereBufferData b,
+                                                                         const float4* __restrict__ T, int tw, int th,
+                                                                         float4* __restrict__ out, int w, int h) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MsTotals totals[kMsThetas];
     const AtmDev A = make_atm(b);
-    const int texel = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int n = row_step_count(A.ms_steps), ix = blockIdx.x * kMsTexels + (threadIdx.x >> 6), iy = blockIdx.y;
     const int lane = threadIdx.x & 63;
-    if (texel >= w * h) return;  // wave-uniform
-    float4 v = multiscattering_texel(A, T, tw, th, texel % w, texel / w, w, h, lane);
-    if (lane == 0) out[texel] = v;
+    if (n > kMsMaxSteps) {
+        if (ix >= w) return;  // wave-uniform
+        const float4 v = multiscattering_texel(A, T, tw, th, ix, iy, w, h, lane);
+        if (lane == 0) out[iy * w + ix] = v;
+        return;
+    }
+    MsStep* steps = reinterpret_cast<MsStep*>(smem);
+    ms_row_tables(A, iy, h, tw, th, n, steps, totals);
+    __syncthreads();
+    if (ix >= w) return;
+    const MsRay ray = ms_ray(A, ix, iy, w, h, lane);
+    const F3 L = ms_row_steps<false>(T, tw, th, steps, n, ray, 0, n);
+    const float4 v = multiscattering_reduce(A, T, tw, th, ray, L, totals[lane >> 3].tr, totals[lane >> 3].lf);
+    if (lane == 0) out[iy * w + ix] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -52,6 +69,21 @@ __global__ __launch_bounds__(256) void sky_view_kernel(SkyhipAtmosphereBufferDat
     sky_view_texel(A, R, T, tw, th, MS, mw, mh, blue_noise, bn_size, t % w, t / w, w, h, L, Tr);
     out_l[t] = make_float4(L.x, L.y, L.z, 0.0f);
     out_t[t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
+}
+
+// The same without dither, by rows: a wave takes 64 columns of a row.  A single LUT is latency-bound,
+// so a lane takes one ray, where the batched builder's takes up to three.
+__global__ __launch_bounds__(64) void sky_view_rows_kernel(SkyhipAtmosphereBufferData b,
+                                                           SkyhipAtmosphereRenderBufferData rbd,
+                                                           const float4* __restrict__ T, int tw, int th,
+                                                           const float4* __restrict__ MS, int mw, int mh,
+                                                           float4* __restrict__ out_l, float4* __restrict__ out_t,
+                                                           int w, int h) {
+    __shared__ RowLds lds;
+    const AtmDev A = make_atm(b);
+    const RenderDev R = make_render(rbd);
+    sky_view_row<1>([&] { return A; }, R, sky_view_row_setup(A, R, blockIdx.y, h), T, tw, th, MS, mw, mh, blockIdx.y,
+                    blockIdx.x * 64, w, lds, out_l, out_t);
 }
 
 // ---------------------------------------------------------------------------
@@ -261,8 +293,9 @@ int launch_transmittance(hipStream_t st, const SkyhipAtmosphereBufferData& b, fl
 
 int launch_multiscattering(hipStream_t st, const SkyhipAtmosphereBufferData& b, const float* T, int tw, int th,
                            float* out, int w, int h) {
-    hipLaunchKernelGGL(multiscattering_kernel, dim3(div_up(w * h, 4)), dim3(256), 0, st, b,
-                       reinterpret_cast<const float4*>(T), tw, th, reinterpret_cast<float4*>(out), w, h);
+    hipLaunchKernelGGL(multiscattering_kernel, dim3(div_up(w, kMsTexels), h), dim3(64 * kMsTexels),
+                       ms_table_bytes(b.multiscattering_steps), st, b, reinterpret_cast<const float4*>(T), tw, th,
+                       reinterpret_cast<float4*>(out), w, h);
     SKYHIP_LAUNCH_CHECK("multiscattering_kernel");
     return SKYHIP_OK;
 }
@@ -270,6 +303,15 @@ int launch_multiscattering(hipStream_t st, const SkyhipAtmosphereBufferData& b, 
 int launch_sky_view(hipStream_t st, const SkyhipAtmosphereBufferData& b, const SkyhipAtmosphereRenderBufferData& r,
                     const float* T, int tw, int th, const float* MS, int mw, int mh, const uint16_t* bn, int bn_size,
                     float* L, float* Tr, int w, int h) {
+    // Rows share their march unless the dither starts every texel's elsewhere, or the LUTs are wider
+    // than a wave's entries.  128 x 128, 30 steps: 12.7 us by rows, 31.6 texel by texel.
+    if (bn == nullptr && row_luts_fit(tw, mw)) {
+        hipLaunchKernelGGL(sky_view_rows_kernel, dim3(div_up(w, 64), h), dim3(64), 0, st, b, r,
+                           reinterpret_cast<const float4*>(T), tw, th, reinterpret_cast<const float4*>(MS), mw, mh,
+                           reinterpret_cast<float4*>(L), reinterpret_cast<float4*>(Tr), w, h);
+        SKYHIP_LAUNCH_CHECK("sky_view_rows_kernel");
+        return SKYHIP_OK;
+    }
     hipLaunchKernelGGL(sky_view_kernel, dim3(div_up(w * h, 256)), dim3(256), 0, st, b, r,
                        reinterpret_cast<const float4*>(T), tw, th, reinterpret_cast<const float4*>(MS), mw, mh, bn,
                        bn_size, reinterpret_cast<float4*>(L), reinterpret_cast<float4*>(Tr), w, h);

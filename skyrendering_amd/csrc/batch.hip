@@ -3,19 +3,20 @@
 // each with its own sky-view LUT, at mixed resolutions, built by one hipGraph
 // launch.
 //
-// The graph holds four kernel nodes: a counter reset, then one persistent
+// The graph holds five kernel nodes: a counter reset, then one persistent
 // kernel per pass (transmittance -> multiple scattering -> sky view; kernel
-// order carries the dependencies).  Each persistent kernel runs a fixed number
+// order carries the dependencies), and the transmittance LUTs' cell-corner
+// copy before multiple scattering.  Each persistent kernel runs a fixed number
 // of workgroups per CU that pull tiles (item, first texel) from a device
 // counter until the tile list is exhausted, so items of very different sizes
 // share the machine without one launch per item.  Every texel runs the
-// single-set arithmetic of lut_texels.h.  Tile sizes, workgroup sizes,
+// single-set arithmetic of lut_texels.h and sky_rows.h.  Tile sizes, workgroup sizes,
 // workgroups per CU and the sky-view tile order are chosen by the autotuner
 // below, which times each pass's candidates on the batch itself.
 #include <algorithm>
 #include <vector>
 
-#include "lut_texels.h"
+#include "sky_rows.h"
 
 namespace skyhip {
 
@@ -44,32 +45,37 @@ __global__ void batch_reset_kernel(unsigned* __restrict__ ctr) {
 __device__ __forceinline__ int next_tile(unsigned* ctr, int* s_tile) {
     if (threadIdx.x == 0) *s_tile = int(atomicAdd(ctr, 1u));
     __syncthreads();
-    int tile = *s_tile;
+    const int tile = __builtin_amdgcn_readfirstlane(*s_tile);  // uniform, so an item's blocks are scalar loads
     __syncthreads();
     return tile;
 }
 
-// Cell-corner copies of every item's T (kind 0) or MS (kind 1) LUT: texel (x, y) of an item is
-// followed by the rest of its bilinear footprint, (x, y), (x1, y), (x, y1), (x1, y1) with
-// x1 = min(x + 1, w - 1) and y1 likewise (4 float4 per texel, lut_bilinear<true>).  Items stride
-// over blockIdx.y, texels over blockIdx.x.
+// Cell-corner copies of every item's T LUT: texel (x, y) of an item is followed by the rest of its
+// bilinear footprint, (x, y), (x1, y), (x, y1), (x1, y1) with x1 = min(x + 1, w - 1) and y1 likewise
+// (4 float4 per texel, lut_bilinear<true>).  Items stride over blockIdx.y, texels over blockIdx.x.
 __global__ __launch_bounds__(256) void batch_lut_cells_kernel(const BatchSetDev* __restrict__ sets, int n_sets,
-                                                              int kind, const float4* __restrict__ pool,
+                                                              const float4* __restrict__ pool,
                                                               float4* __restrict__ cells) {
     for (int item = blockIdx.y; item < n_sets; item += gridDim.y) {
         const BatchSetDev S = sets[item];
-        const int w = kind == 0 ? S.tw : S.mw, h = kind == 0 ? S.th : S.mh;
-        const long long off = kind == 0 ? S.t_off : S.ms_off;
-        const float4* src = pool + off;
+        const int w = S.tw, h = S.th;
+        const float4* src = pool + S.t_off;
         for (int t = blockIdx.x * 256 + threadIdx.x; t < w * h; t += gridDim.x * 256) {
             const int x = t % w, y = t / w, x1 = min(x + 1, w - 1), y1 = min(y + 1, h - 1);
-            float4* dst = cells + 4 * (off + t);
+            float4* dst = cells + 4 * (S.t_off + t);
             dst[0] = src[y * w + x];
             dst[1] = src[y * w + x1];
             dst[2] = src[y1 * w + x];
             dst[3] = src[y1 * w + x1];
         }
     }
+}
+
+// Rows of a view in a sky-view tile of about tile_size texels.
+constexpr int kMaxTileRows = 32;
+__host__ __device__ inline int sky_view_tile_rows(int tile_size, int w) {
+    const int rows = tile_size / w;
+    return rows < 1 ? 1 : rows > kMaxTileRows ? kMaxTileRows : rows;
 }
 
 template <int kBlock>
@@ -91,52 +97,108 @@ __global__ __launch_bounds__(kBlock) void batch_transmittance_kernel(
     }
 }
 
+// A tile is up to kMsTileTexels texels per wave of one row of an item's LUT: the workgroup builds the
+// row's step tables, then its waves take the texels.  256 LUTs of 32 x 32: 1.05 ms, 2.4 ms with every
+// direction evaluating its own densities and exponentials.
+constexpr int kMsTileTexels = 8;
 template <int kWaves>
 __global__ __launch_bounds__(64 * kWaves) void batch_multiscattering_kernel(
     const SkyhipAtmosphereBufferData* __restrict__ atm, const BatchSetDev* __restrict__ sets,
     const Tile* __restrict__ tiles, int n_tiles, const float4* __restrict__ t_cells, float4* __restrict__ pool,
     unsigned* ctr) {
+    extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_tile;
+    __shared__ MsTotals totals[kMsThetas];
+    MsStep* steps = reinterpret_cast<MsStep*>(smem);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (;;) {
         const int tile = next_tile(ctr + kCtrMS, &s_tile);
         if (tile >= n_tiles) return;
         const Tile tl = tiles[tile];
         const BatchSetDev S = sets[tl.item];
-        const int texel = int(tl.first) + wave;
-        if (texel < S.mw * S.mh) {  // wave-uniform
-            const AtmDev A = make_atm(atm[tl.item]);
-            float4 v = multiscattering_texel<true>(A, t_cells + 4 * S.t_off, S.tw, S.th, texel % S.mw, texel / S.mw,
-                                                   S.mw, S.mh, lane);
-            if (lane == 0) pool[S.ms_off + texel] = v;
+        const AtmDev A = make_atm(atm[tl.item]);
+        const float4* T = t_cells + 4 * S.t_off;
+        const int iy = int(tl.first) / S.mw, x0 = int(tl.first) - iy * S.mw;
+        const int n = row_step_count(A.ms_steps);
+        const bool tables = n <= kMsMaxSteps;
+        if (tables) {
+            ms_row_tables(A, iy, S.mh, S.tw, S.th, n, steps, totals);
+            __syncthreads();  // next_tile's barriers order these reads before the next tables
+        }
+        for (int ix = x0 + wave; ix < min(x0 + kMsTileTexels * kWaves, S.mw); ix += kWaves) {  // wave-uniform
+            float4 v;
+            if (tables) {
+                const MsRay ray = ms_ray(A, ix, iy, S.mw, S.mh, lane);
+                const F3 L = ms_row_steps<true>(T, S.tw, S.th, steps, n, ray, 0, n);
+                v = multiscattering_reduce<true>(A, T, S.tw, S.th, ray, L, totals[lane >> 3].tr, totals[lane >> 3].lf);
+            } else {
+                v = multiscattering_texel<true>(A, T, S.tw, S.th, ix, iy, S.mw, S.mh, lane);
+            }
+            if (lane == 0) pool[S.ms_off + iy * S.mw + ix] = v;
         }
     }
 }
 
+// A pointer the compiler takes for a new one, so that what is read through it is not kept from before.
+template <class B>
+__device__ __forceinline__ const B* reload(const B* p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// A tile is whole rows of a view, each taken by the workgroup's waves in pieces of 64 to 192 columns.
+// Bound by vector instructions (97 % of the issue slots).  256 sets x 8 suns: 2.9 ms, 11.2 ms with
+// every texel marching for itself; three rays per lane against six 2.9 / 4.3 ms (six leave two waves
+// a SIMD), runs of steps of one kind against a three-way branch per step 3.0 / 3.9 ms (the branch's
+// joins copy the sums), tiles of 4,096 texels against 1,024 2.8 / 3.0 ms (rows set up a lane each).
 template <int kBlock>
-__global__ __launch_bounds__(kBlock) void batch_sky_view_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void batch_sky_view_kernel(
     const SkyhipAtmosphereBufferData* __restrict__ atm, const SkyhipAtmosphereRenderBufferData* __restrict__ renders,
     const BatchSetDev* __restrict__ sets, const BatchViewDev* __restrict__ views, const Tile* __restrict__ tiles,
-    int n_tiles, int tile_size, const float4* __restrict__ t_cells, const float4* __restrict__ ms_cells,
+    int n_tiles, int tile_size, const float4* __restrict__ t_pool, const float4* __restrict__ ms_pool,
     float4* __restrict__ l_pool, float4* __restrict__ tr_pool, unsigned* ctr) {
     __shared__ int s_tile;
+    __shared__ RowLds lds[kBlock / 64];
+    __shared__ SkyViewRow rows[kMaxTileRows];
+    const int wave = threadIdx.x >> 6;
     for (;;) {
         const int tile = next_tile(ctr + kCtrSV, &s_tile);
         if (tile >= n_tiles) return;
         const Tile tl = tiles[tile];
         const BatchViewDev V = views[tl.item];
         const BatchSetDev S = sets[V.set];
-        const AtmDev A = make_atm(atm[V.set]);
-        const RenderDev R = make_render(renders[tl.item]);
-        const int n = V.sw * V.sh;
-        for (int k = threadIdx.x; k < tile_size; k += kBlock) {
-            const int t = int(tl.first) + k;
-            if (t >= n) break;
-            F3 L, Tr;
-            sky_view_texel<true>(A, R, t_cells + 4 * S.t_off, S.tw, S.th, ms_cells + 4 * S.ms_off, S.mw, S.mh,
-                                 nullptr, 1, t % V.sw, t / V.sw, V.sw, V.sh, L, Tr);
-            l_pool[V.sv_off + t] = make_float4(L.x, L.y, L.z, 0.0f);
-            tr_pool[V.sv_off + t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
+        // The blocks are read again (scalar loads) where they are used, instead of held through the march.
+        const auto get_atm = [&] { return make_atm(*reload(atm + V.set)); };
+        const auto get_render = [&] { return make_render(*reload(renders + tl.item)); };
+        const float4 *T = t_pool + S.t_off, *MS = ms_pool + S.ms_off;
+        float4 *out_l = l_pool + V.sv_off, *out_t = tr_pool + V.sv_off;
+        const int y0 = int(tl.first) / V.sw, y1 = min(y0 + sky_view_tile_rows(tile_size, V.sw), V.sh);
+        if (!row_luts_fit(S.tw, S.mw)) {  // LUTs wider than a wave's entries: texel by texel
+            const AtmDev A = get_atm();
+            const RenderDev R = get_render();
+            for (int t = y0 * V.sw + int(threadIdx.x); t < y1 * V.sw; t += kBlock) {
+                F3 L, Tr;
+                sky_view_texel(A, R, T, S.tw, S.th, MS, S.mw, S.mh, nullptr, 1, t % V.sw, t / V.sw, V.sw, V.sh, L, Tr);
+                out_l[t] = make_float4(L.x, L.y, L.z, 0.0f);
+                out_t[t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
+            }
+            continue;
+        }
+        // The rows' rays, a thread each (next_tile's barriers keep the last tile's readers apart).
+        if (int(threadIdx.x) < y1 - y0) rows[threadIdx.x] = sky_view_row_setup(get_atm(), get_render(), y0 + threadIdx.x, V.sh);
+        __syncthreads();
+        const int rays = row_rays_per_lane(V.sw), pieces = (V.sw + 64 * rays - 1) / (64 * rays);
+        for (int i = wave; i < (y1 - y0) * pieces; i += kBlock / 64) {
+            const int y = i / pieces, x0 = (i - y * pieces) * 64 * rays;
+            if (rays == 3)
+                sky_view_row<3>(get_atm, get_render(), rows[y], T, S.tw, S.th, MS, S.mw, S.mh, y0 + y, x0, V.sw,
+                                lds[wave], out_l, out_t);
+            else if (rays == 2)
+                sky_view_row<2>(get_atm, get_render(), rows[y], T, S.tw, S.th, MS, S.mw, S.mh, y0 + y, x0, V.sw,
+                                lds[wave], out_l, out_t);
+            else
+                sky_view_row<1>(get_atm, get_render(), rows[y], T, S.tw, S.th, MS, S.mw, S.mh, y0 + y, x0, V.sw,
+                                lds[wave], out_l, out_t);
         }
     }
 }
@@ -161,8 +223,9 @@ struct SkyhipLutBatch {
     BatchSetDev* d_sets = nullptr;
     BatchViewDev* d_views = nullptr;
     float4 *t_pool = nullptr, *ms_pool = nullptr, *l_pool = nullptr, *tr_pool = nullptr;
-    float4 *t_cells = nullptr, *ms_cells = nullptr;  // cell-corner copies of the T and MS pools (4x)
-    int max_t_texels = 0, max_ms_texels = 0;
+    float4* t_cells = nullptr;  // cell-corner copy of the T pool (4x)
+    int max_t_texels = 0;
+    size_t ms_lds_bytes = 0;  // the largest set's step tables
     unsigned* d_ctr = nullptr;
     Tile *d_t_tiles = nullptr, *d_ms_tiles = nullptr, *d_sv_tiles = nullptr;
     int n_t_tiles = 0, n_ms_tiles = 0, n_sv_tiles = 0;
@@ -216,7 +279,9 @@ int build_tiles(SkyhipLutBatch* b) {
     for (int s = 0; s < b->n_sets; ++s) {
         const BatchSetDev& S = b->sets[s];
         for (int f = 0; f < S.tw * S.th; f += t.transmittance_tile) tt.push_back({uint32_t(s), uint32_t(f)});
-        for (int f = 0; f < S.mw * S.mh; f += t.multiscattering_waves) mt.push_back({uint32_t(s), uint32_t(f)});
+        for (int y = 0; y < S.mh; ++y)
+            for (int x = 0; x < S.mw; x += kMsTileTexels * t.multiscattering_waves)
+                mt.push_back({uint32_t(s), uint32_t(y * S.mw + x)});
     }
     std::vector<int> order(b->n_views);
     for (int v = 0; v < b->n_views; ++v) order[v] = v;
@@ -226,7 +291,8 @@ int build_tiles(SkyhipLutBatch* b) {
         });
     for (int v : order) {
         const BatchViewDev& V = b->views[v];
-        for (int f = 0; f < V.sw * V.sh; f += t.sky_view_tile) st.push_back({uint32_t(v), uint32_t(f)});
+        for (int y = 0; y < V.sh; y += sky_view_tile_rows(t.sky_view_tile, V.sw))
+            st.push_back({uint32_t(v), uint32_t(y * V.sw)});
     }
     b->n_t_tiles = int(tt.size());
     b->n_ms_tiles = int(mt.size());
@@ -261,10 +327,10 @@ void enqueue_t(SkyhipLutBatch* b, hipStream_t st) {
 void enqueue_ms(SkyhipLutBatch* b, hipStream_t st) {
     const SkyhipLutBatchTuning& t = b->tuning;
     hipLaunchKernelGGL(batch_lut_cells_kernel, cells_grid(b->max_t_texels, b->n_sets), dim3(256), 0, st, b->d_sets,
-                       b->n_sets, 0, b->t_pool, b->t_cells);
+                       b->n_sets, b->t_pool, b->t_cells);
     dim3 g(grid_for(b, t.multiscattering_blocks_per_cu, b->n_ms_tiles));
 #define SKYHIP_MS(W)                                                                                              \
-    hipLaunchKernelGGL(batch_multiscattering_kernel<W>, g, dim3(64 * W), 0, st, b->d_atm, b->d_sets,            \
+    hipLaunchKernelGGL(batch_multiscattering_kernel<W>, g, dim3(64 * W), b->ms_lds_bytes, st, b->d_atm, b->d_sets, \
                        b->d_ms_tiles, b->n_ms_tiles, b->t_cells, b->ms_pool, b->d_ctr)
     if (t.multiscattering_waves == 1) SKYHIP_MS(1);
     else if (t.multiscattering_waves == 2) SKYHIP_MS(2);
@@ -273,16 +339,12 @@ void enqueue_ms(SkyhipLutBatch* b, hipStream_t st) {
 #undef SKYHIP_MS
 }
 
-// The sky-view pass, with the multiple-scattering cell copy it reads built first (the
-// transmittance one comes from the multiple-scattering pass).
 void enqueue_sv(SkyhipLutBatch* b, hipStream_t st) {
     const SkyhipLutBatchTuning& t = b->tuning;
-    hipLaunchKernelGGL(batch_lut_cells_kernel, cells_grid(b->max_ms_texels, b->n_sets), dim3(256), 0, st, b->d_sets,
-                       b->n_sets, 1, b->ms_pool, b->ms_cells);
     dim3 g(grid_for(b, t.sky_view_blocks_per_cu, b->n_sv_tiles));
 #define SKYHIP_SV(B)                                                                                              \
     hipLaunchKernelGGL(batch_sky_view_kernel<B>, g, dim3(B), 0, st, b->d_atm, b->d_render, b->d_sets, b->d_views, \
-                       b->d_sv_tiles, b->n_sv_tiles, t.sky_view_tile, b->t_cells, b->ms_cells, b->l_pool,        \
+                       b->d_sv_tiles, b->n_sv_tiles, t.sky_view_tile, b->t_pool, b->ms_pool, b->l_pool,          \
                        b->tr_pool, b->d_ctr)
     if (t.sky_view_block == 64) SKYHIP_SV(64);
     else if (t.sky_view_block == 128) SKYHIP_SV(128);
@@ -364,7 +426,7 @@ SkyhipLutBatchTuning default_tuning() {
     t.multiscattering_waves = 4;
     t.multiscattering_blocks_per_cu = 8;
     t.sky_view_block = 256;
-    t.sky_view_tile = 1024;
+    t.sky_view_tile = 4096;
     t.sky_view_blocks_per_cu = 4;
     t.sky_view_largest_first = 1;
     return t;
@@ -403,7 +465,7 @@ extern "C" int skyhip_lut_batch_create(SkyhipContext* ctx, const SkyhipLutBatchS
         t_total += (long long)d.tw * d.th;
         ms_total += (long long)d.mw * d.mh;
         b->max_t_texels = std::max(b->max_t_texels, d.tw * d.th);
-        b->max_ms_texels = std::max(b->max_ms_texels, d.mw * d.mh);
+        b->ms_lds_bytes = std::max(b->ms_lds_bytes, ms_table_bytes(S.atmosphere.multiscattering_steps));
         b->steps += (unsigned long long)d.tw * d.th * loop_iterations(S.atmosphere.transmittance_steps) +
                     64ull * d.mw * d.mh * loop_iterations(S.atmosphere.multiscattering_steps);
     }
@@ -434,7 +496,6 @@ extern "C" int skyhip_lut_batch_create(SkyhipContext* ctx, const SkyhipLutBatchS
         (rc = alloc(reinterpret_cast<void**>(&b->t_pool), sizeof(float4) * t_total)) ||
         (rc = alloc(reinterpret_cast<void**>(&b->ms_pool), sizeof(float4) * ms_total)) ||
         (rc = alloc(reinterpret_cast<void**>(&b->t_cells), 4 * sizeof(float4) * t_total)) ||
-        (rc = alloc(reinterpret_cast<void**>(&b->ms_cells), 4 * sizeof(float4) * ms_total)) ||
         (rc = alloc(reinterpret_cast<void**>(&b->l_pool), sizeof(float4) * sv_total)) ||
         (rc = alloc(reinterpret_cast<void**>(&b->tr_pool), sizeof(float4) * sv_total)) ||
         (rc = alloc(reinterpret_cast<void**>(&b->d_ctr), 16)))
@@ -462,7 +523,7 @@ extern "C" int skyhip_lut_batch_destroy(SkyhipLutBatch* b) {
     release_graph(b);
     free_tiles(b);
     for (void* p : {(void*)b->d_atm, (void*)b->d_render, (void*)b->d_sets, (void*)b->d_views, (void*)b->t_pool,
-                    (void*)b->ms_pool, (void*)b->t_cells, (void*)b->ms_cells, (void*)b->l_pool, (void*)b->tr_pool,
+                    (void*)b->ms_pool, (void*)b->t_cells, (void*)b->l_pool, (void*)b->tr_pool,
                     (void*)b->d_ctr})
         if (p) (void)hipFree(p);
     if (b->capture) (void)hipStreamDestroy(b->capture);

@@ -211,14 +211,11 @@ __device__ inline void start_from_space(const AtmDev& A, RayStart& s, float& mar
     }
 }
 
-// The ray of one sky-view texel (:74-186): its start, marching distance (0: nothing to
-// integrate) and the float counter's start value.
-struct SkyViewRay {
-    RayStart s;
-    float dist, start_i;
+// The latitude of a sky-view row, and the sun-view cosine of a column of it.
+struct SkyViewLatitude {
+    float cos_lat, sin_lat;
 };
-__device__ inline SkyViewRay sky_view_ray(const AtmDev& A, const RenderDev& R, const uint16_t* __restrict__ blue_noise,
-                                          int bn_size, int ix, int iy, int w, int h) {
+__device__ inline SkyViewLatitude sky_view_latitude(const AtmDev& A, const RenderDev& R, int iy, int h) {
     const float r = R.r;
     const float alt0 = r - A.rb;
     // GetHorizonDownAngleFromR (:74-78) and GetCosLatLonFromSkyViewTextureIndex (:81-102).
@@ -230,7 +227,6 @@ __device__ inline SkyViewRay sky_view_ray(const AtmDev& A, const RenderDev& R, c
     const float horizon_down = acosf(rho / r);
     const float horizon_up = kPiF - horizon_down;
     const float cos_hu = -rho / r, sin_hu = A.rb / r;
-    const float x_lon = float(ix) / float(w - 1);
     const float x_lat = float(iy) / float(h - 1);
     float delta;
     if (x_lat < 0.5f) {
@@ -242,13 +238,28 @@ __device__ inline SkyViewRay sky_view_ray(const AtmDev& A, const RenderDev& R, c
     }
     float sin_d, cos_d;
     sincosf(delta, &sin_d, &cos_d);
-    const float cos_lat = cos_hu * cos_d - sin_hu * sin_d;
-    const float sin_lat = clamp01(sin_hu * cos_d + cos_hu * sin_d);
+    return {cos_hu * cos_d - sin_hu * sin_d, clamp01(sin_hu * cos_d + cos_hu * sin_d)};
+}
+__device__ inline float sky_view_nu(const RenderDev& R, const SkyViewLatitude& lat, int ix, int w) {
+    const float x_lon = float(ix) / float(w - 1);
     const float cos_lon = -(x_lon * x_lon * 2.0f - 1.0f);
     const float sin_lon = clamp01(2.0f * x_lon * sqrtf(fmaxf(1.0f - x_lon * x_lon, 0.0f)));
     // GetViewDirectionFromCosLatLon (:104-111)
-    const F3 view = R.up * cos_lat + R.front * (sin_lat * cos_lon) + R.right * (sin_lat * sin_lon);
-    SkyViewRay ray{RayStart{r, alt0, cos_lat, dot(R.sun, R.up), dot(view, R.sun)}, 0.0f, 0.5f};
+    const F3 view = R.up * lat.cos_lat + R.front * (lat.sin_lat * cos_lon) + R.right * (lat.sin_lat * sin_lon);
+    return dot(view, R.sun);
+}
+
+// The ray of one sky-view texel (:74-186): its start, marching distance (0: nothing to
+// integrate) and the float counter's start value.
+struct SkyViewRay {
+    RayStart s;
+    float dist, start_i;
+};
+__device__ inline SkyViewRay sky_view_ray(const AtmDev& A, const RenderDev& R, const uint16_t* __restrict__ blue_noise,
+                                          int bn_size, int ix, int iy, int w, int h) {
+    const SkyViewLatitude lat = sky_view_latitude(A, R, iy, h);
+    const float r = R.r, alt0 = r - A.rb;
+    SkyViewRay ray{RayStart{r, alt0, lat.cos_lat, dot(R.sun, R.up), sky_view_nu(R, lat, ix, w)}, 0.0f, 0.5f};
     const bool hit = ray_hits_ground(A, r, alt0, ray.s.mu);
     ray.dist = hit ? distance_to_bottom(A, r, alt0, ray.s.mu) : distance_to_top(A, r, alt0, ray.s.mu);
     start_from_space(A, ray.s, ray.dist);
