@@ -139,13 +139,6 @@ __global__ __launch_bounds__(64 * kWaves) void batch_multiscattering_kernel(
     }
 }
 
-// A pointer the compiler takes for a new one, so that what is read through it is not kept from before.
-template <class B>
-__device__ __forceinline__ const B* reload(const B* p) {
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
 // A tile is whole rows of a view, each taken by the workgroup's waves in pieces of 64 to 192 columns.
 // Bound by vector instructions (97 % of the issue slots).  256 sets x 8 suns: 2.9 ms, 11.2 ms with
 // every texel marching for itself; three rays per lane against six 2.9 / 4.3 ms (six leave two waves

@@ -331,6 +331,13 @@ __host__ __device__ inline int row_rays_per_lane(int w) {
     return w <= 64 ? 1 : idle3 <= idle2 ? 3 : 2;
 }
 
+// A pointer the compiler takes for a new one, so that what is read through it is not kept from before.
+template <class B>
+__device__ __forceinline__ const B* reload(const B* p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // The wave's bounds of P values per lane.
 template <int P>
 __device__ inline void wave_bounds(const float (&v)[P], float& lo, float& hi) {

@@ -11,6 +11,7 @@ import pytest
 import oracle
 from skyrendering_amd import Atmosphere, AtmosphereRenderer, AtmosphereRenderInitParameters, presets
 from skyrendering_amd.atmosphere import AtmosphereRenderParameters
+from skyrendering_amd import surrogate as sg
 from skyrendering_amd.batch import LutBatch
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +79,33 @@ def test_multiscattering_tables_match_oracle(ctx, size, steps, radius):
     batch.launch()
     ctx.synchronize()
     assert np.array_equal(batch.set_outputs(0)[1], ms)
+
+
+@pytest.mark.parametrize("w,h,steps,t_size,ms_size", [(16, 16, 30.0, (256, 64), (32, 32)), (1, 1, 32.0, (64, 16), (8, 8)),
+                                                      (37, 50, 33.0, (64, 16), (16, 16)),
+                                                      (50, 17, 0.5, (64, 16), (16, 16)),
+                                                      (275, 33, 70.5, (288, 16), (33, 8))])
+def test_panorama_tiles_and_probes_match_oracle(ctx, w, h, steps, t_size, ms_size):
+    """The plain pass's tiles (ragged edges, more steps than a table, a count of 0) and the residual check's
+    probes, by rows and, for LUTs past a wave's entries, one by one, against the FP64 oracle."""
+    scales, views = sg.evaluation_views(2, seed=5)
+    atm = sg.SkyAtmospheres(ctx, scales, t_size=t_size, ms_size=ms_size, steps=steps)
+    pano = sg.SkyPanoramas(ctx, atm, views, w, h)
+    blocks, T, MS = atm.host_luts()
+    ys, xs = (v.ravel() for v in np.meshgrid(np.arange(h), np.arange(w), indexing="ij"))
+    refs = [oracle.sky_radiance(blocks, T, MS, steps, pano.pixel_queries(v, xs, ys)).reshape(h, w, 3) for v in range(2)]
+    # Rays within 1e-3 rad of the horizon pass it on one side or the other by rounding.
+    mu = np.cos(np.pi * (np.arange(h) + 0.5) / h)
+    sure = [np.abs(np.arccos(mu) - np.pi / 2 - np.arccos(6360.0 / (6360.0 + v["altitude"]))) > 1e-3 for v in views]
+    pano.render_plain()
+    image = pano.image()[..., :3]
+    for v in range(2):
+        assert _rel(image[v][sure[v]], refs[v][sure[v]]) < TOL if steps > 0.5 else not image[v].any()
+    pano.render_surrogate(sg.SkySurrogate(ctx, seed=3), tolerance=1e30)
+    image = pano.image()[..., :3]
+    py = sorted({min(t + o, h - 1) for t in range(0, h, 16) for o in (4, 12)})
+    px = sorted({min(t + o, w - 1) for t in range(0, w, 16) for o in (4, 12)})
+    for v in range(2):
+        rows = [y for y in py if sure[v][y]]
+        got, ref = image[v][np.ix_(rows, px)], refs[v][np.ix_(rows, px)]
+        assert _rel(got, ref) < TOL if steps > 0.5 else not got.any()
