@@ -45,9 +45,8 @@ __global__ __launch_bounds__(64 * kMsTexels) void multiscattering_kernel(SkyhipA
     ms_row_tables(A, iy, h, tw, th, n, steps, totals);
     __syncthreads();
     if (ix >= w) return;
-    const MsRay ray = ms_ray(A, ix, iy, w, h, lane);
-    const F3 L = ms_row_steps<false>(T, tw, th, steps, n, ray, 0, n);
-    const float4 v = multiscattering_reduce(A, T, tw, th, ray, L, totals[lane >> 3].tr, totals[lane >> 3].lf);
+    const MsSun sun = ms_sun(ix, w, lane);
+    const float4 v = ms_row_reduce<false>(A, T, tw, th, totals, sun, ms_row_steps<false>(T, tw, th, steps, n, sun, 0, n));
     if (lane == 0) out[iy * w + ix] = v;
 }
 
@@ -153,50 +152,38 @@ __global__ __launch_bounds__(256) void set_transmittance_kernel(SkyhipAtmosphere
     if (part == 0) out[t] = make_float4(v.x, v.y, v.z, 1.0f);
 }
 
-// Multiple scattering with each direction's march split over kSetMsParts waves: wave p of a
-// texel's workgroup integrates part p of all 64 directions, waves 1.. leave their partial sums
-// in LDS, and wave 0 combines them in order and reduces over the directions as the per-pass
-// kernel does.
+// Multiple scattering with the steps of a texel's 64 directions split over kSetMsParts waves: the
+// workgroup builds the step tables (whose weights hold the transmittance up to each step, so parts
+// simply add), wave p marches part p, and wave 0 adds the parts in order and reduces over the
+// directions as the per-pass kernel does.  Marches of more than kMsMaxSteps steps take that kernel.
 constexpr int kSetMsParts = 4;
 __global__ __launch_bounds__(64 * kSetMsParts) void set_multiscattering_kernel(SkyhipAtmosphereBufferData b,
                                                                                const float4* __restrict__ T, int tw,
                                                                                int th, float4* __restrict__ out,
                                                                                int w, int h) {
     constexpr int P = kSetMsParts;
-    __shared__ float part_sums[P - 1][9][64];
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MsTotals totals[kMsThetas];
+    __shared__ float part_sums[P - 1][3][64];
+    MsStep* steps = reinterpret_cast<MsStep*>(smem);
     const AtmDev A = make_atm(b);
-    const int texel = blockIdx.x, part = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const MsRay ray = ms_ray(A, texel % w, texel / w, w, h, lane);
-    int n = 0;
-    for (float i = 0.5f; i < A.ms_steps; i += 1.0f) ++n;
-    const int c = (n + P - 1) / P, first = min(part * c, n);
-    const ScatterRay sc = scatter_ray<true>(A, ray.s, ray.dist, A.ms_steps);
-    F3 L, Tr, Lf;
-    scattered_luminance_part_ms(A, T, tw, th, ray.s, sc, 0.5f + float(first), max(0, min(c, n - first)), L, Tr, Lf);
+    const int ix = blockIdx.x, iy = blockIdx.y, part = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int n = row_step_count(A.ms_steps);
+    ms_row_tables(A, iy, h, tw, th, n, steps, totals);
+    const MsSun sun = ms_sun(ix, w, lane);
+    __syncthreads();
+    const int c = (n + P - 1) / P;
+    F3 L = ms_row_steps<false>(T, tw, th, steps, n, sun, min(part * c, n), min(part * c + c, n));
     if (part > 0) {
-        const float v[9] = {L.x, L.y, L.z, Tr.x, Tr.y, Tr.z, Lf.x, Lf.y, Lf.z};
-        for (int k = 0; k < 9; ++k) part_sums[part - 1][k][lane] = v[k];
+        part_sums[part - 1][0][lane] = L.x;
+        part_sums[part - 1][1][lane] = L.y;
+        part_sums[part - 1][2][lane] = L.z;
     }
     __syncthreads();
     if (part != 0) return;
-    F3 aL = f3(0.0f), aT = f3(1.0f), aF = f3(0.0f);  // the parts after this one, combined
-    for (int p = P - 1; p >= 1; --p) {
-        const F3 pL = {part_sums[p - 1][0][lane], part_sums[p - 1][1][lane], part_sums[p - 1][2][lane]};
-        const F3 pT = {part_sums[p - 1][3][lane], part_sums[p - 1][4][lane], part_sums[p - 1][5][lane]};
-        const F3 pF = {part_sums[p - 1][6][lane], part_sums[p - 1][7][lane], part_sums[p - 1][8][lane]};
-        if (p == P - 1) {
-            aL = pL, aT = pT, aF = pF;
-        } else {
-            aL = pL + pT * aL;
-            aF = pF + pT * aF;
-            aT = pT * aT;
-        }
-    }
-    L = L + Tr * aL;
-    Lf = Lf + Tr * aF;
-    Tr = Tr * aT;
-    const float4 v = multiscattering_reduce(A, T, tw, th, ray, L, Tr, Lf);
-    if (lane == 0) out[texel] = v;
+    for (int p = 0; p < P - 1; ++p) L += F3{part_sums[p][0][lane], part_sums[p][1][lane], part_sums[p][2][lane]};
+    const float4 v = ms_row_reduce<false>(A, T, tw, th, totals, sun, L);
+    if (lane == 0) out[iy * w + ix] = v;
 }
 
 // Blocks [0, sv_blocks) build the sky view, kSetSkyViewParts lanes per texel; the rest the
@@ -438,10 +425,15 @@ extern "C" int skyhip_atmosphere_lut_set(SkyhipContext* ctx, const SkyhipAtmosph
     hipLaunchKernelGGL(set_transmittance_kernel, dim3(div_up((long long)tw * th * kSetTransmittanceParts, 256)),
                        dim3(256), 0, st, *atmosphere, reinterpret_cast<float4*>(transmittance_rgba), tw, th);
     SKYHIP_LAUNCH_CHECK("set_transmittance_kernel");
-    hipLaunchKernelGGL(set_multiscattering_kernel, dim3(mw * mh), dim3(64 * kSetMsParts), 0, st, *atmosphere,
-                       reinterpret_cast<const float4*>(transmittance_rgba), tw, th,
-                       reinterpret_cast<float4*>(multiscattering_rgba), mw, mh);
-    SKYHIP_LAUNCH_CHECK("set_multiscattering_kernel");
+    if (row_step_count(atmosphere->multiscattering_steps) <= kMsMaxSteps) {
+        hipLaunchKernelGGL(set_multiscattering_kernel, dim3(mw, mh), dim3(64 * kSetMsParts),
+                           ms_table_bytes(atmosphere->multiscattering_steps), st, *atmosphere,
+                           reinterpret_cast<const float4*>(transmittance_rgba), tw, th,
+                           reinterpret_cast<float4*>(multiscattering_rgba), mw, mh);
+        SKYHIP_LAUNCH_CHECK("set_multiscattering_kernel");
+    } else {
+        SKYHIP_CHECK(launch_multiscattering(st, *atmosphere, transmittance_rgba, tw, th, multiscattering_rgba, mw, mh));
+    }
     // Whole waves of 64 / parts groups each (a group never straddles two waves).
     const int sv_blocks = int(div_up(div_up((long long)sky_view_width * sky_view_height, 64 / kSetSkyViewParts) * 64, 256));
     const int ap_blocks =

@@ -128,9 +128,9 @@ __global__ __launch_bounds__(64 * kWaves) void batch_multiscattering_kernel(
         for (int ix = x0 + wave; ix < min(x0 + kMsTileTexels * kWaves, S.mw); ix += kWaves) {  // wave-uniform
             float4 v;
             if (tables) {
-                const MsRay ray = ms_ray(A, ix, iy, S.mw, S.mh, lane);
-                const F3 L = ms_row_steps<true>(T, S.tw, S.th, steps, n, ray, 0, n);
-                v = multiscattering_reduce<true>(A, T, S.tw, S.th, ray, L, totals[lane >> 3].tr, totals[lane >> 3].lf);
+                const MsSun sun = ms_sun(ix, S.mw, lane);
+                v = ms_row_reduce<true>(A, T, S.tw, S.th, totals, sun,
+                                        ms_row_steps<true>(T, S.tw, S.th, steps, n, sun, 0, n));
             } else {
                 v = multiscattering_texel<true>(A, T, S.tw, S.th, ix, iy, S.mw, S.mh, lane);
             }

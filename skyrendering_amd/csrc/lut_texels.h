@@ -116,23 +116,28 @@ struct MsRay {
     float dist;
     bool hit;
 };
-__device__ inline MsRay ms_ray(const AtmDev& A, int ix, int iy, int w, int h, int lane) {
+// The sun of a texel column as a direction sees it.
+struct MsSun {
+    float mu_s0, nu;
+};
+__device__ inline MsSun ms_sun(int ix, int w, int lane) {
     // GetAltitudeMuSFromMultiscatteringTextureIndex
-    const float altitude = (float(iy) / float(h - 1)) * A.thickness;
     const float mu_s = (float(ix) / float(w - 1)) * 2.0f - 1.0f;
     const float sun_z = sqrtf(1.0f - mu_s * mu_s);
-    // GetDirectionFromLocalIndex
-    const float unit_theta = (0.5f + float(lane >> 3)) / 8.0f;
-    const float unit_phi = (0.5f + float(lane & 7)) / 8.0f;
-    const float cos_theta = 1.0f - 2.0f * unit_theta;
+    // GetDirectionFromLocalIndex: polar angles acos(1 - 2 (0.5 + t) / 8), azimuths pi / 8 (2 p + 1), of
+    // which only the sine enters (the sun has x = 0).
+    const float cos_theta = 1.0f - 2.0f * ((0.5f + float(lane >> 3)) / 8.0f);
     const float sin_theta = sqrtf(clamp01(1.0f - cos_theta * cos_theta));
-    float sin_phi, cos_phi;
-    sincosf(2.0f * kPiF * unit_phi, &sin_phi, &cos_phi);
-    const F3 view = {cos_phi * sin_theta, cos_theta, sin_phi * sin_theta};
-
+    const int p = lane & 7;
+    const float s = ((p + 1) & 2) ? 0.92387953251128675613f : 0.38268343236508977173f;  // sin 3 pi / 8, sin pi / 8
+    return {mu_s, cos_theta * mu_s + (p < 4 ? s : -s) * sin_theta * sun_z};
+}
+__device__ inline MsRay ms_ray(const AtmDev& A, int ix, int iy, int w, int h, int lane) {
+    const float altitude = (float(iy) / float(h - 1)) * A.thickness;
     const float r = altitude + A.rb;
-    const float mu = view.y;
-    const float nu = view.y * mu_s + view.z * sun_z;
+    const float mu = 1.0f - 2.0f * ((0.5f + float(lane >> 3)) / 8.0f);
+    const MsSun sun = ms_sun(ix, w, lane);
+    const float mu_s = sun.mu_s0, nu = sun.nu;
     const bool hit = ray_hits_ground(A, r, altitude, mu);
     const float dist = hit ? distance_to_bottom(A, r, altitude, mu) : distance_to_top(A, r, altitude, mu);
     return {RayStart{r, altitude, mu, mu_s, nu}, dist, hit};

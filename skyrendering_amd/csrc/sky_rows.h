@@ -427,8 +427,10 @@ inline size_t ms_table_bytes(float ms_steps) {
     const int n = row_step_count(ms_steps);
     return n > kMsMaxSteps ? 0 : size_t(kMsThetas) * n * sizeof(MsStep);
 }
-struct MsTotals {                // per polar angle: transmittance and multiple-scattering transfer
+struct MsTotals {                // per polar angle: transmittance, multiple-scattering transfer, the ray
     F3 tr, lf;
+    float r, dist;
+    bool hit;
 };
 
 // The zenith cosine of polar angle t (ms_ray's, for lanes 8 t .. 8 t + 7).
@@ -465,25 +467,34 @@ __device__ inline void ms_row_tables(const AtmDev& A, int iy, int h, int tw, int
                 d.c[3] = make_float4(s.ty, 0.0f, 0.0f, 0.0f);
             }
         }
-        if ((e & 31) == 0) totals[t] = {tr, lf};
+        if ((e & 31) == 0) totals[t] = {tr, lf, r, ray.dist, hit};
     }
 }
 
 // Steps [first, last) of a texel's 64 directions (the lane's): the luminance they add.
 template <bool kCells>
 __device__ __forceinline__ F3 ms_row_steps(const float4* __restrict__ T, int tw, int th, const MsStep* steps, int n,
-                                           const MsRay& ray, int first, int last) {
+                                           const MsSun& sun, int first, int last) {
     F3 L = f3(0.0f);
     const MsStep* row = steps + ((threadIdx.x & 63) >> 3) * n;
 #pragma unroll 2
     for (int j = first; j < last; ++j) {
         const float4 c0 = row[j].c[0], c1 = row[j].c[1], c2 = row[j].c[2];
-        const float mu_s = fmaf(c0.y, ray.s.nu, c0.x * ray.s.mu_s0);
+        const float mu_s = fmaf(c0.y, sun.nu, c0.x * sun.mu_s0);
         const float tx = sun_column(c1.x, c0.z, c0.w, c1.y, c1.z, mu_s);
         const F3 V = lut_bilinear<kCells>(T, tw, th, tx, row[j].c[3].x) * sun_fade(c1.w, c2.w, mu_s);
         L = fma3(F3{c2.x, c2.y, c2.z}, V, L);
     }
     return L;
+}
+
+// A row texel from the luminance of its 64 directions (ms_row_steps'; the lane's).  Valid in lane 0.
+template <bool kCells>
+__device__ __forceinline__ float4 ms_row_reduce(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
+                                                const MsTotals* totals, const MsSun& sun, F3 L) {
+    const MsTotals t = totals[(threadIdx.x & 63) >> 3];
+    const MsRay ray{RayStart{t.r, 0.0f, 0.0f, sun.mu_s0, sun.nu}, t.dist, t.hit};
+    return multiscattering_reduce<kCells>(A, T, tw, th, ray, L, t.tr, t.lf);
 }
 
 }  // namespace skyhip
