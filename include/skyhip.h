@@ -1036,7 +1036,7 @@ int skyhip_surrogate_gradient(SkyhipContext* ctx, int32_t network, const float* 
  * cannot allocate (code under HIP graph capture, tight training loops, harnesses that forbid
  * hipMalloc).  No reference counterpart.  The partial gradients live in a fixed device array, one
  * per GPU, resolved when a context is created on that GPU and held until the process ends
- * (13.5 MB); count must be at most SKYHIP_SURROGATE_NOALLOC_MAX_COUNT (larger counts fail with
+ * (6.8 MB); count must be at most SKYHIP_SURROGATE_NOALLOC_MAX_COUNT (larger counts fail with
  * SKYHIP_ERR_INVALID_SIZE; use skyhip_surrogate_gradient).  All calls on one GPU share the array:
  * calls that overlap on one GPU (on different streams or from different threads) race. */
 #define SKYHIP_SURROGATE_NOALLOC_MAX_COUNT 8192

@@ -21,9 +21,9 @@
 //    a layer's accumulators (rows = neurons, columns = samples) become the next layer's
 //    B operand in place, the k order inside each 32-wide block being permuted to match
 //    the accumulator layout (the weights are loaded with the same permutation).
-//  - surrogate_train_kernel: forward and backward for 32 samples per workgroup with
-//    LDS-staged FP16 operands (any transpose is an LDS stride), writing the workgroup's
-//    gradient to its own slice (no atomics; the reduction order is fixed).  The deltas
+//  - surrogate_train_kernel: forward and backward for 16 samples per wave in registers, the
+//    weight gradients over a workgroup's 64 from LDS, written to the workgroup's own slice (no
+//    atomics; the reduction order is fixed).  The deltas
 //    are kept without the loss scale (2 w (y - t) and its back-propagation, well inside
 //    FP16's range) and the scale multiplies the gradient sums.
 //  - surrogate_reduce_kernel / surrogate_adam_kernel: gradient sum and Adam update.
@@ -316,16 +316,12 @@ __device__ __forceinline__ f32x4 mlp_forward16(const MlpRegs<Net>& R, const floa
 }
 
 // Biases b1..b4 at 64 (l - 1), b5 at 256 (3 used, zero to 271).
+__device__ __forceinline__ float mlp_bias(const float* __restrict__ p, int i) {
+    const int l = i >> 6, at = l == 0 ? kOffB1 : l == 1 ? kOffB2 : l == 2 ? kOffB3 : l == 3 ? kOffB4 : kOffB5;
+    return i < 259 ? p[at + (i & 63)] : 0.0f;
+}
 __device__ inline void load_biases(const float* __restrict__ p, float* s_bias) {
-    for (int i = threadIdx.x; i < 272; i += blockDim.x) {
-        float v = 0.0f;
-        if (i < 64) v = p[kOffB1 + i];
-        else if (i < 128) v = p[kOffB2 + i - 64];
-        else if (i < 192) v = p[kOffB3 + i - 128];
-        else if (i < 256) v = p[kOffB4 + i - 192];
-        else if (i < 259) v = p[kOffB5 + i - 256];
-        s_bias[i] = v;
-    }
+    for (int i = threadIdx.x; i < 272; i += blockDim.x) s_bias[i] = mlp_bias(p, i);
     __syncthreads();
 }
 
@@ -361,159 +357,279 @@ __global__ __launch_bounds__(256, 2) void surrogate_forward_kernel(const float* 
 }
 
 // ---------------------------------------------------------------------------
-// Training: 32 samples per workgroup, LDS-staged operands.
+// Training: 64 samples per workgroup.  Each wave takes 16 of them through the forward and backward
+// chains in registers: as in inference, a layer's accumulators (rows = neurons, columns = samples)
+// become the next operand in place, forward with the weights and backward with their transposes, so
+// the chain needs no barrier.  The activations and deltas also go to LDS, neuron-major; after one
+// barrier every wave forms 16 rows of each weight gradient from them, over the 64 samples.  Bias
+// gradients are products with a column of ones.
+//
+// Bound by latency: the 8,192-sample step is 128 workgroups of a few thousand cycles each, then 6.8 MB of
+// partial gradients.  BF16 at 8,192 samples: 15.6 us, 34.6 with 32 samples per workgroup, every
+// operand gathered from LDS element by element and a barrier per layer (256 partial gradients).
 // ---------------------------------------------------------------------------
-constexpr int kTS = 32;  // samples per workgroup
-
-// C[M x N] = A[M x K] B[K x N] with FP16 LDS operands at element strides
-// A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn]; 16 x 16 tiles spread over
-// the workgroup's waves, K a multiple of 32.  ep(m, n, value) consumes each output once.
-template <class Net, class Ep>
-__device__ inline void lds_gemm(const typename Net::T* A, int sam, int sak, const typename Net::T* B, int sbk, int sbn,
-                                int M, int N,
-                                int K, Ep ep) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-    const int q = lane >> 4, r = lane & 15;
-    const int tn_count = N / 16;
-    for (int t = wave; t < (M / 16) * tn_count; t += nw) {
-        const int m0 = (t / tn_count) * 16, n0 = (t % tn_count) * 16;
-        f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k0 = 0; k0 < K; k0 += 32) {
-            typename Net::V8 a, b;
-            for (int i = 0; i < 8; ++i) {
-                const int k = k0 + 8 * q + i;
-                a[i] = A[(m0 + r) * sam + k * sak];
-                b[i] = B[k * sbk + (n0 + r) * sbn];
-            }
-            c = Net::mfma(a, b, c);
-        }
-        for (int i = 0; i < 4; ++i) ep(m0 + 4 * q + i, n0 + r, c[i]);
-    }
-}
+constexpr int kTS = 64;         // samples per workgroup and round
+constexpr int kTrainWaves = 4;  // of 16 samples each
+constexpr int kMaxTrainGroups = 256;
+constexpr int kTRow = 72;       // row stride of the 64-wide LDS matrices: 16-byte rows that start in different banks
 
 template <class T>
 struct TrainLds {
-    T w1[64 * 32];   // [neuron][input] (inputs 7..31 zero)
-    T wh[3][64 * 64];
-    T w5[32 * 64];   // [output][neuron] (outputs 3..31 zero)
-    T x[32 * kTS];   // [input][sample]
-    float z[4][64 * kTS]; // pre-activations [neuron][sample]
-    T a[4][64 * kTS];
-    float y[16 * kTS];
-    T d5[32 * kTS];  // output deltas 2 w (y - t) [output][sample] (rows 3..31 zero)
-    T d[2][64 * kTS];  // hidden deltas (without the loss scale)
+    T w1[64][8];             // [neuron][input]
+    T wh[3][64][kTRow];      // [neuron][input]
+    T wt[3][64][kTRow];      // transposed
+    T w5[16][kTRow];         // [output][neuron] (outputs 3..15 zero)
+    T w5t[64][8];            // [neuron][output] (outputs 3..7 zero)
+    T x[16][kTRow];          // [input][sample]; input 7 is 1 (the bias), 8..15 zero
+    T a[4][64][kTRow];       // activations [neuron][sample]
+    T d[4][64][kTRow];       // hidden deltas (without the loss scale) [neuron][sample]
+    T d5[16][kTRow];         // output deltas 2 w (y - t) [output][sample] (rows 3..15 zero)
     float bias[272];
-    float loss;
+    float loss[kTrainWaves];
 };
 
+// The operand whose lane (r, q) holds row r's columns permuted_neuron(b, q, 0 .. 7) of a matrix in LDS.
 template <class Net>
-__global__ __launch_bounds__(256) void surrogate_train_kernel(const float* __restrict__ params,
-                                                              const float* __restrict__ feats,
-                                                              const float* __restrict__ targets,
-                                                              const float* __restrict__ weights, int n,
-                                                              float loss_scale, float* __restrict__ partial,
-                                                              float* __restrict__ partial_loss) {
+__device__ __forceinline__ typename Net::V8 permuted_operand(const typename Net::T (*m)[kTRow], int r, int b, int q) {
+    typedef typename Net::T T;
+    typedef T V4 __attribute__((ext_vector_type(4)));
+    const V4 lo = *reinterpret_cast<const V4*>(&m[r][32 * b + 4 * q]),
+             hi = *reinterpret_cast<const V4*>(&m[r][32 * b + 16 + 4 * q]);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Stores the chain's next operand (h[b][i]: neuron permuted_neuron(b, q, i) of sample column s).
+template <class Net>
+__device__ __forceinline__ void store_operand(typename Net::T (*m)[kTRow], const typename Net::V8 h[2], int q, int s) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m[permuted_neuron(b, q, i)][s] = h[b][i];
+}
+
+// Sample s as its lanes q == 0 hold it (zero, with weight 0, past the last).
+struct TrainSample {
+    float x[7], t[3], w;
+};
+__device__ __forceinline__ TrainSample train_sample(const float* __restrict__ feats, const float* __restrict__ targets,
+                                                    const float* __restrict__ weights, int s, int n, int q) {
+    TrainSample v = {};
+    if (q == 0 && s < n) {
+#pragma unroll
+        for (int k = 0; k < 7; ++k) v.x[k] = feats[8ll * s + k];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) v.t[m] = targets[3ll * s + m];
+        v.w = weights ? weights[s] : 1.0f;
+    }
+    return v;
+}
+
+template <class Net>
+__global__ __launch_bounds__(64 * kTrainWaves, 1) void surrogate_train_kernel(
+    const float* __restrict__ params, const float* __restrict__ feats, const float* __restrict__ targets,
+    const float* __restrict__ weights, int n, float loss_scale, float* __restrict__ partial,
+    float* __restrict__ partial_loss) {
     extern __shared__ __align__(16) unsigned char smem[];
     typedef typename Net::T T;
+    typedef typename Net::V8 V8;
     TrainLds<T>& S = *reinterpret_cast<TrainLds<T>*>(smem);
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int s0 = blockIdx.x * kTS;
-    float* G = partial + (long long)blockIdx.x * kParams;
-    // Weights to FP16 (zero padding), inputs, biases.
-    for (int i = tid; i < 64 * 32; i += nt) {
-        int m = i / 32, k = i % 32;
-        S.w1[i] = (T)(k < 7 ? params[kOffW1 + m * 7 + k] : 0.0f);
-    }
+    const int tid = threadIdx.x, nt = 64 * kTrainWaves;
+    const int wave = tid >> 6, lane = tid & 63, q = lane >> 4, r = lane & 15;
+    // Weights to 16 bits (zero padding), all their loads on the way together.  A thread takes four rows
+    // of a column, four columns apart, so that its transposed stores are four neighbours.
     const int offs[3] = {kOffW2, kOffW3, kOffW4};
+    float hidden[3][4][4];
+    const int wc = tid & 63, wr = 4 * (tid >> 6);  // column; rows wr + 16 j + c
+#pragma unroll
     for (int L = 0; L < 3; ++L)
-        for (int i = tid; i < 64 * 64; i += nt) S.wh[L][i] = (T)params[offs[L] + i];
-    for (int i = tid; i < 32 * 64; i += nt) S.w5[i] = (T)(i < 3 * 64 ? params[kOffW5 + i] : 0.0f);
-    for (int i = tid; i < 32 * kTS; i += nt) {
-        int k = i / kTS, s = i % kTS;
-        S.x[i] = (T)((k < 8 && s0 + s < n) ? feats[8 * (s0 + s) + k] : 0.0f);
-        S.d5[i] = (T)0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) hidden[L][j][c] = params[offs[L] + (wr + 16 * j + c) * 64 + wc];
+    float w1[2], w5 = 0.0f, bias2[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int i = tid + nt * c, m = i >> 3, k = i & 7;  // 512 = 64 x 8
+        w1[c] = k < 7 ? params[kOffW1 + m * 7 + k] : 0.0f;
+        bias2[c] = i < 272 ? mlp_bias(params, i) : 0.0f;
     }
-    if (tid == 0) S.loss = 0.0f;
-    load_biases(params, S.bias);  // synchronises
-    // Forward.
-    lds_gemm<Net>(S.w1, 32, 1, S.x, kTS, 1, 64, kTS, 32, [&](int m, int s, float c) {
-        float z = c + S.bias[m];
-        S.z[0][m * kTS + s] = z;
-        S.a[0][m * kTS + s] = Net::act(z);
-    });
+    if (tid < 192) w5 = params[kOffW5 + tid];
+    TrainSample next = train_sample(feats, targets, weights, blockIdx.x * kTS + 16 * wave + r, n, q);
+    for (int i = tid; i < 64 * 8; i += nt) S.w5t[i >> 3][i & 7] = (T)0.0f;
+    for (int i = tid; i < 16 * kTRow; i += nt) {
+        const int m = i / kTRow, k = i - m * kTRow;
+        S.w5[m][k] = (T)0.0f;
+        S.x[m][k] = (T)(m == 7 ? 1.0f : 0.0f);
+        S.d5[m][k] = (T)0.0f;
+    }
+#pragma unroll
+    for (int L = 0; L < 3; ++L)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            typedef T V4 __attribute__((ext_vector_type(4)));
+            V4 v;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                v[c] = (T)hidden[L][j][c];
+                S.wh[L][wr + 16 * j + c][wc] = v[c];
+            }
+            *reinterpret_cast<V4*>(&S.wt[L][wc][wr + 16 * j]) = v;
+        }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int i = tid + nt * c;
+        S.w1[i >> 3][i & 7] = (T)w1[c];
+        if (i < 272) S.bias[i] = bias2[c];
+    }
+    __syncthreads();  // the zeros under w5's rows
+    if (tid < 192) S.w5[tid >> 6][tid & 63] = S.w5t[tid & 63][tid >> 6] = (T)w5;
     __syncthreads();
+
+    V8 ones, zeros = {};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = (T)1.0f;
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 gh[3][4], gb[3], g1 = zero4, g5 = zero4, gb5 = zero4;  // this wave's rows (columns of layer 5's)
+#pragma unroll
     for (int L = 0; L < 3; ++L) {
-        lds_gemm<Net>(S.wh[L], 64, 1, S.a[L], kTS, 1, 64, kTS, 64, [&](int m, int s, float c) {
-            float z = c + S.bias[64 * (L + 1) + m];
-            S.z[L + 1][m * kTS + s] = z;
-            S.a[L + 1][m * kTS + s] = Net::act(z);
-        });
-        __syncthreads();
+        gb[L] = zero4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) gh[L][j] = zero4;
     }
-    lds_gemm<Net>(S.w5, 64, 1, S.a[3], kTS, 1, 16, kTS, 64,
-             [&](int m, int s, float c) { S.y[m * kTS + s] = c + S.bias[256 + m]; });
-    __syncthreads();
-    // Loss loss_scale * sum w (y - t)^2 and the output deltas 2 w (y - t); the gradient
-    // sums below multiply by loss_scale.
-    for (int i = tid; i < 3 * kTS; i += nt) {
-        int m = i / kTS, s = i % kTS;
-        float d = 0.0f, w = 0.0f;
-        if (s0 + s < n) {
-            d = S.y[m * kTS + s] - targets[3 * (s0 + s) + m];
-            w = weights ? weights[s0 + s] : 1.0f;
+    float loss = 0.0f;
+    const int s = wave * 16 + r;  // this lane's sample column
+    for (int s0 = blockIdx.x * kTS; s0 < n; s0 += gridDim.x * kTS) {  // workgroup-uniform
+        const TrainSample sample = next;
+        if (s0 + int(gridDim.x) * kTS < n)
+            next = train_sample(feats, targets, weights, s0 + int(gridDim.x) * kTS + s, n, q);
+        // Forward.
+        V8 x = zeros;
+        if (q == 0) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) {
+                x[k] = (T)sample.x[k];
+                S.x[k][s] = x[k];
+            }
         }
-        atomicAdd(&S.loss, w * d * d * loss_scale);
-        S.d5[m * kTS + s] = (T)(2.0f * w * d);
-    }
-    __syncthreads();
-    // Output layer gradient: dW5 = d5 a4^T, db5 = sum d5.
-    lds_gemm<Net>(S.d5, kTS, 1, S.a[3], 1, kTS, 16, 64, kTS, [&](int m, int k, float c) {
-        if (m < 3) G[kOffW5 + m * 64 + k] = c * loss_scale;
-    });
-    for (int m = tid; m < 3; m += nt) {
-        float sum = 0.0f;
-        for (int s = 0; s < kTS; ++s) sum += float(S.d5[m * kTS + s]);
-        G[kOffB5 + m] = sum * loss_scale;
-    }
-    // delta4 = (W5^T d5) * a'(z4)
-    lds_gemm<Net>(S.w5, 1, 64, S.d5, kTS, 1, 64, kTS, 32, [&](int m, int s, float c) {
-        S.d[0][m * kTS + s] = (T)(c * Net::act_grad(S.z[3][m * kTS + s]));
-    });
-    __syncthreads();
-    // Hidden layers 4, 3, 2 (weights wh[2], wh[1], wh[0]).
-    const int woffs[3] = {kOffW2, kOffW3, kOffW4}, boffs[4] = {kOffB1, kOffB2, kOffB3, kOffB4};
-    int cur = 0;
-    for (int L = 2; L >= 0; --L) {
-        const T* dl = S.d[cur];
-        // dW = delta a_prev^T ; a_prev = a[L] (input of wh[L])
-        lds_gemm<Net>(dl, kTS, 1, S.a[L], 1, kTS, 64, 64, kTS,
-                 [&](int m, int k, float c) { G[woffs[L] + m * 64 + k] = c * loss_scale; });
-        for (int m = tid; m < 64; m += nt) {
-            float sum = 0.0f;
-            for (int s = 0; s < kTS; ++s) sum += float(dl[m * kTS + s]);
-            G[boffs[L + 1] + m] = sum * loss_scale;
+        f32x4 z[4][4];
+        V8 h[2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float* bias = S.bias + 16 * j + 4 * q;
+            const V8 w = q == 0 ? *reinterpret_cast<const V8*>(S.w1[16 * j + r]) : zeros;
+            z[0][j] = Net::mfma(w, x, f32x4{bias[0], bias[1], bias[2], bias[3]});
         }
-        // delta_prev = (W^T delta) * a'(z[L])
-        T* dn = S.d[cur ^ 1];
-        lds_gemm<Net>(S.wh[L], 1, 64, dl, kTS, 1, 64, kTS, 64, [&](int m, int s, float c) {
-            dn[m * kTS + s] = (T)(c * Net::act_grad(S.z[L][m * kTS + s]));
-        });
+        activate<Net>(z[0], h);
+        store_operand<Net>(S.a[0], h, q, s);
+#pragma unroll
+        for (int L = 0; L < 3; ++L) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float* bias = S.bias + 64 * (L + 1) + 16 * j + 4 * q;
+                f32x4 c = {bias[0], bias[1], bias[2], bias[3]};
+                c = Net::mfma(permuted_operand<Net>(S.wh[L], 16 * j + r, 0, q), h[0], c);
+                z[L + 1][j] = Net::mfma(permuted_operand<Net>(S.wh[L], 16 * j + r, 1, q), h[1], c);
+            }
+            activate<Net>(z[L + 1], h);
+            store_operand<Net>(S.a[L + 1], h, q, s);
+        }
+        const float* bias5 = S.bias + 256 + 4 * q;
+        f32x4 y = {bias5[0], bias5[1], bias5[2], bias5[3]};
+        y = Net::mfma(permuted_operand<Net>(S.w5, r, 0, q), h[0], y);
+        y = Net::mfma(permuted_operand<Net>(S.w5, r, 1, q), h[1], y);
+        // Loss loss_scale * sum w (y - t)^2 and the output deltas 2 w (y - t); the gradient sums below
+        // multiply by loss_scale.
+        V8 dy = zeros;
+        if (q == 0) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const float e = s0 + s < n ? y[m] - sample.t[m] : 0.0f;
+                loss += sample.w * e * e * loss_scale;
+                dy[m] = (T)(2.0f * sample.w * e);
+                S.d5[m][s] = dy[m];
+            }
+        }
+        // Backward: the deltas of layer l, (W^T delta) a'(z_l), as the next operand.
+        V8 g[2];
+        const auto delta = [&](const f32x4 (&c)[4], const f32x4 (&zl)[4], T (*out)[kTRow]) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    g[b][i] = (T)(c[2 * b][i] * Net::act_grad(zl[2 * b][i]));
+                    g[b][4 + i] = (T)(c[2 * b + 1][i] * Net::act_grad(zl[2 * b + 1][i]));
+                }
+            store_operand<Net>(out, g, q, s);
+        };
+        f32x4 c[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            c[j] = Net::mfma(q == 0 ? *reinterpret_cast<const V8*>(S.w5t[16 * j + r]) : zeros, dy, zero4);
+        delta(c, z[3], S.d[3]);
+#pragma unroll
+        for (int L = 2; L >= 0; --L) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                c[j] = Net::mfma(permuted_operand<Net>(S.wt[L], 16 * j + r, 0, q), g[0], zero4);
+                c[j] = Net::mfma(permuted_operand<Net>(S.wt[L], 16 * j + r, 1, q), g[1], c[j]);
+            }
+            delta(c, z[L], S.d[L]);
+        }
         __syncthreads();
-        cur ^= 1;
+        // Weight gradients: wave w forms rows 16 w .. of each (columns of the output layer's), 32 samples a product.
+        const int m0 = 16 * wave + r;
+#pragma unroll
+        for (int k0 = 0; k0 < kTS; k0 += 32) {
+            const int k = k0 + 8 * q;
+#pragma unroll
+            for (int L = 0; L < 3; ++L) {
+                const V8 d = *reinterpret_cast<const V8*>(&S.d[L + 1][m0][k]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    gh[L][j] = Net::mfma(d, *reinterpret_cast<const V8*>(&S.a[L][16 * j + r][k]), gh[L][j]);
+                gb[L] = Net::mfma(d, ones, gb[L]);
+            }
+            g1 = Net::mfma(*reinterpret_cast<const V8*>(&S.d[0][m0][k]), *reinterpret_cast<const V8*>(&S.x[r][k]), g1);
+            const V8 d5 = *reinterpret_cast<const V8*>(&S.d5[r][k]);
+            g5 = Net::mfma(d5, *reinterpret_cast<const V8*>(&S.a[3][m0][k]), g5);
+            gb5 = Net::mfma(d5, ones, gb5);
+        }
+        __syncthreads();  // before the next round's stores
     }
-    // First layer: dW1 = delta1 x^T, db1.
-    const T* d1 = S.d[cur];
-    lds_gemm<Net>(d1, kTS, 1, S.x, 1, kTS, 64, 32, kTS, [&](int m, int k, float c) {
-        if (k < 7) G[kOffW1 + m * 7 + k] = c * loss_scale;
-    });
-    for (int m = tid; m < 64; m += nt) {
-        float sum = 0.0f;
-        for (int s = 0; s < kTS; ++s) sum += float(d1[m * kTS + s]);
-        G[kOffB1 + m] = sum * loss_scale;
+    // The workgroup's slice (lane (r, q): rows 4 q + i, column r of each product).
+    float* G = partial + (long long)blockIdx.x * kParams;
+    const int woffs[3] = {kOffW2, kOffW3, kOffW4}, boffs[3] = {kOffB2, kOffB3, kOffB4};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = 16 * wave + 4 * q + i;
+#pragma unroll
+        for (int L = 0; L < 3; ++L) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) G[woffs[L] + m * 64 + 16 * j + r] = gh[L][j][i] * loss_scale;
+            if (r == 0) G[boffs[L] + m] = gb[L][i] * loss_scale;
+        }
+        if (r < 7)
+            G[kOffW1 + m * 7 + r] = g1[i] * loss_scale;
+        else if (r == 7)
+            G[kOffB1 + m] = g1[i] * loss_scale;
+        if (q == 0 && i < 3) {
+            G[kOffW5 + i * 64 + 16 * wave + r] = g5[i] * loss_scale;
+            if (wave == 0 && r == 0) G[kOffB5 + i] = gb5[i] * loss_scale;
+        }
     }
+    for (int off = 8; off >= 1; off >>= 1) loss += __shfl_xor(loss, off, 64);  // lanes q == 0 hold the samples'
+    if (lane == 0) S.loss[wave] = loss;
     __syncthreads();
-    if (tid == 0) partial_loss[blockIdx.x] = S.loss;
+    if (tid == 0) {
+        float sum = 0.0f;
+        for (int w = 0; w < kTrainWaves; ++w) sum += S.loss[w];
+        partial_loss[blockIdx.x] = sum;
+    }
 }
+
+// Workgroups (partial gradients) of a training call: one per 64 samples, and at most one per CU of the
+// largest part, which then take several rounds each.
+__host__ inline int train_groups(int count) { return std::min(div_up(count, kTS), unsigned(kMaxTrainGroups)); }
 
 // grad[p] = sum over workgroups of partial[wg][p]; loss likewise (as parameter kParams).
 // A 1024-thread block covers 64 parameters x 16 ranges of workgroups: each thread sums
@@ -969,14 +1085,14 @@ extern "C" int skyhip_surrogate_forward(SkyhipContext* ctx, int32_t network, con
 
 extern "C" size_t skyhip_surrogate_workspace_bytes(int32_t count) {
     if (count <= 0) return 0;
-    size_t groups = size_t((count + kTS - 1) / kTS);
+    const size_t groups = size_t(train_groups(count));
     return groups * kParams * sizeof(float) + groups * sizeof(float);
 }
 
 namespace skyhip {
 
 // Launches the training kernels for `count` samples with the per-workgroup partial gradients
-// (div_up(count, kTS) x kParams floats, then one loss per workgroup) at `partial`; every
+// (train_groups(count) x kParams floats, then one loss per workgroup) at `partial`; every
 // workgroup writes its whole slice, so the buffer needs no clearing.
 static int gradient_launch(SkyhipContext* ctx, int32_t network, const float* params, const float* features,
                            const float* targets, const float* weights, int32_t count, float loss_scale,
@@ -993,13 +1109,13 @@ static int gradient_launch(SkyhipContext* ctx, int32_t network, const float* par
                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
         lds_ready = true;
     }
-    const int groups = div_up(count, kTS);
+    const int groups = train_groups(count);
     float* partial_loss = partial + (size_t)groups * kParams;
     if (network == SKYHIP_SURROGATE_F16_GATE)
-        hipLaunchKernelGGL(surrogate_train_kernel<NetF16Gate>, dim3(groups), dim3(256), lds_bytes, ctx->stream,
+        hipLaunchKernelGGL(surrogate_train_kernel<NetF16Gate>, dim3(groups), dim3(64 * kTrainWaves), lds_bytes, ctx->stream,
                            params, features, targets, weights, count, loss_scale, partial, partial_loss);
     else
-        hipLaunchKernelGGL(surrogate_train_kernel<NetBF16SiLU>, dim3(groups), dim3(256), lds_bytes, ctx->stream,
+        hipLaunchKernelGGL(surrogate_train_kernel<NetBF16SiLU>, dim3(groups), dim3(64 * kTrainWaves), lds_bytes, ctx->stream,
                            params, features, targets, weights, count, loss_scale, partial, partial_loss);
     SKYHIP_LAUNCH_CHECK("surrogate_train_kernel");
     hipLaunchKernelGGL(surrogate_reduce_kernel, dim3(div_up(kParams + 1, 64)), dim3(1024), 0, ctx->stream, partial,
@@ -1019,7 +1135,7 @@ static int check_gradient_args(SkyhipContext* ctx, int32_t network, const float*
 }
 
 // The allocation-free gradient's partial gradients: one copy of this array per GPU, held until the
-// process ends (13.5 MB: SKYHIP_SURROGATE_NOALLOC_MAX_COUNT / 32 workgroups x (13,187 + 1) floats).
+// process ends (6.8 MB: SKYHIP_SURROGATE_NOALLOC_MAX_COUNT / 64 workgroups x (13,187 + 1) floats).
 // Host code never uses the array's name as an address: surrogate_scratch_setup resolves each
 // device's copy with hipGetSymbolAddress when a context is created on it.
 constexpr int kNoAllocMaxGroups = SKYHIP_SURROGATE_NOALLOC_MAX_COUNT / kTS;
