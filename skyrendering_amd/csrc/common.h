@@ -98,6 +98,13 @@ __device__ inline float fast_exp(float x) { return __expf(x); }
 __device__ inline F3 fast_exp3(F3 v) { return {__expf(v.x), __expf(v.y), __expf(v.z)}; }
 __device__ inline float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+// Orders a wave's own LDS writes before its reads (and the reads before the next writes).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ inline float smoothstepf(float e0, float e1, float x) {
     float t = clamp01((x - e0) / (e1 - e0));
     return t * t * (3.0f - 2.0f * t);

@@ -516,41 +516,12 @@ __device__ __forceinline__ bool begin_path(const PtArgs& a, F3 view, PathState& 
     return a.max_bounces > 0;
 }
 
-// One iteration of Trace's bounce loop (:182-247).  False when the path ends in it (it leaves
-// the region, escapes, or reaches the bounce limit or zero throughput).
-template <int kMat, bool kBricks, bool kCount, bool kCells, bool kFlat>
-__device__ __forceinline__ bool bounce(Rng& rng, PathState& p, PtCount& wc) {
-    const PtArgs& a = kernel_args();
-    float t0, t1;
-    region(a, p.o, p.d, t0, t1);
-    if (t0 >= t1) return false;
-    float t;
-    if (!delta_track<kMat, kBricks, kCount, kCells, kFlat>(a, rng, p.o, p.d, t0, t1, t, wc)) {
-        if (a.env == SKYHIP_ENV_OFF || !p.has_scattered) return false;
-        if (a.env == SKYHIP_ENV_CONST_ENVIRONMENT_MAP) {
-            p.L += p.thr * environment(a, p.d);
-            return false;
-        }
-        const F3 o = p.o, d = p.d;
-        float q = o.x * o.x + o.y * o.y + o.z * (o.z + 2.0f * a.R) + (a.R - a.A.rb) * (a.R + a.A.rb);
-        float r = sqrtf(fmaxf(q + a.A.rb * a.A.rb, 0.0f));
-        float alt = q / (r + a.A.rb);
-        float mu = (d.x * o.x + d.y * o.y + d.z * (o.z + a.R)) / r;
-        if (!ray_hits_ground(a.A, r, alt, mu)) {
-            p.L += p.thr * environment(a, d);
-            return false;
-        }
-        p.o = o + d * distance_to_bottom(a.A, r, alt, mu);
-        F3 N = F3{p.o.x, p.o.y, p.o.z + a.R};
-        N = N * (1.0f / length3(N));
-        if (kCount) wc.vertices++;
-        F3 bsdf = a.A.albedo * ((1.0f / kPiF) * dot(N, a.sun));
-        p.L += p.thr * (ratio_track<kMat, kBricks, kCount, kCells, kFlat>(a, rng, p.o, a.sun, wc) * sun_illuminance(a, p.o) *
-                        bsdf);
-        if (a.env == SKYHIP_ENV_GROUND_SINGLE_BOUNCE) return false;
-        p.d = lambert_sample(rng, N);
-        p.thr *= a.A.albedo;
-    } else {
+// What a path does after its free flight (:197-247), in two parts around the shadow ray from p.o to the
+// sun.  The first takes the path to its collision at distance t, or out to the environment or the
+// ground; false when the path ends there.
+template <bool kCount>
+__device__ __forceinline__ bool flight_end(const PtArgs& a, PathState& p, bool hit, float t, PtCount& wc) {
+    if (hit) {
         if (!p.has_scattered) p.scattered_t = length3(p.o - a.cam);  // the segment start, as :232-233
         p.has_scattered = true;
         p.o = p.o + p.d * t;
@@ -558,13 +529,61 @@ __device__ __forceinline__ bool bounce(Rng& rng, PathState& p, PtCount& wc) {
         // A real collision scatters with probability albedo (the reference's is 1): the sun
         // estimate at this vertex and the continuation both carry it.
         p.thr = p.thr * a.albedo;
+        return true;
+    }
+    if (a.env == SKYHIP_ENV_OFF || !p.has_scattered) return false;
+    if (a.env == SKYHIP_ENV_CONST_ENVIRONMENT_MAP) {
+        p.L += p.thr * environment(a, p.d);
+        return false;
+    }
+    const F3 o = p.o, d = p.d;
+    float q = o.x * o.x + o.y * o.y + o.z * (o.z + 2.0f * a.R) + (a.R - a.A.rb) * (a.R + a.A.rb);
+    float r = sqrtf(fmaxf(q + a.A.rb * a.A.rb, 0.0f));
+    float alt = q / (r + a.A.rb);
+    float mu = (d.x * o.x + d.y * o.y + d.z * (o.z + a.R)) / r;
+    if (!ray_hits_ground(a.A, r, alt, mu)) {
+        p.L += p.thr * environment(a, d);
+        return false;
+    }
+    p.o = o + d * distance_to_bottom(a.A, r, alt, mu);
+    if (kCount) wc.vertices++;
+    return true;
+}
+// The second part: the sun's light through the shadow ray's transmittance tr, and the new direction
+// (hit: the vertex is a collision, else on the ground).  False when the path ends.
+__device__ __forceinline__ bool scatter(const PtArgs& a, Rng& rng, PathState& p, bool hit, float tr) {
+    if (hit) {
         float ph = pt_phase(a, dot(p.d, a.sun));
-        p.L += p.thr * (ratio_track<kMat, kBricks, kCount, kCells, kFlat>(a, rng, p.o, a.sun, wc) * ph * sun_illuminance(a, p.o));
+        p.L += p.thr * (tr * ph * sun_illuminance(a, p.o));
         float vop;
         p.d = hg_sample(a, rng, p.d, vop);
         p.thr = p.thr * vop;
+    } else {
+        F3 N = F3{p.o.x, p.o.y, p.o.z + a.R};
+        N = N * (1.0f / length3(N));
+        F3 bsdf = a.A.albedo * ((1.0f / kPiF) * dot(N, a.sun));
+        p.L += p.thr * (tr * sun_illuminance(a, p.o) * bsdf);
+        if (a.env == SKYHIP_ENV_GROUND_SINGLE_BOUNCE) return false;
+        p.d = lambert_sample(rng, N);
+        p.thr *= a.A.albedo;
     }
     return ++p.istep < a.max_bounces && fmaxf(p.thr.x, fmaxf(p.thr.y, p.thr.z)) > 0.0f;
+}
+
+// One iteration of Trace's bounce loop (:182-247).  False when the path ends in it (it leaves
+// the region, escapes, or reaches the bounce limit or zero throughput).  One shadow-ray call serves
+// collisions and ground hits, so that lanes with either track together.
+template <int kMat, bool kBricks, bool kCount, bool kCells, bool kFlat>
+__device__ __forceinline__ bool bounce(Rng& rng, PathState& p, PtCount& wc) {
+    const PtArgs& a = kernel_args();
+    float t0, t1;
+    region(a, p.o, p.d, t0, t1);
+    if (t0 >= t1) return false;
+    float t;
+    const bool hit = delta_track<kMat, kBricks, kCount, kCells, kFlat>(a, rng, p.o, p.d, t0, t1, t, wc);
+    if (!flight_end<kCount>(a, p, hit, t, wc)) return false;
+    const float tr = ratio_track<kMat, kBricks, kCount, kCells, kFlat>(a, rng, p.o, a.sun, wc);
+    return scatter(a, rng, p, hit, tr);
 }
 
 // Trace (:160-249)
@@ -605,15 +624,13 @@ __device__ __forceinline__ float4 add_sample(const PtArgs& a, float u, float v, 
     return acc;
 }
 
-// Five waves per SIMD (96 VGPRs; 3 VGPRs of the path state spill to scratch): more waves hide
-// more of the tracking's fetch latency.  Measured on the 1024^2 brick-majorant workload with the
-// nested loops: 3 waves (no cap) 14.2 ms per frame, 4 waves 12.0, 5 waves 11.2, 6 waves 11.4, 7
-// and 8 waves 12.0-12.2; with the flat loops and cell-corner lookups at 16^3: 4 waves 7.81-7.88,
-// 5 waves 7.27-7.28 (24 VGPRs spilled), 6 waves 9.45; with the accumulator read after the path:
-// 5 waves 7.26-7.27 (3 spilled), 6 waves 7.51-7.58 (21 spilled).  Every variant gives the same
-// image.
+// Six waves per SIMD (80 VGPRs; 2 VGPRs of the path state spill to scratch): more waves hide more of
+// the tracking's fetch latency.  Measured on the 1024^2 brick-majorant workload at 16^3 (ms per frame,
+// one box): 5 waves 6.17-6.19, 6 waves 5.89-5.97, 7 waves (15 VGPRs spilled) 5.96-6.11, 8 waves (33)
+// 6.71-6.73; 6.33-6.37 with 5 waves while collisions and ground hits called the shadow ray's tracking
+// separately (lanes with either waited for the other's).  Every variant gives the same image.
 template <int kMat, bool kBricks, bool kCount, bool kCells, bool kFlat>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void path_trace_kernel(PtArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void path_trace_kernel(PtArgs a) {
     const int lane = threadIdx.x;  // one wave64 per workgroup, an 8x8-pixel tile
     const int x = a.region[0] + blockIdx.x * 8 + (lane & 7);
     const int y = a.region[1] + blockIdx.y * 8 + (lane >> 3);

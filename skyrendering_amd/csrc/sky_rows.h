@@ -125,13 +125,6 @@ struct RowLds {
 };
 __host__ __device__ inline bool row_luts_fit(int tw, int mw) { return tw + mw <= kRowColumns; }
 
-// Orders the wave's own LDS writes before its reads (and the reads before the next writes).
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The next lane's value (lane 63 keeps its own).
 __device__ __forceinline__ float next_lane(float x) {
     const int v = __float_as_int(x);
