@@ -80,6 +80,7 @@ struct PtArgs {
     uint8_t* mask;
     unsigned long long* counters;  // samples, density lookups, majorant segments, path vertices, shadow rays
     unsigned* queue;               // path_trace_refill_kernel's tile counter (zero at launch)
+    int coop_log_x, coop_log_y;    // path_trace_coop_kernel's tile of paths
 };
 
 struct PtCount {
@@ -749,6 +750,193 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void p
     }
 }
 
+// ---------------------------------------------------------------------------
+// Single-majorant tracking by the whole wave.  A path's tentative collisions follow one another through
+// the random sequence, which is cheap, but their density lookups, which are not, depend only on their
+// positions; and most of a wave's lanes idle, their paths shorter.  So each tracking lane draws its next
+// K = 64 / (tracking lanes) positions, all 64 lanes look one up each, and the lane goes on from the
+// results in order: the same draws, lookups and products as delta_track and ratio_track (a free
+// flight's draws past its collision are dropped and its random state put back).  Bound by the lookups
+// and the draws about equally.  The 321 x 181 procedural frame: 6.3 ms, 17.1 with one lane per path
+// (13 % of the lanes busy).
+//
+// A wave has a tile of up to 64 paths, in its first lanes: a small image leaves SIMDs idle at 64 to a
+// wave, and a wave of fewer paths waits for a shorter longest path and gives each more of its lanes.
+// ---------------------------------------------------------------------------
+struct CoopLds {
+    float t[64], accept[64], sigma[64];  // slot K rank + j: the rank's position j, its acceptance draw, its density
+    uint32_t state[64];                  // the random state after that draw
+    float ray[6][64];                    // per rank: origin, direction
+    int count[64];
+};
+
+// The lookups of a round: lane e takes slot e.  K divides the slots among the `tracking` lanes.
+template <int kMat>
+__device__ __forceinline__ float coop_lookup(const PtArgs& a, const CoopLds& s, int tracking, int K) {
+    const int e = threadIdx.x;
+    const int rank = (e * (65535 / K + 1)) >> 16;  // e / K for e, K <= 64
+    if (rank >= tracking || e - rank * K >= s.count[rank]) return 0.0f;
+    const F3 o = {s.ray[0][rank], s.ray[1][rank], s.ray[2][rank]}, d = {s.ray[3][rank], s.ray[4][rank], s.ray[5][rank]};
+    return sigma_at<kMat>(a, o + d * s.t[e]);
+}
+__device__ __forceinline__ void coop_store_ray(CoopLds& s, int rank, F3 o, F3 d) {
+    s.ray[0][rank] = o.x, s.ray[1][rank] = o.y, s.ray[2][rank] = o.z;
+    s.ray[3][rank] = d.x, s.ray[4][rank] = d.y, s.ray[5][rank] = d.z;
+}
+
+// delta_track<kMat, false> for the lanes with `track`; every lane calls it.
+template <int kMat>
+__device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bool track, Rng& rng, F3 o, F3 d, float t0,
+                                                 float t1, float& t) {
+    bool on = track && a.sigma_t_max > 0.0f, hit = false;
+    t = t0;
+    int it = 0, ahead = 4;  // draws ahead, doubled while flights go on (those past a collision are wasted)
+    for (;;) {
+        const unsigned long long m = __ballot(on);
+        if (m == 0ull) return hit;
+        const int tracking = __popcll(m), K = min(64 / tracking, ahead), rank = __popcll(m & ((1ull << threadIdx.x) - 1ull));
+        ahead = min(2 * ahead, 64);
+        if (K == 1) {  // more than half the lanes: each looks up its own
+            if (on) {
+                t += exp_sample(rng.next()) * a.inv_sigma_t_max;
+                if (t > t1) {
+                    on = false;
+                } else {
+                    const float sg = sigma_at<kMat>(a, o + d * t);
+                    hit = rng.next() < sg * a.inv_sigma_t_max;
+                    on = !hit && ++it < kMaxTrackingSteps;
+                }
+            }
+            continue;
+        }
+        wave_lds_fence();
+        bool left = false;  // past t1 after the round's positions
+        int n = 0;
+        float tt = t;
+        if (on) {
+            coop_store_ray(s, rank, o, d);
+            for (; n < K; ++n) {
+                tt += exp_sample(rng.next()) * a.inv_sigma_t_max;
+                left = tt > t1;
+                if (left) break;
+                s.t[K * rank + n] = tt;
+                s.accept[K * rank + n] = rng.next();
+                s.state[K * rank + n] = rng.s;
+            }
+            s.count[rank] = n;
+        }
+        wave_lds_fence();
+        const float sg = coop_lookup<kMat>(a, s, tracking, K);
+        const int e = threadIdx.x, er = (e * (65535 / K + 1)) >> 16;
+        const bool taken = er < tracking && e - er * K < s.count[er] && s.accept[e] < sg * a.inv_sigma_t_max;
+        const unsigned long long hits = __ballot(taken);
+        if (on) {
+            const unsigned long long mine = (hits >> (K * rank)) & (K == 64 ? ~0ull : (1ull << K) - 1ull);
+            if (mine != 0ull) {
+                const int j = K * rank + __builtin_ctzll(mine);
+                t = s.t[j];
+                rng.s = s.state[j];
+                hit = true;
+                on = false;
+            } else {
+                t = tt;
+                it += n;
+                on = !left && it < kMaxTrackingSteps;
+            }
+        }
+    }
+}
+
+// ratio_track<kMat, false> for the lanes with `track`; every lane calls it.
+template <int kMat>
+__device__ __forceinline__ float coop_ratio_track(const PtArgs& a, CoopLds& s, bool track, Rng rng, F3 o, F3 d) {
+    float t = 0.0f, t1 = 0.0f, tr = 1.0f;
+    if (track) region(a, o, d, t, t1);
+    bool on = track && t < t1;
+    int it = 0;
+    for (;;) {
+        const unsigned long long m = __ballot(on);
+        if (m == 0ull) return clamp01(tr);
+        const int tracking = __popcll(m), K = 64 / tracking, rank = __popcll(m & ((1ull << threadIdx.x) - 1ull));
+        if (K == 1) {
+            if (on) {
+                t += exp_sample(rng.next()) * a.inv_sigma_t_max;
+                if (t > t1) {
+                    on = false;
+                } else {
+                    tr *= 1.0f - fmaxf(0.0f, sigma_at<kMat>(a, o + d * t) * a.inv_sigma_t_max);
+                    on = ++it < kMaxTrackingSteps;
+                }
+            }
+            continue;
+        }
+        wave_lds_fence();
+        bool left = false;
+        int n = 0;
+        if (on) {
+            coop_store_ray(s, rank, o, d);
+            for (; n < K; ++n) {
+                t += exp_sample(rng.next()) * a.inv_sigma_t_max;
+                left = t > t1;
+                if (left) break;
+                s.t[K * rank + n] = t;
+            }
+            s.count[rank] = n;
+        }
+        wave_lds_fence();
+        s.sigma[threadIdx.x] = coop_lookup<kMat>(a, s, tracking, K);
+        wave_lds_fence();
+        if (on) {
+            for (int j = 0; j < n; ++j) tr *= 1.0f - fmaxf(0.0f, s.sigma[K * rank + j] * a.inv_sigma_t_max);
+            it += n;
+            on = !left && it < kMaxTrackingSteps;
+        }
+    }
+}
+
+template <int kMat>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void path_trace_coop_kernel(PtArgs a0) {
+    __shared__ CoopLds lds;
+    const int lane = threadIdx.x, lx = a0.coop_log_x, ly = a0.coop_log_y;
+    const int x = a0.region[0] + (int(blockIdx.x) << lx) + (lane & ((1 << lx) - 1));
+    const int y = a0.region[1] + (int(blockIdx.y) << ly) + (lane >> lx);
+    const bool active = (lane >> (lx + ly)) == 0 && x < a0.region[2] && y < a0.region[3];
+    F3 view = {0.0f, 0.0f, 1.0f};
+    if (active) {
+        const float u = (float(x) + 0.5f) / float(a0.width), v = (float(y) + 0.5f) / float(a0.height);
+        float frag_dist;
+        view = unproject(a0.inv_mvp, u * 2.0f - 1.0f, v * 2.0f - 1.0f, 1.0f, a0.cam, &frag_dist);
+    }
+    Rng rng;
+    rng.pcg = a0.prng;
+    const uint32_t seed_xy = rng.hash(rng.hash(uint32_t(x)) + uint32_t(y));
+    PtCount wc;
+    for (int f = 0; f < a0.frames; ++f) {
+        rng.s = rng.hash(seed_xy + a0.first_frame + uint32_t(f));  // :260
+        PathState p;
+        bool alive = active && begin_path(kernel_args(), view, p);
+        while (__ballot(alive) != 0ull) {  // the bounces, as in bounce()
+            const PtArgs& a = kernel_args();
+            float t0 = 0.0f, t1 = 0.0f, t;
+            if (alive) {
+                region(a, p.o, p.d, t0, t1);
+                alive = t0 < t1;
+            }
+            const bool hit = coop_delta_track<kMat>(a, lds, alive, rng, p.o, p.d, t0, t1, t);
+            if (alive) alive = flight_end<false>(a, p, hit, t, wc);
+            const float tr = coop_ratio_track<kMat>(a, lds, alive, rng, p.o, a.sun);
+            if (alive) alive = scatter(a, rng, p, hit, tr);
+        }
+        if (active) {
+            const PtArgs& a = kernel_args();
+            const float u = (float(x) + 0.5f) / float(a.width), v = (float(y) + 0.5f) / float(a.height);
+            const long long pix = (long long)y * a.width + x;
+            a.accum[pix] = add_sample(a, u, v, view.z, p.L, p.has_scattered, p.scattered_t, a.accum[pix]);
+        }
+    }
+    if (active && a0.mask) a0.mask[(long long)y * a0.width + x] = 1;
+}
+
 __global__ void queue_reset_kernel(unsigned* q) {
     if (threadIdx.x == 0) q[0] = 0u;
 }
@@ -828,8 +1016,33 @@ constexpr int kRefillBlocksPerCu = 5;
 // body in every iteration.
 constexpr int kRefillMaxBrick = 4;
 
+// The tile of paths of a wave: the largest of 8 x 8, 8 x 4, .. 1 x 1 that makes three waves for every
+// SIMD.  ms per frame of the procedural cloud at 64 / 32 / 16 / 8 / 4 / 2 paths: 96 x 64 12.0 / 7.8 /
+// 5.4 / 4.2 / 3.4 / 2.9, 321 x 181 12.5 / 9.0 / 6.3 / 7.3, 640 x 360 14.3 / 15.3 / 15.4 / 18.9,
+// 1280 x 720 33.5 / 38.8 / 48.4 / 67.0.
+template <int kMat>
+static void launch_coop(hipStream_t st, PtArgs a, int cu_count) {
+    const long long w = a.region[2] - a.region[0], h = a.region[3] - a.region[1], waves = 3ll * 4 * cu_count;
+    a.coop_log_x = a.coop_log_y = 3;
+    while (a.coop_log_x + a.coop_log_y > 0 &&
+           (long long)div_up(w, 1 << a.coop_log_x) * div_up(h, 1 << a.coop_log_y) < waves)
+        --(a.coop_log_x == a.coop_log_y ? a.coop_log_y : a.coop_log_x);
+    hipLaunchKernelGGL(path_trace_coop_kernel<kMat>, dim3(div_up(w, 1 << a.coop_log_x), div_up(h, 1 << a.coop_log_y)),
+                       dim3(64), 0, st, a);
+}
+
 template <bool kBricks, bool kCount>
 static void launch_path_trace(hipStream_t st, const PtArgs& a, int cu_count) {
+    if constexpr (!kBricks && !kCount) {
+        switch (a.mat.kind) {
+            case SKYHIP_MATERIAL_DEFAULT0: return launch_coop<SKYHIP_MATERIAL_DEFAULT0>(st, a, cu_count);
+            case SKYHIP_MATERIAL_DEFAULT1: return launch_coop<SKYHIP_MATERIAL_DEFAULT1>(st, a, cu_count);
+            case SKYHIP_MATERIAL_DEFAULT1_WORLEY: return launch_coop<SKYHIP_MATERIAL_DEFAULT1_WORLEY>(st, a, cu_count);
+            case SKYHIP_MATERIAL_MINIMAL: return launch_coop<SKYHIP_MATERIAL_MINIMAL>(st, a, cu_count);
+            case SKYHIP_MATERIAL_VOXEL: return launch_coop<SKYHIP_MATERIAL_VOXEL>(st, a, cu_count);
+            default: return launch_coop<SKYHIP_MATERIAL_VOXEL_F16>(st, a, cu_count);
+        }
+    }
     // One wave64 per workgroup (8x8 pixels): a finished wave's slot takes the next tile by itself,
     // where a 256-lane workgroup's four waves are placed on one CU together.  Measured on the
     // 1024^2 workload: 6.71-6.73 against 7.26-7.30 ms per frame (16x16-pixel workgroups).
