@@ -267,19 +267,6 @@ __device__ inline void scattered_luminance_part(const AtmDev& A, const float4* _
     for (int k = 0; k < count; ++k, i += 1.0f) scatter_step<false>(A, T, tw, th, MS, mw, mh, s, c, i, L, Tr, Lf);
 }
 
-// The same for the multiple-scattering variant (isotropic phase, no MS term, and the
-// multiple-scattering transfer Lf beside L): parts combine as L = L_a + Tr_a L_b,
-// Lf = Lf_a + Tr_a Lf_b, Tr = Tr_a Tr_b.
-__device__ inline void scattered_luminance_part_ms(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
-                                                   const RayStart& s, const ScatterRay& c, float i0, int count, F3& L,
-                                                   F3& Tr, F3& Lf) {
-    L = f3(0.0f);
-    Tr = f3(1.0f);
-    Lf = f3(0.0f);
-    float i = i0;
-    for (int k = 0; k < count; ++k, i += 1.0f) scatter_step<true>(A, T, tw, th, nullptr, 0, 0, s, c, i, L, Tr, Lf);
-}
-
 // scattered_luminance<false> spread over kParts consecutive lanes of a wave (kParts a power of
 // two dividing 64; part = lane index within the group).  Part p integrates steps
 // [p c, (p + 1) c), c = ceil(n / kParts), of the shader's float counter (n its trip count,

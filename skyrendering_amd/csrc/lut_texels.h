@@ -272,9 +272,7 @@ __device__ inline SkyViewRay sky_view_ray(const AtmDev& A, const RenderDev& R, c
     return ray;
 }
 
-// One sky-view texel (:74-186): luminance and transmittance (kCells: T and MS are cell-corner
-// copies).
-template <bool kCells = false>
+// One sky-view texel (:74-186): luminance and transmittance.
 __device__ inline void sky_view_texel(const AtmDev& A, const RenderDev& R, const float4* __restrict__ T, int tw,
                                       int th, const float4* __restrict__ MS, int mw, int mh,
                                       const uint16_t* __restrict__ blue_noise, int bn_size, int ix, int iy, int w,
@@ -284,8 +282,7 @@ __device__ inline void sky_view_texel(const AtmDev& A, const RenderDev& R, const
     Tr = f3(1.0f);
     F3 Lf;
     if (ray.dist > 0.0f)
-        scattered_luminance<false, kCells>(A, T, tw, th, MS, mw, mh, ray.s, ray.dist, R.sv_steps, ray.start_i, L, Tr,
-                                           Lf);
+        scattered_luminance<false>(A, T, tw, th, MS, mw, mh, ray.s, ray.dist, R.sv_steps, ray.start_i, L, Tr, Lf);
 }
 
 // ProjectiveMul(inv_view_projection, (x, y, z)) - camera, normalised; the

@@ -4,8 +4,8 @@
 // environment term from the sky-view LUT and aerial perspective at the first
 // scattering event.
 //
-// One path per lane; a wave64, one workgroup, covers an 8x8 pixel tile and
-// loops over the requested frames, adding each frame's
+// One path per lane; a wave64, one workgroup, covers a tile of pixels (8x8, with one majorant
+// also fewer) and loops over the requested frames, adding each frame's
 // sample to the pixel's accumulator in frame order as the reference's
 // per-frame imageLoad/imageStore does.  Tracking runs either with the
 // reference's single majorant kSigmaTMax, drawing the reference's random
@@ -14,6 +14,8 @@
 // walked with a 3D DDA in texel space: empty bricks cost one majorant fetch,
 // and inside occupied bricks the tentative-collision rate follows the local
 // maximum instead of the global one.
+#include <type_traits>
+
 #include "cloud_device.h"
 #include "sky_env.h"
 
@@ -1031,65 +1033,49 @@ static void launch_coop(hipStream_t st, PtArgs a, int cu_count) {
                        dim3(64), 0, st, a);
 }
 
-template <bool kBricks, bool kCount>
-static void launch_path_trace(hipStream_t st, const PtArgs& a, int cu_count) {
-    if constexpr (!kBricks && !kCount) {
-        switch (a.mat.kind) {
-            case SKYHIP_MATERIAL_DEFAULT0: return launch_coop<SKYHIP_MATERIAL_DEFAULT0>(st, a, cu_count);
-            case SKYHIP_MATERIAL_DEFAULT1: return launch_coop<SKYHIP_MATERIAL_DEFAULT1>(st, a, cu_count);
-            case SKYHIP_MATERIAL_DEFAULT1_WORLEY: return launch_coop<SKYHIP_MATERIAL_DEFAULT1_WORLEY>(st, a, cu_count);
-            case SKYHIP_MATERIAL_MINIMAL: return launch_coop<SKYHIP_MATERIAL_MINIMAL>(st, a, cu_count);
-            case SKYHIP_MATERIAL_VOXEL: return launch_coop<SKYHIP_MATERIAL_VOXEL>(st, a, cu_count);
-            default: return launch_coop<SKYHIP_MATERIAL_VOXEL_F16>(st, a, cu_count);
+// Without a brick grid (one majorant): every material.
+static void launch_single_majorant(hipStream_t st, const PtArgs& a, int cu_count, bool count) {
+    const dim3 grid(div_up(a.region[2] - a.region[0], 8), div_up(a.region[3] - a.region[1], 8));
+    auto with = [&](auto kind) {
+        constexpr int kMat = decltype(kind)::value;
+        if (count)
+            hipLaunchKernelGGL((path_trace_kernel<kMat, false, true, false, false>), grid, dim3(64), 0, st, a);
+        else
+            launch_coop<kMat>(st, a, cu_count);
+    };
+    switch (a.mat.kind) {
+        case SKYHIP_MATERIAL_DEFAULT0: return with(std::integral_constant<int, SKYHIP_MATERIAL_DEFAULT0>());
+        case SKYHIP_MATERIAL_DEFAULT1: return with(std::integral_constant<int, SKYHIP_MATERIAL_DEFAULT1>());
+        case SKYHIP_MATERIAL_DEFAULT1_WORLEY: return with(std::integral_constant<int, SKYHIP_MATERIAL_DEFAULT1_WORLEY>());
+        case SKYHIP_MATERIAL_MINIMAL: return with(std::integral_constant<int, SKYHIP_MATERIAL_MINIMAL>());
+        case SKYHIP_MATERIAL_VOXEL: return with(std::integral_constant<int, SKYHIP_MATERIAL_VOXEL>());
+        default: return with(std::integral_constant<int, SKYHIP_MATERIAL_VOXEL_F16>());
+    }
+}
+
+// Over an FP16 volume's brick grid.
+template <bool kCount>
+static void launch_bricks(hipStream_t st, const PtArgs& a, int cu_count) {
+    if (!kCount && a.cells && a.brick <= kRefillMaxBrick) {
+        // One persistent launch per frame, its tile counter cleared by a kernel before it.
+        for (int f = 0; f < a.frames; ++f) {
+            PtArgs af = a;
+            af.first_frame = a.first_frame + uint32_t(f);
+            af.frames = 1;
+            hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, st, a.queue);
+            hipLaunchKernelGGL((path_trace_refill_kernel<SKYHIP_MATERIAL_VOXEL_F16, true, true, false>),
+                               dim3(cu_count * kRefillBlocksPerCu), dim3(256), 0, st, af);
         }
+        return;
     }
     // One wave64 per workgroup (8x8 pixels): a finished wave's slot takes the next tile by itself,
     // where a 256-lane workgroup's four waves are placed on one CU together.  Measured on the
     // 1024^2 workload: 6.71-6.73 against 7.26-7.30 ms per frame (16x16-pixel workgroups).
-    dim3 grid(div_up(a.region[2] - a.region[0], 8), div_up(a.region[3] - a.region[1], 8));
-    switch (a.mat.kind) {
-        case SKYHIP_MATERIAL_DEFAULT0:
-            hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_DEFAULT0, false, kCount, false, false>), grid, dim3(64), 0, st,
-                               a);
-            break;
-        case SKYHIP_MATERIAL_DEFAULT1:
-            hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_DEFAULT1, false, kCount, false, false>), grid, dim3(64), 0, st,
-                               a);
-            break;
-        case SKYHIP_MATERIAL_DEFAULT1_WORLEY:
-            hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_DEFAULT1_WORLEY, false, kCount, false, false>), grid, dim3(64), 0,
-                               st, a);
-            break;
-        case SKYHIP_MATERIAL_MINIMAL:
-            hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_MINIMAL, false, kCount, false, false>), grid, dim3(64), 0, st,
-                               a);
-            break;
-        case SKYHIP_MATERIAL_VOXEL:
-            hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_VOXEL, false, kCount, false, false>), grid, dim3(64), 0, st, a);
-            break;
-        default:
-            if constexpr (kBricks && !kCount) {
-                if (a.cells && a.brick <= kRefillMaxBrick) {
-                    // One persistent launch per frame, its tile counter cleared by a kernel before it.
-                    for (int f = 0; f < a.frames; ++f) {
-                        PtArgs af = a;
-                        af.first_frame = a.first_frame + uint32_t(f);
-                        af.frames = 1;
-                        hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, st, a.queue);
-                        hipLaunchKernelGGL((path_trace_refill_kernel<SKYHIP_MATERIAL_VOXEL_F16, true, true, false>),
-                                           dim3(cu_count * kRefillBlocksPerCu), dim3(256), 0, st, af);
-                    }
-                    break;
-                }
-            }
-            if (kBricks && a.cells)
-                hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_VOXEL_F16, kBricks, kCount, kBricks, kBricks>),
-                                   grid, dim3(64), 0, st, a);
-            else
-                hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_VOXEL_F16, kBricks, kCount, false, kBricks>),
-                                   grid, dim3(64), 0, st, a);
-            break;
-    }
+    const dim3 grid(div_up(a.region[2] - a.region[0], 8), div_up(a.region[3] - a.region[1], 8));
+    if (a.cells)
+        hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_VOXEL_F16, true, kCount, true, true>), grid, dim3(64), 0, st, a);
+    else
+        hipLaunchKernelGGL((path_trace_kernel<SKYHIP_MATERIAL_VOXEL_F16, true, kCount, false, true>), grid, dim3(64), 0, st, a);
 }
 
 }  // namespace skyhip
@@ -1291,17 +1277,12 @@ extern "C" int skyhip_cloud_path_trace(SkyhipContext* ctx, const SkyhipAtmospher
         a.inv_majorants = ctx->pt_inv_majorants;
     }
     const int cus = std::max(ctx->cu_count, 1);
-    if (bricks) {
-        if (work_counters)
-            launch_path_trace<true, true>(ctx->stream, a, cus);
-        else
-            launch_path_trace<true, false>(ctx->stream, a, cus);
-    } else {
-        if (work_counters)
-            launch_path_trace<false, true>(ctx->stream, a, cus);
-        else
-            launch_path_trace<false, false>(ctx->stream, a, cus);
-    }
+    if (!bricks)
+        launch_single_majorant(ctx->stream, a, cus, work_counters != nullptr);
+    else if (work_counters)
+        launch_bricks<true>(ctx->stream, a, cus);
+    else
+        launch_bricks<false>(ctx->stream, a, cus);
     SKYHIP_LAUNCH_CHECK("path_trace_kernel");
     return SKYHIP_OK;
 }
