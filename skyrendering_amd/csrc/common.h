@@ -88,7 +88,8 @@ __host__ __device__ inline F3 operator*(F3 a, float s) { return {a.x * s, a.y * 
 __host__ __device__ inline F3 operator*(float s, F3 a) { return {a.x * s, a.y * s, a.z * s}; }
 __host__ __device__ inline F3& operator+=(F3& a, F3 b) { a = a + b; return a; }
 __host__ __device__ inline F3& operator*=(F3& a, F3 b) { a = a * b; return a; }
-__host__ __device__ inline float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__host__ __device__ __forceinline__ F3 fma3(F3 a, F3 b, F3 c) { return {fmaf(a.x, b.x, c.x), fmaf(a.y, b.y, c.y), fmaf(a.z, b.z, c.z)}; }
+__device__ inline float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __host__ __device__ inline F3 cross(F3 a, F3 b) {
     return {a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y};
 }

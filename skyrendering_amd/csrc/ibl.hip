@@ -2,15 +2,13 @@
 // precomputation:
 //  - env_luminance_kernel: one thread per cube texel, the sky-view LUT pair looked up along
 //    the texel's direction plus the lit ground (AtmosphereRenderer.glsl:248-275), stored as
-//    RGBA16F (a = 0);
-//  - cube_mip_kernel, cube_mip_tail_kernel: the cube's mip chain, a 2x2 box per level
+//    RGBA16F (a = 0), and its tile's part of the mip chain, a 2x2 box per level
 //    (glGenerateTextureMipmap, AtmosphereRenderer.cpp:242; the filter is the implementation's,
-//    here a box), the levels of at most 64^2 texels a face in one launch;
+//    here a box); cube_mip_tail_kernel: the levels below a tile's, in one launch;
 //  - prefilter_kernel: the 9 spherical-harmonic radiance coefficients (EnvRadianceSH.comp), one
 //    workgroup per coefficient over 1024 stratified directions summed by the shader's halving
 //    tree, and in the same launch the GGX-prefiltered radiance cube, one level per roughness
-//    (PrefilterRadiance.comp, IBL.cpp:25-45), a texel's samples spread over a group of lanes.
-// Each pass is tiny (at most 98,304 texels); the sequence is bound by launch latency.
+//    (PrefilterRadiance.comp, IBL.cpp:25-45).
 #include "sky_env.h"
 
 namespace skyhip {
@@ -41,35 +39,7 @@ int log2i(int w) {
 
 }  // namespace
 
-__global__ __launch_bounds__(256) void env_luminance_kernel(AtmDev A, EnvFrame e, const float4* __restrict__ T,
-                                                            int tw, int th, const float4* __restrict__ sv_l,
-                                                            const float4* __restrict__ sv_t, int sw, int sh,
-                                                            ushort4* __restrict__ out, int w) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= 6 * w * w) return;
-    const int face = i / (w * w), y = (i / w) % w, x = i % w;
-    const F3 d = cube_texel_dir(face, x, y, w);
-    out[i] = to_rgba16f(env_luminance(A, e, T, tw, th, sv_l, sv_t, sw, sh, d), 0.0f);
-}
-
-// Level `level` of the cube from level - 1: the mean of the 2x2 parent texels per channel.
-__global__ __launch_bounds__(256) void cube_mip_kernel(ushort4* cube, int w, int level) {
-    const int wl = max(w >> level, 1), wp = max(w >> (level - 1), 1);
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= 6 * wl * wl) return;
-    const int face = i / (wl * wl), y = (i / wl) % wl, x = i % wl;
-    const ushort4* src = cube + cube_level_offset(w, level - 1) + (long long)face * wp * wp;
-    const int x0 = min(2 * x, wp - 1), x1 = min(2 * x + 1, wp - 1), y0 = min(2 * y, wp - 1), y1 = min(2 * y + 1, wp - 1);
-    const ushort4 a = src[y0 * wp + x0], b = src[y0 * wp + x1], c = src[y1 * wp + x0], d = src[y1 * wp + x1];
-    ushort4 o;
-    o.x = __half_as_ushort(__float2half_rn(((h2f(a.x) + h2f(b.x)) + (h2f(c.x) + h2f(d.x))) * 0.25f));
-    o.y = __half_as_ushort(__float2half_rn(((h2f(a.y) + h2f(b.y)) + (h2f(c.y) + h2f(d.y))) * 0.25f));
-    o.z = __half_as_ushort(__float2half_rn(((h2f(a.z) + h2f(b.z)) + (h2f(c.z) + h2f(d.z))) * 0.25f));
-    o.w = __half_as_ushort(__float2half_rn(((h2f(a.w) + h2f(b.w)) + (h2f(c.w) + h2f(d.w))) * 0.25f));
-    cube[cube_level_offset(w, level) + (long long)face * wl * wl + y * wl + x] = o;
-}
-
-// The mean of a 2x2 parent block per channel (cube_mip_kernel's arithmetic).
+// The mean of a 2x2 parent block per channel.
 __device__ inline ushort4 box4(ushort4 a, ushort4 b, ushort4 c, ushort4 d) {
     ushort4 o;
     o.x = __half_as_ushort(__float2half_rn(((h2f(a.x) + h2f(b.x)) + (h2f(c.x) + h2f(d.x))) * 0.25f));
@@ -79,10 +49,42 @@ __device__ inline ushort4 box4(ushort4 a, ushort4 b, ushort4 c, ushort4 d) {
     return o;
 }
 
-// Levels first_level .. levels - 1 of one face (blockIdx.x) in one workgroup, for the levels of at
-// most kMipTailWidth^2 texels a face: the first from the parent level in global memory, each
-// later one from the previous level kept in LDS, every level also stored to the cube.  The same
-// arithmetic as cube_mip_kernel level by level, without a launch per level.
+// A workgroup computes a tile of a face (16 x 16 texels, or the face if that is smaller) and, the
+// tile's texels being in LDS, its part of the next levels down to one texel.  A launch of six
+// workgroups, one a face, reading level 0 back for the whole chain took 10.3 us at 128^2; the levels left
+// to it take 5.1 and the tiles 0.4 more.
+constexpr int kEnvTile = 16, kEnvTileLog = 4;
+__global__ __launch_bounds__(256) void env_luminance_kernel(AtmDev A, EnvFrame e, const float4* __restrict__ T,
+                                                            int tw, int th, const float4* __restrict__ sv_l,
+                                                            const float4* __restrict__ sv_t, int sw, int sh,
+                                                            ushort4* __restrict__ out, int w, int tile_log) {
+    __shared__ ushort4 s_a[kEnvTile * kEnvTile], s_b[kEnvTile * kEnvTile / 4];
+    const int t = threadIdx.x, face = blockIdx.z;
+    const int x0 = int(blockIdx.x) << tile_log, y0 = int(blockIdx.y) << tile_log;
+    if (t < 1 << (2 * tile_log)) {
+        const int x = x0 + (t & ((1 << tile_log) - 1)), y = y0 + (t >> tile_log);
+        const ushort4 v =
+            to_rgba16f(env_luminance(A, e, T, tw, th, sv_l, sv_t, sw, sh, cube_texel_dir(face, x, y, w)), 0.0f);
+        out[(long long)face * w * w + (long long)y * w + x] = v;
+        s_a[t] = v;
+    }
+    for (int l = 1; l <= tile_log; ++l) {  // a face of one texel is a chain of one level
+        __syncthreads();
+        const int lw = tile_log - l, wl = w >> l;
+        const ushort4* src = (l & 1) ? s_a : s_b;
+        ushort4* dst = (l & 1) ? s_b : s_a;
+        if (t < 1 << (2 * lw)) {
+            const int x = t & ((1 << lw) - 1), y = t >> lw, s = (2 * y << (lw + 1)) + 2 * x;
+            const ushort4 v = box4(src[s], src[s + 1], src[s + (2 << lw)], src[s + (2 << lw) + 1]);
+            out[cube_level_offset(w, l) + (long long)face * wl * wl + (long long)((y0 >> l) + y) * wl + (x0 >> l) + x] = v;
+            dst[t] = v;
+        }
+    }
+}
+
+// Levels first_level .. levels - 1 of one face (blockIdx.x) in one workgroup: the first from the
+// parent level in global memory, each later one from the previous level kept in LDS, every level
+// also stored to the cube.  Levels after the first are at most kMipTailWidth / 2 wide (the launch's).
 constexpr int kMipTailWidth = 64;
 __global__ __launch_bounds__(1024) void cube_mip_tail_kernel(ushort4* cube, int w, int first_level, int levels) {
     __shared__ ushort4 s_a[kMipTailWidth * kMipTailWidth];
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(1024) void cube_mip_tail_kernel(ushort4* cube, int 
                       y1 = min(2 * y + 1, wp - 1);
             const ushort4* src = from_global ? gsrc : lsrc;
             const ushort4 o = box4(src[y0 * wp + x0], src[y0 * wp + x1], src[y1 * wp + x0], src[y1 * wp + x1]);
-            ldst[t] = o;
+            if (wl <= kMipTailWidth) ldst[t] = o;
             gdst[t] = o;
         }
         __syncthreads();
@@ -110,10 +112,8 @@ __global__ __launch_bounds__(1024) void cube_mip_tail_kernel(ushort4* cube, int 
 
 // EnvRadianceSH.comp: coefficient `index` from 1024 directions on a 32 x 32 stratified grid
 // (uniform in cos theta and phi, y up), each sample weighted 4 pi / 1024, summed by the shader's
-// halving tree over the 1024 values (at half = 512, 256, ..., 1: s[i] += s[i + half]).  A
-// 256-thread workgroup holds samples t, t + 256, t + 512 and t + 768 in thread t and forms the
-// tree's first two levels in registers, (s_t + s_(t+512)) + (s_(t+256) + s_(t+768)), the rest
-// over LDS: the same additions in the same order.
+// halving tree over the 1024 values (at half = 512, 256, ..., 1: s[i] += s[i + half]), the first
+// level in registers: a 512-thread workgroup holds samples t and t + 512 in thread t.
 __device__ inline F3 sh9_sample(const ushort4* __restrict__ cube, int w, int levels, int index, int li) {
     const float unit_theta = (0.5f + float(li >> 5)) / 32.0f;
     const float unit_phi = (0.5f + float(li & 31)) / 32.0f;
@@ -140,11 +140,9 @@ __device__ inline F3 sh9_sample(const ushort4* __restrict__ cube, int w, int lev
 __device__ inline void sh9_block(const ushort4* __restrict__ cube, int w, int levels, int index,
                                  float4* __restrict__ out, F3* s) {
     const int t = threadIdx.x;
-    const F3 lo = sh9_sample(cube, w, levels, index, t) + sh9_sample(cube, w, levels, index, t + 512);
-    const F3 hi = sh9_sample(cube, w, levels, index, t + 256) + sh9_sample(cube, w, levels, index, t + 768);
-    s[t] = lo + hi;
+    s[t] = sh9_sample(cube, w, levels, index, t) + sh9_sample(cube, w, levels, index, t + 512);
     __syncthreads();
-    for (int half = 128; half >= 1; half >>= 1) {
+    for (int half = 256; half >= 1; half >>= 1) {
         if (t < half) s[t] = s[t] + s[t + half];
         __syncthreads();
     }
@@ -172,88 +170,168 @@ __device__ inline void onb_frame(F3 N, F3& t0, F3& t1) {
 
 constexpr int kMaxPrefilterLevels = 13;  // roughness_count <= log2(4096) + 1
 
-// PrefilterRadiance.comp for level `level` (width wl) of the output cube at roughness r.  Each
-// texel's samples are spread over a group of `group` = n lanes (the level's sample count, at most
-// 64; 1 at roughness 0), 256 / n texels to a workgroup: lane k evaluates sample k into LDS, and
-// the group's first lane adds the terms in sample order, so the sums are the
-// one-thread-per-texel loop's.
-// The rough levels have few texels (384 at 8^2 x 6) and up to 64 samples each, which one thread
-// per texel left as a chain of dependent cube fetches.
-// All levels run in one launch, after the kSh9Blocks workgroups that compute the SH9
-// coefficients (sh9_block; both read the environment cube only): workgroups kSh9Blocks +
+// PrefilterRadiance.comp, all levels in one launch, after the kSh9Blocks workgroups that compute the
+// SH9 coefficients (sh9_block; both read the environment cube only): workgroups kSh9Blocks +
 // [block_start[l], block_start[l + 1]) build level l.
+//
+// The view direction is the normal, so a level's samples are the same in every texel's tangent frame:
+// direction, cosine, density and mip level (H = (sin cos phi, sin sin phi, cos), L = 2 cos H - N).  A
+// workgroup's first wave makes the table of those above the horizon; then a lane is a texel, the
+// workgroup's kPrefilterWaves waves share its 64 texels' samples (wave v takes entries v,
+// v + kPrefilterWaves, ..), and an entry's mip levels are wave-uniform.  Bound by the cube lookups'
+// instructions.  128^2, 5 levels, with SH9: 11.4 us; 39.6 with a lane per sample of a texel, which
+// evaluated the sample again in each texel.
 struct PrefilterLevels {
     int count;
     int block_start[kMaxPrefilterLevels + 1];
     float roughness[kMaxPrefilterLevels];
-    int group[kMaxPrefilterLevels];  // lanes per texel (the sample count)
+    int samples[kMaxPrefilterLevels];  // at most 64; 1 at roughness 0
 };
 
-__global__ __launch_bounds__(256) void prefilter_kernel(const ushort4* __restrict__ env, int ew, int elevels,
-                                                        float4* __restrict__ sh9_out, ushort4* __restrict__ out,
-                                                        int pw, PrefilterLevels lv) {
-    __shared__ float4 s_term[256];
-    __shared__ F3 s_sh[256];
+constexpr int kPrefilterWaves = 8;
+struct PrefilterSample {
+    float x, y, z;  // direction in the texel's frame; z is also the weight
+    float blend;    // of level + 1
+    int level;
+};
+
+// Sample k of n (lane k < n) and whether it lies above the horizon.
+__device__ inline bool prefilter_sample(uint32_t k, uint32_t n, float a2, float inv_sa_texel, int levels,
+                                        PrefilterSample& s) {
+    // Hammersley (shaders/Base/Noise.glsl:113-117) with no random offset
+    const float q = float(k) / float(n);
+    const float e1 = q - floorf(q);
+    const float e2 = float(reverse_bits32(k)) * 2.3283064365386963e-10f;
+    // ImportanceSampleGGX (shaders/Base/BRDF.glsl:48-67)
+    const float phi = 2.0f * kPiF * e1;
+    const float cos_t = sqrtf((1.0f - e2) / (1.0f + (a2 - 1.0f) * e2));
+    const float sin_t = sqrtf(1.0f - cos_t * cos_t);
+    s.x = 2.0f * cos_t * (sin_t * cosf(phi));
+    s.y = 2.0f * cos_t * (sin_t * sinf(phi));
+    s.z = fminf(2.0f * cos_t * cos_t - 1.0f, 1.0f);
+    const float dg = (cos_t * a2 - cos_t) * cos_t + 1.0f;  // D_GGX (BRDF.glsl:36-40), NoH = HoV = cos_t
+    const float D = a2 / (kPiF * dg * dg);
+    const float pdf = fmaxf(D * cos_t / (4.0f * cos_t), 0.0001f);
+    const float sa_sample = 1.0f / fmaxf(float(n) * pdf, 0.00001f);
+    const float mip = 0.5f * log2f(sa_sample * inv_sa_texel) + 2.5f;
+    const float lod = mip > 0.0f ? fminf(mip, float(levels - 1)) : 0.0f;
+    s.level = int(lod);
+    s.blend = lod - float(s.level);
+    return s.z > 0.0f;
+}
+
+// Adds weight x (cube_level_bilinear's value) of a level of width 1 << log_w.
+__device__ __forceinline__ void prefilter_add(const ushort4* __restrict__ level, int log_w, int face, float s, float t,
+                                              float weight, F3& sum) {
+    const int wl = 1 << log_w;
+    const float top = float(wl - 1);
+    const float fx = __builtin_amdgcn_fmed3f(fmaf(s, float(wl), -0.5f), 0.0f, top);
+    const float fy = __builtin_amdgcn_fmed3f(fmaf(t, float(wl), -0.5f), 0.0f, top);
+    const int x0 = int(fx), y0 = int(fy);
+    const int dx = x0 < wl - 1 ? 1 : 0, dy = y0 < wl - 1 ? wl : 0;
+    const unsigned at = (unsigned(face) << (2 * log_w)) + (unsigned(y0) << log_w) + unsigned(x0);
+    const ushort4 a = level[at], b = level[at + dx], c = level[at + dy], d = level[at + dy + dx];
+    const float ax = __builtin_amdgcn_fractf(fx), ay = __builtin_amdgcn_fractf(fy);
+    const float wc = weight * ay, wa = weight * (1.0f - ay);
+    const float w0 = wa * (1.0f - ax), w1 = wa * ax, w2 = wc * (1.0f - ax), w3 = wc * ax;
+    sum = fma3(f3(w0), rgba16f_rgb(a), sum);
+    sum = fma3(f3(w1), rgba16f_rgb(b), sum);
+    sum = fma3(f3(w2), rgba16f_rgb(c), sum);
+    sum = fma3(f3(w3), rgba16f_rgb(d), sum);
+}
+
+__global__ __launch_bounds__(64 * kPrefilterWaves) void prefilter_kernel(const ushort4* __restrict__ env, int log_ew,
+                                                                         float4* __restrict__ sh9_out,
+                                                                         ushort4* __restrict__ out, int pw,
+                                                                         PrefilterLevels lv) {
+    constexpr int kThreads = 64 * kPrefilterWaves;
+    __shared__ F3 s_sum[kThreads];
+    __shared__ PrefilterSample s_sample[64];
+    __shared__ float s_weight;
+    __shared__ int s_count;
+    const int ew = 1 << log_ew, elevels = log_ew + 1;
     if (int(blockIdx.x) < kSh9Blocks) {
-        sh9_block(env, ew, elevels, int(blockIdx.x), sh9_out, s_sh);
+        static_assert(kThreads == 512, "sh9_block's threads");
+        sh9_block(env, ew, elevels, int(blockIdx.x), sh9_out, s_sum);
         return;
     }
     const int block = int(blockIdx.x) - kSh9Blocks;
     int level = 0;
     while (level + 1 < lv.count && block >= lv.block_start[level + 1]) ++level;
     const float roughness = lv.roughness[level];
-    const int group = lv.group[level];
     const int wl = max(pw >> level, 1);
-    const int per_block = 256 / group;
-    const int j = int(threadIdx.x) / group, k = int(threadIdx.x) - j * group;
-    const int i = (block - lv.block_start[level]) * per_block + j;
-    const bool texel = j < per_block && i < 6 * wl * wl;
-    const int face = i / (wl * wl), y = (i / wl) % wl, x = i % wl;
-    const F3 R = cube_texel_dir(face, x, y, wl);
-    const F3 N = R, V = R;
-    const float a = roughness * roughness, a2 = a * a;
-    // uint(mix(1, 64, pow(roughness, 0.3))), evaluated on the host with the group sizes
-    const uint32_t n = uint32_t(group);
-    const float inv_sa_texel = (6.0f * float(wl) * float(wl)) / (4.0f * kPiF);
-    float4 term = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (sample * NoL, NoL), NoL = 0: no contribution
-    if (texel && uint32_t(k) < n) {
-        F3 t0, t1;
-        onb_frame(N, t0, t1);
-        // Hammersley (shaders/Base/Noise.glsl:113-117) with no random offset
-        const float q = float(uint32_t(k)) / float(n);
-        const float e1 = q - floorf(q);
-        const float e2 = float(reverse_bits32(uint32_t(k))) * 2.3283064365386963e-10f;
-        // ImportanceSampleGGX (shaders/Base/BRDF.glsl:48-67)
-        const float phi = 2.0f * kPiF * e1;
-        const float cos_t = sqrtf((1.0f - e2) / (1.0f + (a2 - 1.0f) * e2));
-        const float sin_t = sqrtf(1.0f - cos_t * cos_t);
-        const F3 H = t0 * (sin_t * cosf(phi)) + t1 * (sin_t * sinf(phi)) + N * cos_t;
-        const F3 L = H * (2.0f * dot(V, H)) - V;
+    const int tile = block - lv.block_start[level];
+    ushort4* dst = out + cube_level_offset(pw, level);
+    if (roughness == 0.0f) {  // one sample, along the normal, at level 0
+        const long long i = (long long)tile * kThreads + threadIdx.x;
+        if (i >= 6ll * wl * wl) return;
+        const int face = int(i / (wl * wl)), y = int(i / wl) % wl, x = int(i % wl);
+        const F3 N = cube_texel_dir(face, x, y, wl);
+        const F3 L = N * (2.0f * dot(N, N)) - N;
         const float NoL = clamp01(dot(N, L));
-        if (NoL > 0.0f) {
-            const float NoH = clamp01(dot(N, H)), HoV = clamp01(dot(H, V));
-            const float dg = (NoH * a2 - NoH) * NoH + 1.0f;  // D_GGX (BRDF.glsl:36-40)
-            const float D = a2 / (kPiF * dg * dg);
-            const float pdf = fmaxf(D * NoH / (4.0f * HoV), 0.0001f);
-            const float sa_sample = 1.0f / fmaxf(float(n) * pdf, 0.00001f);
-            const float mip = roughness == 0.0f ? 0.0f : 0.5f * log2f(sa_sample * inv_sa_texel) + 2.5f;
-            const F3 c = cube_sample_lod(env, ew, elevels, L, mip) * NoL;
-            term = make_float4(c.x, c.y, c.z, NoL);
-        }
+        const F3 c = cube_sample_lod(env, ew, elevels, L, 0.0f) * NoL;
+        dst[i] = to_rgba16f(c * (1.0f / NoL), 0.0f);
+        return;
     }
-    s_term[threadIdx.x] = term;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // The workgroup's texels: 8 x 8 of a face, or 64 in a row where a face is smaller.
+    const long long p = (long long)tile * 64 + lane;
+    const bool texel = p < 6ll * wl * wl;
+    const int face = int(p / (wl * wl)), q = int(p % (wl * wl));
+    const int per_row = wl >> 3;
+    const int x = wl >= 8 ? ((q >> 6) % per_row) * 8 + (q & 7) : q % wl;
+    const int y = wl >= 8 ? ((q >> 6) / per_row) * 8 + ((q >> 3) & 7) : q / wl;
+    const F3 N = cube_texel_dir(min(face, 5), x, y, wl);
+    F3 t0, t1;
+    onb_frame(N, t0, t1);
+    if (wave == 0) {
+        const float a = roughness * roughness;
+        const uint32_t n = uint32_t(lv.samples[level]);
+        PrefilterSample s;
+        const bool up =
+            uint32_t(lane) < n &&
+            prefilter_sample(uint32_t(lane), n, a * a, (6.0f * float(wl) * float(wl)) / (4.0f * kPiF), elevels, s);
+        const uint64_t mask = __ballot(up);
+        if (up) s_sample[__popcll(mask & ((1ull << lane) - 1))] = s;
+        float weight = up ? s.z : 0.0f;
+        for (int m = 32; m >= 1; m >>= 1) weight += __shfl_xor(weight, m, 64);
+        if (lane == 0) s_weight = weight, s_count = __popcll(mask);
+    }
     __syncthreads();
-    if (!texel || k != 0) return;
-    F3 color = f3(0.0f);
-    float total = 0.0f;
-    for (uint32_t m = 0; m < n; ++m) {
-        const float4 t = s_term[int(threadIdx.x) + int(m)];
-        if (t.w > 0.0f) {
-            color += F3{t.x, t.y, t.z};
-            total += t.w;
+    const int count = s_count;
+    F3 sum = f3(0.0f);
+#pragma unroll 2
+    for (int k = wave; k < count; k += kPrefilterWaves) {
+        const PrefilterSample s = s_sample[k];
+        const F3 L = fma3(t0, f3(s.x), fma3(t1, f3(s.y), N * s.z));
+        const float ax = fabsf(L.x), ay = fabsf(L.y), az = fabsf(L.z);
+        const bool mx = ax >= ay && ax >= az, my = !mx && ay >= az;  // cube_face_st, without its branches
+        const float major = mx ? L.x : my ? L.y : L.z;
+        const bool neg = !(major >= 0.0f);
+        const float sc0 = mx ? -L.z : L.x, tc0 = my ? L.z : -L.y;
+        const float sc = neg && !my ? -sc0 : sc0, tc = neg && my ? -tc0 : tc0;
+        const float ma = fabsf(major);
+        float inv = __builtin_amdgcn_rcpf(ma);
+        inv = fmaf(fmaf(-ma, inv, 1.0f), inv, inv);
+        const float cs = fmaf(0.5f * sc, inv, 0.5f), ct = fmaf(0.5f * tc, inv, 0.5f);
+        const int cface = (mx ? 0 : my ? 2 : 4) + (neg ? 1 : 0);
+        const int l0 = __builtin_amdgcn_readfirstlane(s.level);
+        const float blend = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.blend)));
+        // Level l starts at 8 (w^2 - w_l^2) texels.
+        const int log0 = log_ew - l0;
+        const ushort4* base = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * log0)));
+        prefilter_add(base, log0, cface, cs, ct, s.z * (1.0f - blend), sum);
+        if (blend > 0.0f) {  // so there is a level l0 + 1
+            const ushort4* next = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * (log0 - 1))));
+            prefilter_add(next, log0 - 1, cface, cs, ct, s.z * blend, sum);
         }
     }
-    out[cube_level_offset(pw, level) + i] = to_rgba16f(color * (1.0f / total), 0.0f);
+    s_sum[threadIdx.x] = sum;
+    __syncthreads();
+    if (wave != 0 || !texel) return;
+#pragma unroll
+    for (int v = 1; v < kPrefilterWaves; ++v) sum = sum + s_sum[64 * v + lane];
+    dst[(long long)face * wl * wl + y * wl + x] = to_rgba16f(sum * (1.0f / s_weight), 0.0f);
 }
 
 }  // namespace skyhip
@@ -282,23 +360,19 @@ extern "C" int skyhip_environment_luminance(SkyhipContext* ctx, const SkyhipAtmo
     const AtmDev A = make_atm(*atmosphere);
     const EnvFrame e = make_env_frame(*render, *atmosphere);
     ushort4* cube = reinterpret_cast<ushort4*>(out_cube_rgba16f);
-    hipLaunchKernelGGL(env_luminance_kernel, dim3(div_up(6LL * width * width, 256)), dim3(256), 0, ctx->stream, A, e,
+    const int levels = log2i(width) + 1, tile_log = std::min(kEnvTileLog, levels - 1), tiles = width >> tile_log;
+    hipLaunchKernelGGL(env_luminance_kernel, dim3(tiles, tiles, 6), dim3(256), 0, ctx->stream, A, e,
                        reinterpret_cast<const float4*>(transmittance), transmittance_width, transmittance_height,
                        reinterpret_cast<const float4*>(sky_view_luminance),
                        reinterpret_cast<const float4*>(sky_view_transmittance), sky_view_width, sky_view_height, cube,
-                       width);
+                       width, tile_log);
     SKYHIP_LAUNCH_CHECK("env_luminance_kernel");
-    const int levels = log2i(width) + 1;
-    int l = 1;
-    for (; l < levels && (width >> l) > kMipTailWidth; ++l) {  // levels wider than the tail's buffer
-        const int wl = width >> l;
-        hipLaunchKernelGGL(cube_mip_kernel, dim3(div_up(6LL * wl * wl, 256)), dim3(256), 0, ctx->stream, cube, width,
-                           l);
-    }
-    SKYHIP_LAUNCH_CHECK("cube_mip_kernel");
-    if (l < levels) {
-        hipLaunchKernelGGL(cube_mip_tail_kernel, dim3(6), dim3(1024), 0, ctx->stream, cube, width, l, levels);
+    int l = tile_log + 1;
+    while (l < levels) {
+        const int last = (width >> l) > kMipTailWidth ? l + 1 : levels;  // a level too wide for the LDS by itself
+        hipLaunchKernelGGL(cube_mip_tail_kernel, dim3(6), dim3(1024), 0, ctx->stream, cube, width, l, last);
         SKYHIP_LAUNCH_CHECK("cube_mip_tail_kernel");
+        l = last;
     }
     return SKYHIP_OK;
 }
@@ -316,7 +390,6 @@ extern "C" int skyhip_ibl_precompute(SkyhipContext* ctx, const void* environment
     if (roughness_count < 1 || roughness_count > kMaxPrefilterLevels || (1 << (roughness_count - 1)) > prefiltered_width)
         return fail(SKYHIP_ERR_INVALID_SIZE, "roughness_count outside [1, log2(prefiltered_width) + 1]");
     const ushort4* env = reinterpret_cast<const ushort4*>(environment_cube_rgba16f);
-    const int elevels = log2i(environment_width) + 1;
     ushort4* out = reinterpret_cast<ushort4*>(out_prefiltered_rgba16f);
     PrefilterLevels lv{};
     lv.count = roughness_count;
@@ -326,15 +399,15 @@ extern "C" int skyhip_ibl_precompute(SkyhipContext* ctx, const void* environment
         lv.roughness[l] = roughness_count > 1 ? float(l) / float(roughness_count - 1) : 0.0f;
         // The level's sample count uint(mix(1, 64, pow(roughness, 0.3))) in FP32 (1 at roughness 0,
         // 64 at 1; in between, for every level of up to 13, at least 0.011 from an integer, so no
-        // powf rounding moves it), which the kernel uses as its group size and its sample count.
+        // powf rounding moves it).
         const float p = std::pow(lv.roughness[l], 0.3f);
-        lv.group[l] = std::min(std::max(int(uint32_t(1.0f * (1.0f - p) + 64.0f * p)), 1), 64);
+        lv.samples[l] = std::min(std::max(int(uint32_t(1.0f * (1.0f - p) + 64.0f * p)), 1), 64);
         lv.block_start[l] = int(blocks);
-        blocks += div_up(6LL * wl * wl, 256 / lv.group[l]);
+        blocks += div_up(6LL * wl * wl, lv.roughness[l] == 0.0f ? 64 * kPrefilterWaves : 64);
     }
     lv.block_start[roughness_count] = int(blocks);
-    hipLaunchKernelGGL(prefilter_kernel, dim3(unsigned(kSh9Blocks + blocks)), dim3(256), 0, ctx->stream, env,
-                       environment_width, elevels, reinterpret_cast<float4*>(out_sh9_rgba), out, prefiltered_width, lv);
+    hipLaunchKernelGGL(prefilter_kernel, dim3(unsigned(kSh9Blocks + blocks)), dim3(64 * kPrefilterWaves), 0, ctx->stream,
+                       env, log2i(environment_width), reinterpret_cast<float4*>(out_sh9_rgba), out, prefiltered_width, lv);
     SKYHIP_LAUNCH_CHECK("prefilter_kernel");
     return SKYHIP_OK;
 }

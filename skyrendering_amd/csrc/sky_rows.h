@@ -102,7 +102,6 @@ __device__ __forceinline__ float sun_fade(float fade_c, float fade_k, float mu_s
     const float s = clamp01((mu_s + fade_c) * fade_k);
     return s * s * fmaf(-2.0f, s, 3.0f);
 }
-__device__ __forceinline__ F3 fma3(F3 a, F3 b, F3 c) { return {fmaf(a.x, b.x, c.x), fmaf(a.y, b.y, c.y), fmaf(a.z, b.z, c.z)}; }
 // x clamped to [lo, hi] in one instruction (lo for a NaN).
 __device__ __forceinline__ float clamp_med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
 
