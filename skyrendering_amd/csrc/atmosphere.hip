@@ -6,6 +6,7 @@
 // the 64 lanes), 256-lane workgroups, 1D grids over texels so stores coalesce.
 #include "sky_rows.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace skyhip {
@@ -88,44 +89,65 @@ __global__ __launch_bounds__(64) void sky_view_rows_kernel(SkyhipAtmosphereBuffe
 // ---------------------------------------------------------------------------
 // Aerial perspective (AtmosphereRenderer.glsl:191-243)
 // ---------------------------------------------------------------------------
-// kApLanes consecutive lanes share a froxel (scattered_luminance_split): a 32^3 LUT is 32,768
-// froxels, and one lane each would leave half the SIMDs idle and the rest one wave deep.
-constexpr int kApLanes = 4;
+// Workgroup `block` of slice iz: P waves share 64 froxels (scattered_luminance_split).
+template <int P>
+__device__ __forceinline__ void aerial_perspective_block(const AtmDev& A, const RenderDev& R,
+                                                         const float* inv_view_projection, const float4* __restrict__ T,
+                                                         int tw, int th, const float4* __restrict__ MS, int mw, int mh,
+                                                         const uint16_t* __restrict__ blue_noise, int bn_size,
+                                                         float4* __restrict__ out_l, float4* __restrict__ out_t, int w,
+                                                         int h, int d, int block, int iz, SplitLds& lds) {
+    const int wave = threadIdx.x >> 6;
+    const int texel = block * (256 / P) + 64 * (wave / P) + int(threadIdx.x & 63);
+    const bool valid = texel < w * h;
+    const int t = valid ? texel : 0;
+    const AerialRay ray = aerial_ray(A, R, inv_view_projection, blue_noise, bn_size, t % w, t / w, iz, w, h, d);
+    F3 L, Tr;
+    scattered_luminance_split<P>(A, T, tw, th, MS, mw, mh, ray.s, ray.marching_distance, R.ap_steps,
+                                 ray.start_i, ray.marching_distance > 0.0f, lds, L, Tr);
+    if (wave % P == 0 && valid) {
+        const long long o = (long long)iz * w * h + t;
+        out_l[o] = make_float4(L.x, L.y, L.z, 0.0f);
+        out_t[o] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
+    }
+}
 
+// Bound by the steps' instructions, the lookups' latency and the rays' set-up, which every part repeats.
+// A 32^3 LUT at 51 steps: 12.6 us; 26.1 with four consecutive lanes to a froxel, whose lookups at four
+// distances touch four times the lines per load.  The frame around it with 1, 2 and 4 waves to 64
+// froxels takes 83.8, 72.3 and 68.8 us (consecutive lanes: 83.4, 73.3 and 78.8 with 1, 2 and 4).
+constexpr int kApParts = 4;
+struct ViewProjectionInverse {
+    float m[16];
+};
 __global__ __launch_bounds__(256) void aerial_perspective_kernel(
-    SkyhipAtmosphereBufferData b, SkyhipAtmosphereRenderBufferData rbd, const float4* __restrict__ T, int tw, int th,
+    AtmDev A, RenderDev R, ViewProjectionInverse m, const float4* __restrict__ T, int tw, int th,
     const float4* __restrict__ MS, int mw, int mh, const uint16_t* __restrict__ blue_noise, int bn_size,
     float4* __restrict__ out_l, float4* __restrict__ out_t, int w, int h, int d) {
-    const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-    const int n_texels = w * h * d;
-    const int part = int(g % kApLanes);
-    const bool valid = g / kApLanes < n_texels;
-    const int t = valid ? int(g / kApLanes) : 0;  // every lane of a group reaches the shuffles
-    const AtmDev A = make_atm(b);
-    const RenderDev R = make_render(rbd);
-    const AerialRay ray = aerial_ray(A, R, rbd.inv_view_projection, blue_noise, bn_size, t % w, (t / w) % h,
-                                     t / (w * h), w, h, d);
-    F3 L, Tr;
-    scattered_luminance_split<kApLanes>(A, T, tw, th, MS, mw, mh, ray.s, ray.marching_distance, R.ap_steps,
-                                        ray.start_i, ray.marching_distance > 0.0f, part, L, Tr);
-    if (part == 0 && valid) {
-        out_l[t] = make_float4(L.x, L.y, L.z, 0.0f);
-        out_t[t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
-    }
+    __shared__ SplitLds lds;
+    aerial_perspective_block<kApParts>(A, R, m.m, T, tw, th, MS, mw, mh, blue_noise, bn_size, out_l, out_t, w, h, d,
+                                       blockIdx.x, blockIdx.y, lds);
+}
+ViewProjectionInverse view_projection_inverse(const SkyhipAtmosphereRenderBufferData& r) {
+    ViewProjectionInverse m;
+    std::copy(r.inv_view_projection, r.inv_view_projection + 16, m.m);
+    return m;
 }
 
 // ---------------------------------------------------------------------------
 // Latency-bound form of one frame's LUT set (skyhip_atmosphere_lut_set).  A single set has
 // too few texels to fill 256 CUs one lane per texel (the 256x64 transmittance LUT is one wave
-// per CU, the 192x108 sky view 1.3), so each texel's march is split over consecutive lanes
+// per CU, the 192x108 sky view 1.3), so each texel's march is split over lanes or waves
 // and the parts combined in order, and the sky-view and aerial-perspective passes, which read
 // only T and MS, run as one launch.  Same quantities as the per-pass kernels; the FP32 sums
 // associate differently (parts add in order), which is why the batched builder, which must
 // match the per-pass kernels bit for bit, does not use these.
 // ---------------------------------------------------------------------------
 constexpr int kSetTransmittanceParts = 4;
-constexpr int kSetSkyViewParts = 3;
-constexpr int kSetAerialParts = 8;
+// Waves of a sky-view and of an aerial-perspective ray: the set takes 32.2 us with 2 and 4, 34.8 with 2
+// and 2, 32.8 with 4 and 4, 38.4 with 1 and 2, and 44.3 with 3 and 8 consecutive lanes.
+constexpr int kSetSkyViewParts = 2;
+constexpr int kSetAerialParts = 4;
 
 template <class S, int kParts>
 __device__ inline F3 transmittance_texel_split(const SkyhipAtmosphereBufferData& b, int ix, int iy, int w, int h,
@@ -186,48 +208,33 @@ __global__ __launch_bounds__(64 * kSetMsParts) void set_multiscattering_kernel(S
     if (lane == 0) out[iy * w + ix] = v;
 }
 
-// Blocks [0, sv_blocks) build the sky view, kSetSkyViewParts lanes per texel; the rest the
-// aerial perspective, kSetAerialParts lanes per froxel; a wave holds 64 / parts whole groups (a
-// lane left over idles) (no blue-noise dither, as the set's
-// per-pass calls).
+// Blocks [0, sv_blocks) build the sky view, kSetSkyViewParts waves to a texel; the rest the aerial
+// perspective, ap_blocks to a slice, kSetAerialParts waves to a froxel (no blue-noise dither, as the set's per-pass calls).
 __global__ __launch_bounds__(256) void set_sky_aerial_kernel(
-    SkyhipAtmosphereBufferData b, SkyhipAtmosphereRenderBufferData rbd, const float4* __restrict__ T, int tw, int th,
+    AtmDev A, RenderDev R, ViewProjectionInverse m, const float4* __restrict__ T, int tw, int th,
     const float4* __restrict__ MS, int mw, int mh, float4* __restrict__ sv_l, float4* __restrict__ sv_t, int sw,
-    int sh, int sv_blocks, float4* __restrict__ ap_l, float4* __restrict__ ap_t, int aw, int ah, int ad) {
-    const AtmDev A = make_atm(b);
-    const RenderDev R = make_render(rbd);
-    F3 L, Tr;
+    int sh, int sv_blocks, float4* __restrict__ ap_l, float4* __restrict__ ap_t, int aw, int ah, int ad,
+    int ap_blocks) {
+    __shared__ SplitLds lds;
     if (int(blockIdx.x) < sv_blocks) {
-        constexpr int P = kSetSkyViewParts, kPerWave = 64 / P;  // groups of P lanes within a wave
-        const int g = blockIdx.x * 256 + threadIdx.x, lane = g % 64, slot = lane / P;
-        const int part = lane % P;
-        const int texel = (g / 64) * kPerWave + slot;
-        const bool valid = slot < kPerWave && texel < sw * sh;
-        const int t = valid ? texel : 0;  // every lane of a wave reaches the shuffles
+        F3 L, Tr;
+        constexpr int P = kSetSkyViewParts;
+        const int wave = threadIdx.x >> 6;
+        const int texel = int(blockIdx.x) * (256 / P) + 64 * (wave / P) + int(threadIdx.x & 63);
+        const bool valid = texel < sw * sh;
+        const int t = valid ? texel : 0;
         const SkyViewRay ray = sky_view_ray(A, R, nullptr, 1, t % sw, t / sw, sw, sh);
         scattered_luminance_split<P>(A, T, tw, th, MS, mw, mh, ray.s, ray.dist, R.sv_steps, ray.start_i,
-                                     ray.dist > 0.0f, part, L, Tr);
-        if (part == 0 && valid) {
+                                     ray.dist > 0.0f, lds, L, Tr);
+        if (wave % P == 0 && valid) {
             sv_l[t] = make_float4(L.x, L.y, L.z, 0.0f);
             sv_t[t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
         }
         return;
     }
-    constexpr int P = kSetAerialParts, kPerWave = 64 / P;
-    const long long g = (long long)(blockIdx.x - sv_blocks) * 256 + threadIdx.x;
-    const int n_texels = aw * ah * ad;
-    const int lane = int(g % 64), slot = lane / P, part = lane % P;
-    const long long texel = (g / 64) * kPerWave + slot;
-    const bool valid = slot < kPerWave && texel < n_texels;
-    const int t = valid ? int(texel) : 0;
-    const AerialRay ray = aerial_ray(A, R, rbd.inv_view_projection, nullptr, 1, t % aw, (t / aw) % ah, t / (aw * ah),
-                                     aw, ah, ad);
-    scattered_luminance_split<P>(A, T, tw, th, MS, mw, mh, ray.s, ray.marching_distance, R.ap_steps, ray.start_i,
-                                 ray.marching_distance > 0.0f, part, L, Tr);
-    if (part == 0 && valid) {
-        ap_l[t] = make_float4(L.x, L.y, L.z, 0.0f);
-        ap_t[t] = make_float4(Tr.x, Tr.y, Tr.z, 0.0f);
-    }
+    const int block = int(blockIdx.x) - sv_blocks, iz = block / ap_blocks;
+    aerial_perspective_block<kSetAerialParts>(A, R, m.m, T, tw, th, MS, mw, mh, nullptr, 1, ap_l, ap_t, aw, ah, ad,
+                                              block - iz * ap_blocks, iz, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -310,8 +317,8 @@ int launch_aerial_perspective(hipStream_t st, const SkyhipAtmosphereBufferData& 
                               const SkyhipAtmosphereRenderBufferData& r, const float* T, int tw, int th,
                               const float* MS, int mw, int mh, const uint16_t* bn, int bn_size, float* L, float* Tr,
                               int w, int h, int d) {
-    hipLaunchKernelGGL(aerial_perspective_kernel, dim3(div_up((long long)w * h * d * kApLanes, 256)), dim3(256), 0, st,
-                       b, r,
+    hipLaunchKernelGGL(aerial_perspective_kernel, dim3(div_up((long long)w * h * kApParts, 256), d), dim3(256), 0, st,
+                       make_atm(b), make_render(r), view_projection_inverse(r),
                        reinterpret_cast<const float4*>(T), tw, th, reinterpret_cast<const float4*>(MS), mw, mh, bn,
                        bn_size, reinterpret_cast<float4*>(L), reinterpret_cast<float4*>(Tr), w, h, d);
     SKYHIP_LAUNCH_CHECK("aerial_perspective_kernel");
@@ -434,17 +441,17 @@ extern "C" int skyhip_atmosphere_lut_set(SkyhipContext* ctx, const SkyhipAtmosph
     } else {
         SKYHIP_CHECK(launch_multiscattering(st, *atmosphere, transmittance_rgba, tw, th, multiscattering_rgba, mw, mh));
     }
-    // Whole waves of 64 / parts groups each (a group never straddles two waves).
-    const int sv_blocks = int(div_up(div_up((long long)sky_view_width * sky_view_height, 64 / kSetSkyViewParts) * 64, 256));
-    const int ap_blocks =
-        int(div_up(div_up((long long)ap_width * ap_height * ap_depth, 64 / kSetAerialParts) * 64, 256));
-    hipLaunchKernelGGL(set_sky_aerial_kernel, dim3(sv_blocks + ap_blocks), dim3(256), 0, st, *atmosphere, *render,
+    const int sv_blocks = int(div_up((long long)sky_view_width * sky_view_height * kSetSkyViewParts, 256));
+    const int ap_blocks = int(div_up((long long)ap_width * ap_height * kSetAerialParts, 256));
+    hipLaunchKernelGGL(set_sky_aerial_kernel, dim3(sv_blocks + ap_blocks * ap_depth), dim3(256), 0, st,
+                       make_atm(*atmosphere), make_render(*render), view_projection_inverse(*render),
                        reinterpret_cast<const float4*>(transmittance_rgba), tw, th,
                        reinterpret_cast<const float4*>(multiscattering_rgba), mw, mh,
                        reinterpret_cast<float4*>(sky_view_luminance_rgba),
                        reinterpret_cast<float4*>(sky_view_transmittance_rgba), sky_view_width, sky_view_height,
                        sv_blocks, reinterpret_cast<float4*>(ap_luminance_rgba),
-                       reinterpret_cast<float4*>(ap_transmittance_rgba), ap_width, ap_height, ap_depth);
+                       reinterpret_cast<float4*>(ap_transmittance_rgba), ap_width, ap_height, ap_depth,
+                       ap_blocks);
     SKYHIP_LAUNCH_CHECK("set_sky_aerial_kernel");
     return SKYHIP_OK;
 }

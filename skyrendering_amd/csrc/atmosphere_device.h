@@ -160,15 +160,6 @@ __device__ inline F3 sun_visibility(const AtmDev& A, const float4* __restrict__ 
     return t * (s * s * (3.0f - 2.0f * s));
 }
 
-// GetMultiscatteringContribution (Atmosphere.glsl:169-178).
-template <bool kCells = false>
-__device__ inline F3 ms_contribution(const AtmDev& A, const float4* __restrict__ MS, int mw, int mh, float altitude,
-                                     float mu_s) {
-    float x_mu_s = mu_s * 0.5f + 0.5f;
-    float x_r = altitude * A.inv_thickness;
-    return lut_bilinear<kCells>(MS, mw, mh, x_mu_s * float(mw - 1), x_r * float(mh - 1));
-}
-
 // Geometry of a ray that starts at radius r (altitude alt0 = r - R_b) with
 // zenith cosine mu, sun zenith cosine mu_s0 and sun-view cosine nu.
 struct RayStart {
@@ -197,115 +188,160 @@ __device__ inline float distance_to_bottom(const AtmDev& A, float r, float alt0,
     return fmaxf(d, 0.0f);
 }
 
-// Per-ray constants of the integrator below.
+// Per-ray constants of the integrators below.
 struct ScatterRay {
-    float dx, rp, mp, two_r_mu, rho0_2, rb2;
+    float dx, rp, mp, two_r_mu, r_mu_s, rho0_2, rb2;
 };
 template <bool kMS>
 __device__ inline ScatterRay scatter_ray(const AtmDev& A, const RayStart& s, float marching_distance, float steps) {
     const float iso = 1.0f / (4.0f * kPiF);
     return {marching_distance / steps, kMS ? iso : rayleigh_phase(s.nu), kMS ? iso : mie_phase(A.g, s.nu),
-            2.0f * s.r * s.mu, s.alt0 * (s.r + A.rb), A.rb * A.rb};
+            2.0f * s.r * s.mu, s.r * s.mu_s0, s.alt0 * (s.r + A.rb), A.rb * A.rb};
 }
 
-// One step of the integrator at float counter value i (kCells: T and MS are cell-corner copies).
-template <bool kMS, bool kCells = false>
-__device__ __forceinline__ void scatter_step(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
-                                             const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
-                                             const ScatterRay& c, float i, F3& L, F3& Tr, F3& Lf) {
-    const float dx = c.dx;
-    float d = i * dx;
-    float q = fmaf(d, d + c.two_r_mu, c.rho0_2);  // r_d^2 - R_b^2, negative below ground
-    float r_d = fsqrt_fast(fmaxf(q + c.rb2, 0.0f));
-    float alt = fdiv_fast(q, r_d + A.rb);
-    float mu_s = fdiv_fast(s.r * s.mu_s0 + d * s.nu, r_d);
-    Densities dn = densities(A, alt);
-    F3 sr = A.rayleigh * dn.rayleigh;
-    F3 sm = A.mie_s * dn.mie;
-    F3 ext = sr + A.mie_ext * dn.mie + A.ozone * dn.ozone;
-    const F3 tr = {__expf(-ext.x * dx), __expf(-ext.y * dx), __expf(-ext.z * dx)};
-    F3 one_minus_t = {one_minus_exp(ext.x * dx, tr.x), one_minus_exp(ext.y * dx, tr.y),
-                      one_minus_exp(ext.z * dx, tr.z)};
-    F3 Li = (sr * c.rp + sm * c.mp) * sun_visibility<kCells>(A, T, tw, th, r_d, q, alt, mu_s);
-    F3 inv_ext = {__builtin_amdgcn_rcpf(ext.x), __builtin_amdgcn_rcpf(ext.y), __builtin_amdgcn_rcpf(ext.z)};
-    if (!kMS) {
-        Li += A.ms_mask * ms_contribution<kCells>(A, MS, mw, mh, alt, mu_s) * (sr + sm);
-        Li *= A.solar;
-    }
-    L += Tr * Li * one_minus_t * inv_ext;
-    if (kMS) Lf += Tr * (sr + sm) * one_minus_t * inv_ext;
-    Tr *= tr;
-}
-
-// ComputeScatteredLuminance (Atmosphere.glsl:220-295).  kMS selects the
-// MULTISCATTERING_COMPUTE_PROGRAM variant.  The loop keeps the shader's float
-// counter (i = start_i; i < steps; ++i), so fractional step counts iterate
-// exactly as the GLSL does.
-template <bool kMS, bool kCells = false>
-__device__ inline void scattered_luminance(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
-                                           const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
-                                           float marching_distance, float steps, float start_i, F3& L, F3& Tr,
-                                           F3& Lf) {
-    const ScatterRay c = scatter_ray<kMS>(A, s, marching_distance, steps);
+// ComputeScatteredLuminance (Atmosphere.glsl:220-295), MULTISCATTERING_COMPUTE_PROGRAM variant:
+// isotropic phase, no multiple scattering, and its transfer Lf beside the luminance (kCells: T is a
+// cell-corner copy).
+template <bool kCells>
+__device__ inline void scattered_luminance_ms(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
+                                              const RayStart& s, float marching_distance, F3& L, F3& Tr, F3& Lf) {
+    const ScatterRay c = scatter_ray<true>(A, s, marching_distance, A.ms_steps);
     L = f3(0.0f);
     Tr = f3(1.0f);
     Lf = f3(0.0f);
-    for (float i = kMS ? 0.5f : start_i; i < steps; i += 1.0f)
-        scatter_step<kMS, kCells>(A, T, tw, th, MS, mw, mh, s, c, i, L, Tr, Lf);
+    for (float i = 0.5f; i < A.ms_steps; i += 1.0f) {
+        const float dx = c.dx;
+        float d = i * dx;
+        float q = fmaf(d, d + c.two_r_mu, c.rho0_2);  // r_d^2 - R_b^2, negative below ground
+        float r_d = fsqrt_fast(fmaxf(q + c.rb2, 0.0f));
+        float alt = fdiv_fast(q, r_d + A.rb);
+        float mu_s = fdiv_fast(c.r_mu_s + d * s.nu, r_d);
+        Densities dn = densities(A, alt);
+        F3 sr = A.rayleigh * dn.rayleigh;
+        F3 sm = A.mie_s * dn.mie;
+        F3 ext = sr + A.mie_ext * dn.mie + A.ozone * dn.ozone;
+        const F3 tr = {__expf(-ext.x * dx), __expf(-ext.y * dx), __expf(-ext.z * dx)};
+        F3 one_minus_t = {one_minus_exp(ext.x * dx, tr.x), one_minus_exp(ext.y * dx, tr.y),
+                          one_minus_exp(ext.z * dx, tr.z)};
+        F3 Li = (sr * c.rp + sm * c.mp) * sun_visibility<kCells>(A, T, tw, th, r_d, q, alt, mu_s);
+        F3 inv_ext = {__builtin_amdgcn_rcpf(ext.x), __builtin_amdgcn_rcpf(ext.y), __builtin_amdgcn_rcpf(ext.z)};
+        L += Tr * Li * one_minus_t * inv_ext;
+        Lf += Tr * (sr + sm) * one_minus_t * inv_ext;
+        Tr *= tr;
+    }
 }
 
-// `count` consecutive steps of the same float counter, starting at counter value i0, with
-// (L, Tr) starting at (0, 1): a contiguous part of scattered_luminance's sum.  Parts combine
-// in order as L = L_a + Tr_a L_b, Tr = Tr_a Tr_b (exact in real arithmetic).
-__device__ inline void scattered_luminance_part(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
-                                                const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
-                                                const ScatterRay& c, float i0, int count, F3& L, F3& Tr) {
+// lut_bilinear with one multiply-add per texel and channel, the texels at 32-bit offsets from the
+// LUT's address.  LUTs are at least 2 x 2: the last column (row) is its cell's right (lower) edge.
+__device__ __forceinline__ F3 lut_weighted(const float4* __restrict__ lut, int w, int h, float fx, float fy) {
+    fx = __builtin_amdgcn_fmed3f(fx, 0.0f, float(w - 1));
+    fy = __builtin_amdgcn_fmed3f(fy, 0.0f, float(h - 1));
+    const int x = min(int(fx), w - 2), y = min(int(fy), h - 2);
+    const float ax = fx - float(x), ay = fy - float(y);
+    const unsigned at = 16u * unsigned(y * w + x), below = at + 16u * unsigned(w);
+    const char* base = reinterpret_cast<const char*>(lut);
+    const float4 a = *reinterpret_cast<const float4*>(base + at), b = *reinterpret_cast<const float4*>(base + at + 16);
+    const float4 c = *reinterpret_cast<const float4*>(base + below),
+                 d = *reinterpret_cast<const float4*>(base + below + 16);
+    const float w3 = ax * ay, w1 = ax - w3, w2 = ay - w3, w0 = (1.0f - ax) - w2;
+    return {fmaf(w3, d.x, fmaf(w2, c.x, fmaf(w1, b.x, w0 * a.x))), fmaf(w3, d.y, fmaf(w2, c.y, fmaf(w1, b.y, w0 * a.y))),
+            fmaf(w3, d.z, fmaf(w2, c.z, fmaf(w1, b.z, w0 * a.z)))};
+}
+
+// dx (1 - exp(-x)) / x for x = ext dx >= 0 and e = exp(-x): below x = 1/8 the series of
+// one_minus_exp over x.
+__device__ __forceinline__ float step_weight(float dx, float ext, float x, float e) {
+    const float p = fmaf(-x, fmaf(-x, fmaf(-x, fmaf(-x, 1.0f / 120.0f, 1.0f / 24.0f), 1.0f / 6.0f), 0.5f), 1.0f);
+    return x < 0.125f ? dx * p : (1.0f - e) * __builtin_amdgcn_rcpf(ext);
+}
+
+// One step of the integrator (ComputeScatteredLuminance, Atmosphere.glsl:220-295) at float counter
+// value i; L lacks the solar illuminance.  Bound by its instructions, 190 with both lookups; 261
+// with GetSunVisibility and GetMultiscatteringContribution evaluated as they stand.  With
+// p = r_d mu_s = r mu_s0 + d nu, the sun's distance to the top is sqrt(p^2 + H^2 - q) - p, and the
+// smoothstep's argument over its width (rho + p) / (2 R_b alpha) + 1/2 (alpha the sun's angular radius).
+__device__ __forceinline__ void scatter_step(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
+                                             const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
+                                             const ScatterRay& c, float i, F3& L, F3& Tr) {
+    const float dx = c.dx, d = i * dx;
+    const float q = fmaf(d, d + c.two_r_mu, c.rho0_2);  // r_d^2 - R_b^2, negative below ground
+    const float r_d = fsqrt_fast(fmaxf(q + c.rb2, 0.0f));
+    const float alt = fdiv_fast(q, r_d + A.rb);
+    const float p = fmaf(d, s.nu, c.r_mu_s), mu_s = fdiv_fast(p, r_d);
+    const float rho = fsqrt_fast(fmaxf(q, 0.0f)), d_min = A.thickness - alt;
+    const float to_top = fmaxf(fsqrt_fast(fmaxf(fmaf(p, p, A.H2 - q), 0.0f)) - p, 0.0f);
+    const float x_mu = fdiv_fast(to_top - d_min, (rho + A.H) - d_min);
+    const F3 M = lut_weighted(MS, mw, mh, fmaf(mu_s, 0.5f * float(mw - 1), 0.5f * float(mw - 1)),
+                              alt * (A.inv_thickness * float(mh - 1)));
+    F3 V = lut_weighted(T, tw, th, x_mu * float(tw - 1), rho * (A.inv_H * float(th - 1)));
+    const float f = clamp01(fmaf(rho + p, fdiv_fast(0.5f, A.rb * A.sun_angular_radius), 0.5f));
+    V = V * (f * f * fmaf(-2.0f, f, 3.0f));
+    const Densities dn = densities(A, alt);
+    const F3 sr = A.rayleigh * dn.rayleigh, sm = A.mie_s * dn.mie;
+    const F3 ext = fma3(A.ozone, f3(dn.ozone), fma3(A.mie_ext, f3(dn.mie), sr)), x = ext * dx;
+    const F3 tr = {__expf(-x.x), __expf(-x.y), __expf(-x.z)};
+    const F3 phase = fma3(sr, f3(c.rp), sm * c.mp);
+    const F3 Li = fma3(phase, V, (A.ms_mask * M) * (sr + sm));
+    const F3 weight = {step_weight(dx, ext.x, x.x, tr.x), step_weight(dx, ext.y, x.y, tr.y),
+                       step_weight(dx, ext.z, x.z, tr.z)};
+    L = fma3(Tr * weight, Li, L);
+    Tr *= tr;
+}
+
+// The loop keeps the shader's float counter (i = start_i; i < steps; ++i), so fractional step counts
+// iterate exactly as the GLSL does.
+__device__ inline void scattered_luminance(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
+                                           const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
+                                           float marching_distance, float steps, float start_i, F3& L, F3& Tr) {
+    const ScatterRay c = scatter_ray<false>(A, s, marching_distance, steps);
     L = f3(0.0f);
     Tr = f3(1.0f);
-    F3 Lf = f3(0.0f);
-    float i = i0;
-    for (int k = 0; k < count; ++k, i += 1.0f) scatter_step<false>(A, T, tw, th, MS, mw, mh, s, c, i, L, Tr, Lf);
+    for (float i = start_i; i < steps; i += 1.0f) scatter_step(A, T, tw, th, MS, mw, mh, s, c, i, L, Tr);
+    L *= A.solar;
 }
 
-// scattered_luminance<false> spread over kParts consecutive lanes of a wave (kParts a power of
-// two dividing 64; part = lane index within the group).  Part p integrates steps
-// [p c, (p + 1) c), c = ceil(n / kParts), of the shader's float counter (n its trip count,
-// i0 the counter value the loop reaches at step p c), and part 0 combines the parts in order:
-// L = L0 + Tr0 (L1 + Tr1 (...)), Tr = Tr0 Tr1 ...  All lanes of a group must call this
-// together (it shuffles); `active` (marching_distance > 0) must be the same across a group.
-// The result is valid on part 0.
+// scattered_luminance over 256 lanes, kParts waves to a ray: wave p of a group of kParts integrates steps
+// [p c, (p + 1) c), c = ceil(n / kParts), of its lanes' rays (n the float counter's trip count, i0 the
+// value the loop reaches at step p c), and the parts combine in order as L = L_a + Tr_a L_b,
+// Tr = Tr_a Tr_b (exact in real arithmetic).  Every lane of the workgroup must call this; `active`
+// (marching_distance > 0) is the ray's.  The result is valid on part 0's lanes.
+struct SplitLds {
+    float v[256][6];
+};
 template <int kParts>
 __device__ inline void scattered_luminance_split(const AtmDev& A, const float4* __restrict__ T, int tw, int th,
                                                  const float4* __restrict__ MS, int mw, int mh, const RayStart& s,
                                                  float marching_distance, float steps, float start_i, bool active,
-                                                 int part, F3& L, F3& Tr) {
+                                                 SplitLds& lds, F3& L, F3& Tr) {
+    const int part = (threadIdx.x >> 6) % kParts;
     L = f3(0.0f);
     Tr = f3(1.0f);
     if (active) {
         int n = 0;
-        for (float i = start_i; i < steps; i += 1.0f) ++n;
-        const int c = (n + kParts - 1) / kParts, first = part * c;
-        float i0 = start_i;
-        for (int k = 0; k < first && k < n; ++k) i0 += 1.0f;
-        const ScatterRay sc = scatter_ray<false>(A, s, marching_distance, steps);
-        scattered_luminance_part(A, T, tw, th, MS, mw, mh, s, sc, i0, max(0, min(c, n - first)), L, Tr);
-    }
-    F3 accL = f3(0.0f), accT = f3(1.0f);  // the parts after this lane's, combined
-    for (int p = kParts - 1; p >= 1; --p) {
-        const F3 Lp = {__shfl_down(L.x, p, 64), __shfl_down(L.y, p, 64), __shfl_down(L.z, p, 64)};
-        const F3 Tp = {__shfl_down(Tr.x, p, 64), __shfl_down(Tr.y, p, 64), __shfl_down(Tr.z, p, 64)};
-        if (p == kParts - 1) {
-            accL = Lp;
-            accT = Tp;
+        if (start_i == 0.5f) {  // no dither: the counter is exact
+            n = steps > 0.5f ? int(ceilf(steps - 0.5f)) : 0;
         } else {
-            accL = Lp + Tp * accL;
-            accT = Tp * accT;
+            for (float i = start_i; i < steps; i += 1.0f) ++n;
         }
+        const int c = (n + kParts - 1) / kParts, first = part * c;
+        float i = start_i + float(start_i == 0.5f ? first : 0);
+        if (start_i != 0.5f)
+            for (int k = 0; k < first && k < n; ++k) i += 1.0f;
+        const ScatterRay sc = scatter_ray<false>(A, s, marching_distance, steps);
+        for (int k = first; k < min(first + c, n); ++k, i += 1.0f)
+            scatter_step(A, T, tw, th, MS, mw, mh, s, sc, i, L, Tr);
     }
-    if (kParts > 1) {
-        L = L + Tr * accL;
-        Tr = Tr * accT;
+    float* v = lds.v[threadIdx.x];
+    if (part != 0) v[0] = L.x, v[1] = L.y, v[2] = L.z, v[3] = Tr.x, v[4] = Tr.y, v[5] = Tr.z;
+    __syncthreads();
+    if (part != 0) return;
+#pragma unroll
+    for (int p = 1; p < kParts; ++p) {
+        const float* o = lds.v[threadIdx.x + 64 * p];
+        L = fma3(Tr, F3{o[0], o[1], o[2]}, L);
+        Tr *= F3{o[3], o[4], o[5]};
     }
+    L *= A.solar;
 }
 
 }  // namespace skyhip

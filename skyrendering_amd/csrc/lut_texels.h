@@ -174,7 +174,7 @@ __device__ inline float4 multiscattering_texel(const AtmDev& A, const float4* __
                                                int ix, int iy, int w, int h, int lane) {
     const MsRay ray = ms_ray(A, ix, iy, w, h, lane);
     F3 L, Tr, Lf;
-    scattered_luminance<true, kCells>(A, T, tw, th, nullptr, 0, 0, ray.s, ray.dist, A.ms_steps, 0.5f, L, Tr, Lf);
+    scattered_luminance_ms<kCells>(A, T, tw, th, ray.s, ray.dist, L, Tr, Lf);
     return multiscattering_reduce<kCells>(A, T, tw, th, ray, L, Tr, Lf);
 }
 
@@ -184,7 +184,7 @@ struct RenderDev {
     float r;
     float sv_steps, ap_steps, ap_max_distance;
 };
-__device__ inline RenderDev make_render(const SkyhipAtmosphereRenderBufferData& b) {
+__host__ __device__ inline RenderDev make_render(const SkyhipAtmosphereRenderBufferData& b) {
     RenderDev d;
     d.sun = f3(b.sun_direction);
     d.up = f3(b.up_direction);
@@ -280,24 +280,23 @@ __device__ inline void sky_view_texel(const AtmDev& A, const RenderDev& R, const
     const SkyViewRay ray = sky_view_ray(A, R, blue_noise, bn_size, ix, iy, w, h);
     L = f3(0.0f);
     Tr = f3(1.0f);
-    F3 Lf;
     if (ray.dist > 0.0f)
-        scattered_luminance<false>(A, T, tw, th, MS, mw, mh, ray.s, ray.dist, R.sv_steps, ray.start_i, L, Tr, Lf);
+        scattered_luminance(A, T, tw, th, MS, mw, mh, ray.s, ray.dist, R.sv_steps, ray.start_i, L, Tr);
 }
 
 // ProjectiveMul(inv_view_projection, (x, y, z)) - camera, normalised; the
 // unprojection is done in FP64 (once per texel) so the direction keeps full
 // FP32 accuracy however far the camera is from the world origin.
-__device__ inline F3 unproject_direction(const float* m, float x, float y, float z, F3 cam, double* out_w_dist) {
+__device__ inline F3 unproject_direction(const float* m, float x, float y, float z, F3 cam) {
     double v[4] = {x, y, z, 1.0};
     double o[4];
     for (int row = 0; row < 4; ++row)
         o[row] = double(m[row]) * v[0] + double(m[4 + row]) * v[1] + double(m[8 + row]) * v[2] +
                  double(m[12 + row]) * v[3];
-    double px = o[0] / o[3] - double(cam.x), py = o[1] / o[3] - double(cam.y), pz = o[2] / o[3] - double(cam.z);
-    double len = sqrt(px * px + py * py + pz * pz);
-    if (out_w_dist) *out_w_dist = len;
-    return {float(px / len), float(py / len), float(pz / len)};
+    const double inv_w = 1.0 / o[3];
+    double px = o[0] * inv_w - double(cam.x), py = o[1] * inv_w - double(cam.y), pz = o[2] * inv_w - double(cam.z);
+    const double inv_len = 1.0 / sqrt(px * px + py * py + pz * pz);
+    return {float(px * inv_len), float(py * inv_len), float(pz * inv_len)};
 }
 
 // The set-up of one aerial-perspective froxel (:191-243): the ray start, the marching distance
@@ -310,7 +309,7 @@ __device__ inline AerialRay aerial_ray(const AtmDev& A, const RenderDev& R, cons
                                        const uint16_t* __restrict__ blue_noise, int bn_size, int ix, int iy, int iz,
                                        int w, int h, int d) {
     const float u = float(ix) / float(w - 1), v = float(iy) / float(h - 1), q = float(iz) / float(d - 1);
-    const F3 view = unproject_direction(inv_view_projection, u * 2.0f - 1.0f, v * 2.0f - 1.0f, 0.0f, R.cam, nullptr);
+    const F3 view = unproject_direction(inv_view_projection, u * 2.0f - 1.0f, v * 2.0f - 1.0f, 0.0f, R.cam);
     float marching_distance = q * q * R.ap_max_distance;
     const float r = R.r;
     const float alt0 = r - A.rb;

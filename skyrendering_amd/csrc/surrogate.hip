@@ -123,8 +123,8 @@ __device__ inline F3 sky_radiance(const AtmDev& A, const float4* __restrict__ T,
     const bool hit = ray_hits_ground(A, r, h, mu_v);
     float dist = hit ? distance_to_bottom(A, r, h, mu_v) : distance_to_top(A, r, h, mu_v);
     start_from_space(A, s, dist);
-    F3 L = f3(0.0f), Tr, Lf;
-    if (dist > 0.0f) scattered_luminance<false>(A, T, tw, th, MS, mw, mh, s, dist, steps, 0.5f, L, Tr, Lf);
+    F3 L = f3(0.0f), Tr;
+    if (dist > 0.0f) scattered_luminance(A, T, tw, th, MS, mw, mh, s, dist, steps, 0.5f, L, Tr);
     return L;
 }
 
