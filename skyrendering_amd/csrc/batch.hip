@@ -411,15 +411,22 @@ int time_pass(SkyhipLutBatch* b, F enqueue, int reps, float* out_ms) {
     return SKYHIP_OK;
 }
 
-SkyhipLutBatchTuning default_tuning() {
+// Tiles of many texels set up a row per lane and keep the counter quiet; few of them leave workgroups
+// idle.  us per launch at sky-view tiles of 256 / 1,024 / 4,096 texels: 0.2 M texels 205 / 235 / 331,
+// 1.1 M 295 / 290 / 363, 3.2 M 431 / 359 / 409, 17 M 2,009 / 1,465 / 1,482; 74 M 3.0 against 2.8 ms for
+// the pass at 1,024 and 4,096.  Transmittance tiles of 256 against 1,024 texels (whose last columns
+// integrate in FP64): 6 sets 159 / 205 us, 40 407 / 434, 256 1,776 / 1,842.
+SkyhipLutBatchTuning default_tuning(const SkyhipLutBatch& b) {
+    long long sv_texels = 0;
+    for (const BatchViewDev& v : b.views) sv_texels += (long long)v.sw * v.sh;
     SkyhipLutBatchTuning t{};
     t.transmittance_block = 256;
-    t.transmittance_tile = 1024;
+    t.transmittance_tile = 256;
     t.transmittance_blocks_per_cu = 4;
     t.multiscattering_waves = 4;
     t.multiscattering_blocks_per_cu = 8;
     t.sky_view_block = 256;
-    t.sky_view_tile = 4096;
+    t.sky_view_tile = sv_texels < 1 << 20 ? 256 : sv_texels < 1 << 25 ? 1024 : 4096;
     t.sky_view_blocks_per_cu = 4;
     t.sky_view_largest_first = 1;
     return t;
@@ -505,7 +512,7 @@ extern "C" int skyhip_lut_batch_create(SkyhipContext* ctx, const SkyhipLutBatchS
         return bad(rc);
     hipError_t e = hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking);
     if (e != hipSuccess) return bad(check_hip(e, "hipStreamCreate (batch)"));
-    if ((rc = apply_tuning(b, default_tuning())) != SKYHIP_OK) return bad(rc);
+    if ((rc = apply_tuning(b, default_tuning(*b))) != SKYHIP_OK) return bad(rc);
     *out = b;
     return SKYHIP_OK;
 }
