@@ -45,7 +45,9 @@ HBM_PEAK_GBS = 8000.0
 # divided by the executed sample-steps (raymarch: 7.3665e9 over 35,111,907) or integrator steps
 # (LUT set, counted on the one-lane-per-texel kernels so that the split kernels' repeated ray
 # set-up is not counted as work: 1.0386e9 over 4,914,688; batch: 7.184e11 over 3,024,532,480)
-# of the same launches.
+# of the same launches.  The LUT set's, the batch's and the environment's are the operations of the
+# texel-by-texel, sample-by-sample forms: the kernels share a row's steps and a level's samples since
+# and execute fewer, so their rates are equivalent ones.
 RAYMARCH_KERNEL = "cloud_raymarch_kernel<5,false>"
 RAYMARCH_FP32_FLOP_PER_STEP = 209.8
 LUT_SET_FLOP_PER_STEP = 211.3
