@@ -78,13 +78,14 @@ __host__ __device__ inline AtmDev make_atm(const SkyhipAtmosphereBufferData& b) 
 __device__ __forceinline__ float fdiv_fast(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 __device__ __forceinline__ float fsqrt_fast(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-// 1 - exp(-x) for x >= 0 given e = exp(-x): below x = 1/8 the series x - x^2/2 + ... + x^5/120
-// (truncation < 1e-8 relative), which keeps the relative precision that 1 - e loses to
-// cancellation for small x; above, 1 - e (cancellation costs at most 1/(1 - e^-1/8) ~ 8.5x
-// of e's rounding).
-__device__ __forceinline__ float one_minus_exp(float x, float e) {
-    const float series = x * (1.0f - x * (0.5f - x * (1.0f / 6.0f - x * (1.0f / 24.0f - x * (1.0f / 120.0f)))));
-    return x < 0.125f ? series : 1.0f - e;
+// (1 - exp(-ext dx)) / ext for x = ext dx >= 0 and e = exp(-x), the weight of a step's in-scattering:
+// below x = 1/8 the series dx (1 - x/2 + ... + x^4/120) (truncation < 1e-8 relative), which keeps the
+// relative precision that 1 - e loses to cancellation for small x and is dx where ext is 0 (a
+// reciprocal of it is infinite); above, 1 - e (cancellation costs at most 1/(1 - e^-1/8) ~ 8.5x of e's
+// rounding).
+__device__ __forceinline__ float step_weight(float dx, float ext, float x, float e) {
+    const float p = fmaf(-x, fmaf(-x, fmaf(-x, fmaf(-x, 1.0f / 120.0f, 1.0f / 24.0f), 1.0f / 6.0f), 0.5f), 1.0f);
+    return x < 0.125f ? dx * p : (1.0f - e) * __builtin_amdgcn_rcpf(ext);
 }
 
 // Atmosphere.glsl:119-132 / :156-159 split into densities so the exps are shared.
@@ -221,12 +222,11 @@ __device__ inline void scattered_luminance_ms(const AtmDev& A, const float4* __r
         F3 sm = A.mie_s * dn.mie;
         F3 ext = sr + A.mie_ext * dn.mie + A.ozone * dn.ozone;
         const F3 tr = {__expf(-ext.x * dx), __expf(-ext.y * dx), __expf(-ext.z * dx)};
-        F3 one_minus_t = {one_minus_exp(ext.x * dx, tr.x), one_minus_exp(ext.y * dx, tr.y),
-                          one_minus_exp(ext.z * dx, tr.z)};
+        const F3 weight = {step_weight(dx, ext.x, ext.x * dx, tr.x), step_weight(dx, ext.y, ext.y * dx, tr.y),
+                           step_weight(dx, ext.z, ext.z * dx, tr.z)};
         F3 Li = (sr * c.rp + sm * c.mp) * sun_visibility<kCells>(A, T, tw, th, r_d, q, alt, mu_s);
-        F3 inv_ext = {__builtin_amdgcn_rcpf(ext.x), __builtin_amdgcn_rcpf(ext.y), __builtin_amdgcn_rcpf(ext.z)};
-        L += Tr * Li * one_minus_t * inv_ext;
-        Lf += Tr * (sr + sm) * one_minus_t * inv_ext;
+        L += Tr * Li * weight;
+        Lf += Tr * (sr + sm) * weight;
         Tr *= tr;
     }
 }
@@ -246,13 +246,6 @@ __device__ __forceinline__ F3 lut_weighted(const float4* __restrict__ lut, int w
     const float w3 = ax * ay, w1 = ax - w3, w2 = ay - w3, w0 = (1.0f - ax) - w2;
     return {fmaf(w3, d.x, fmaf(w2, c.x, fmaf(w1, b.x, w0 * a.x))), fmaf(w3, d.y, fmaf(w2, c.y, fmaf(w1, b.y, w0 * a.y))),
             fmaf(w3, d.z, fmaf(w2, c.z, fmaf(w1, b.z, w0 * a.z)))};
-}
-
-// dx (1 - exp(-x)) / x for x = ext dx >= 0 and e = exp(-x): below x = 1/8 the series of
-// one_minus_exp over x.
-__device__ __forceinline__ float step_weight(float dx, float ext, float x, float e) {
-    const float p = fmaf(-x, fmaf(-x, fmaf(-x, fmaf(-x, 1.0f / 120.0f, 1.0f / 24.0f), 1.0f / 6.0f), 0.5f), 1.0f);
-    return x < 0.125f ? dx * p : (1.0f - e) * __builtin_amdgcn_rcpf(ext);
 }
 
 // One step of the integrator (ComputeScatteredLuminance, Atmosphere.glsl:220-295) at float counter

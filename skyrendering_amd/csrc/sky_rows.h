@@ -80,9 +80,8 @@ __device__ inline RowStep row_step(const AtmDev& A, const RowRay& ray, float dx,
     const F3 before = {half_wave_product(in ? tr.x : 1.0f, all.x), half_wave_product(in ? tr.y : 1.0f, all.y),
                        half_wave_product(in ? tr.z : 1.0f, all.z)};
     const F3 w = carry * before *
-                 F3{one_minus_exp(ext.x * dx, tr.x) * __builtin_amdgcn_rcpf(ext.x),
-                    one_minus_exp(ext.y * dx, tr.y) * __builtin_amdgcn_rcpf(ext.y),
-                    one_minus_exp(ext.z * dx, tr.z) * __builtin_amdgcn_rcpf(ext.z)};
+                 F3{step_weight(dx, ext.x, ext.x * dx, tr.x), step_weight(dx, ext.y, ext.y * dx, tr.y),
+                    step_weight(dx, ext.z, ext.z * dx, tr.z)};
     s.wr = w * sr;
     s.wm = w * sm;
     carry *= all;
