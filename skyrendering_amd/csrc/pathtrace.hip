@@ -834,7 +834,8 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
         const unsigned long long hits = __ballot(taken);
         if (on) {
             const unsigned long long mine = (hits >> (K * rank)) & (K == 64 ? ~0ull : (1ull << K) - 1ull);
-            if (mine != 0ull) {
+            const int left_steps = kMaxTrackingSteps - it;  // draws past the limit do not count
+            if (mine != 0ull && __builtin_ctzll(mine) < left_steps) {
                 const int j = K * rank + __builtin_ctzll(mine);
                 t = s.t[j];
                 rng.s = s.state[j];
@@ -843,7 +844,11 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
             } else {
                 t = tt;
                 it += n;
-                on = !left && it < kMaxTrackingSteps;
+                on = !left;
+                if (n >= left_steps) {
+                    rng.s = s.state[K * rank + left_steps - 1];
+                    on = false;
+                }
             }
         }
     }
@@ -889,6 +894,7 @@ __device__ __forceinline__ float coop_ratio_track(const PtArgs& a, CoopLds& s, b
         s.sigma[threadIdx.x] = coop_lookup<kMat>(a, s, tracking, K);
         wave_lds_fence();
         if (on) {
+            n = min(n, kMaxTrackingSteps - it);  // draws past the limit do not count
             for (int j = 0; j < n; ++j) tr *= 1.0f - fmaxf(0.0f, s.sigma[K * rank + j] * a.inv_sigma_t_max);
             it += n;
             on = !left && it < kMaxTrackingSteps;
