@@ -903,7 +903,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
 // ---------------------------------------------------------------------------
 // The residual check by panorama rows.
 // ---------------------------------------------------------------------------
-constexpr int kMaxTilesX = 1024;  // 16,384 pixels
 template <int P, class Atm>
 __device__ __forceinline__ void panorama_scatter(const Atm& atm, const SkyLuts& luts, int atmosphere,
                                                  const PanoramaRow& r, const float (&nu)[P], RowLds& lds, F3 (&L)[P]) {
@@ -921,23 +920,30 @@ __device__ __forceinline__ void panorama_scatter(const Atm& atm, const SkyLuts& 
 }
 
 constexpr int kCheckWaves = 4, kCheckRays = 2;
-// The residual check of tile row blockIdx.x of view blockIdx.y: its tiles' probes lie in two pixel rows.
+constexpr int kCheckTiles = kCheckWaves * kCheckRays * 64 / 4;  // their probes are one march of every wave
+// The residual check of a tile row of view blockIdx.y, or of one of its `parts` of up to kCheckTiles tiles
+// (2,048 pixels; with the network pass an image of 16,384 x 16 takes 47.6 us, 143.6 with a row of tiles in
+// one workgroup, 67.6 with a thread per probe): the tiles' probes lie in two pixel rows.
 // Four waves of two rays a lane take 1920 wide's 2 x 240 probes at once; 16 such views with the network
 // pass 1,364 us, 1,426 with every probe marching for itself (2 waves of four rays 1,367, of one 1,405).
-__global__ __launch_bounds__(64 * kCheckWaves) __attribute__((amdgpu_waves_per_eu(3))) void sky_check_rows_kernel(SkyRenderArgs a) {
+__global__ __launch_bounds__(64 * kCheckWaves) __attribute__((amdgpu_waves_per_eu(3))) void sky_check_rows_kernel(
+    SkyRenderArgs a, int parts) {
     __shared__ RowLds lds[kCheckWaves];
     __shared__ PanoramaRow rows[2];
-    __shared__ uint32_t worst[kMaxTilesX];  // the tiles' largest residuals (float bits, which order as the floats do)
-    const int view = blockIdx.y, ty = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ uint32_t worst[kCheckTiles];  // the tiles' largest residuals (float bits, which order as the floats do)
+    const int view = blockIdx.y, ty = int(blockIdx.x) / parts, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int part_tiles = (a.tiles_x + parts - 1) / parts, t0 = (int(blockIdx.x) - ty * parts) * part_tiles;
+    const int tiles = min(part_tiles, a.tiles_x - t0);
+    if (tiles <= 0) return;  // workgroup-uniform
     const int w = a.width, h = a.height;
     const SkyhipSkyView v = a.views[view];
     const int atmosphere = clamp_index(v.atmosphere, a.luts.count);
     const auto atm = [&] { return make_atm(*reload(a.luts.atm + atmosphere)); };
-    for (int t = threadIdx.x; t < a.tiles_x; t += 64 * kCheckWaves) worst[t] = 0u;
+    for (int t = threadIdx.x; t < tiles; t += 64 * kCheckWaves) worst[t] = 0u;
     if (threadIdx.x < 2) rows[threadIdx.x] = panorama_row(atm(), v, min(ty * 16 + 4 + 8 * int(threadIdx.x), h - 1), h);
     __syncthreads();
     constexpr int P = kCheckRays;
-    const int samples = 2 * a.tiles_x, pieces = (samples + 64 * P - 1) / (64 * P);
+    const int samples = 2 * tiles, pieces = (samples + 64 * P - 1) / (64 * P);
     for (int i = wave; i < 2 * pieces; i += kCheckWaves) {
         const int y = i / pieces, s0 = (i - y * pieces) * 64 * P;
         const PanoramaRow r = rows[y];
@@ -948,7 +954,7 @@ __global__ __launch_bounds__(64 * kCheckWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int s = min(s0 + 64 * p + lane, samples - 1);
-            x[p] = min((s >> 1) * 16 + 4 + 8 * (s & 1), w - 1);
+            x[p] = min((t0 + (s >> 1)) * 16 + 4 + 8 * (s & 1), w - 1);
             nu[p] = panorama_nu(r, x[p], w);
         }
         panorama_scatter<P>(atm, a.luts, atmosphere, r, nu, lds[wave], L);
@@ -968,9 +974,9 @@ __global__ __launch_bounds__(64 * kCheckWaves) __attribute__((amdgpu_waves_per_e
     }
     __syncthreads();
     int failed = 0;
-    for (int t = threadIdx.x; t < a.tiles_x; t += 64 * kCheckWaves) {
+    for (int t = threadIdx.x; t < tiles; t += 64 * kCheckWaves) {
         const unsigned f = __uint_as_float(worst[t]) > a.tolerance ? 1u : 0u;
-        a.flags[((long long)view * a.tiles_y + ty) * a.tiles_x + t] = f;
+        a.flags[((long long)view * a.tiles_y + ty) * a.tiles_x + t0 + t] = f;
         failed += f;
     }
     if (failed) atomicAdd(&a.counters[0], unsigned(failed));
@@ -1267,7 +1273,9 @@ extern "C" int skyhip_sky_render_surrogate(SkyhipContext* ctx, int32_t network, 
         hipLaunchKernelGGL(sky_render_surrogate_kernel<NetBF16SiLU>, dim3(blocks), dim3(256), 0, st, params, a,
                            view_count);
     if (row_luts_fit(a.luts.tw, a.luts.mw)) {
-        hipLaunchKernelGGL(sky_check_rows_kernel, dim3(a.tiles_y, view_count), dim3(64 * kCheckWaves), 0, st, a);
+        const int parts = int(div_up(a.tiles_x, kCheckTiles));
+        hipLaunchKernelGGL(sky_check_rows_kernel, dim3(a.tiles_y * parts, view_count), dim3(64 * kCheckWaves), 0, st, a,
+                           parts);
     } else {
         const long long probes = 4LL * a.tiles_x * a.tiles_y * view_count;
         hipLaunchKernelGGL(sky_render_check_kernel, dim3(unsigned((probes + 255) / 256)), dim3(256), 0, st, a,

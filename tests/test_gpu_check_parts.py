@@ -1,0 +1,45 @@
+"""The residual check of images wider than one workgroup's tiles (128, 2,048 pixels): every tile of every part
+gets its flag and its probes, whether none, some or all tiles fail."""
+
+import numpy as np
+import pytest
+
+from skyrendering_amd import surrogate as sg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("w,h", [(2048, 17), (2049, 16), (4112, 33), (16384, 5)])
+def test_check_parts_flag_every_tile(ctx, w, h):
+    scales, views = sg.evaluation_views(2, seed=5)
+    atm = sg.SkyAtmospheres(ctx, scales)
+    pano = sg.SkyPanoramas(ctx, atm, views, w, h)
+    model = sg.SkySurrogate(ctx, seed=3)
+    tx, ty = (w + 15) // 16, (h + 15) // 16
+
+    def render(tolerance):
+        pano.flags.upload(np.full(2 * pano.tiles, 7, np.uint32))
+        pano.render_surrogate(model, tolerance=tolerance)
+        flags = pano.flags.download(np.uint32, (2, ty, tx))
+        assert pano.fallback_tiles() == flags.sum()
+        return pano.image()[..., :3], flags
+
+    pano.render_plain()
+    plain = pano.image()[..., :3]
+    network, flags = render(1e30)
+    assert not flags.any()
+    ys = sorted({min(t + o, h - 1) for t in range(0, h, 16) for o in (4, 12)})
+    xs = sorted({min(t + o, w - 1) for t in range(0, w, 16) for o in (4, 12)})
+    for v in range(2):
+        probes, ref = network[v][np.ix_(ys, xs)], plain[v][np.ix_(ys, xs)]
+        # Two forms of one march, each within 4e-7 (relative 2-norm) of 64 bits except along the horizon.
+        assert np.linalg.norm(probes - ref) < 1e-4 * np.linalg.norm(ref)
+    image, flags = render(1e-30)
+    assert (flags == 1).all() and np.array_equal(image, plain)
+    # A tolerance between the tiles' residuals (of their other pixels: the probes are the integrator's).
+    residual = (np.abs(network - plain) / np.maximum(plain, 1e-6)).max(-1)
+    tiles = [residual[v, y:y + 16, x:x + 16].max() for v in range(2) for y in range(0, h, 16) for x in range(0, w, 16)]
+    image, flags = render(float(np.median(tiles)))
+    assert 0 < flags.sum() < flags.size and set(np.unique(flags)) == {0, 1}
+    failed = np.repeat(np.repeat(flags, 16, 1), 16, 2)[:, :h, :w, None] == 1
+    assert np.array_equal(image, np.where(failed, plain, network))
