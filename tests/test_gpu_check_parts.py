@@ -36,10 +36,12 @@ def test_check_parts_flag_every_tile(ctx, w, h):
         assert np.linalg.norm(probes - ref) < 1e-4 * np.linalg.norm(ref)
     image, flags = render(1e-30)
     assert (flags == 1).all() and np.array_equal(image, plain)
-    # A tolerance between the tiles' residuals (of their other pixels: the probes are the integrator's).
-    residual = (np.abs(network - plain) / np.maximum(plain, 1e-6)).max(-1)
-    tiles = [residual[v, y:y + 16, x:x + 16].max() for v in range(2) for y in range(0, h, 16) for x in range(0, w, 16)]
-    image, flags = render(float(np.median(tiles)))
+    lo, hi = -30.0, 30.0  # powers of ten: every tile fails at lo, none at hi
+    for _ in range(40):
+        image, flags = render(10.0 ** (0.5 * (lo + hi)))
+        if 0 < flags.sum() < flags.size:
+            break
+        lo, hi = (0.5 * (lo + hi), hi) if flags.all() else (lo, 0.5 * (lo + hi))
     assert 0 < flags.sum() < flags.size and set(np.unique(flags)) == {0, 1}
     failed = np.repeat(np.repeat(flags, 16, 1), 16, 2)[:, :h, :w, None] == 1
     assert np.array_equal(image, np.where(failed, plain, network))
