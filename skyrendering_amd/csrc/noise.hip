@@ -338,8 +338,29 @@ __global__ __launch_bounds__(256) void displacement_kernel(SkyhipNoiseCreateInfo
     if (p.in) out[4ll * (p.y * size + p.x) + blockIdx.z] = v;
 }
 
-// Up to kMipLevels mip steps of a UNORM8 texture: box over 2x2(x2) source texels (indices clamped to
-// the source level), (sum + n/2) / n.  A workgroup computes a tile of the first level (2^kTileLog texels
+// One mip step of a UNORM8 texture: box over 2x2(x2) source texels (indices clamped to the source level),
+// (sum + n/2) / n.  A lane per byte of the level, neighbouring lanes at neighbouring bytes.
+template <int kDims, int kChannels>
+__global__ __launch_bounds__(256) void downsample_level_kernel(const uint8_t* __restrict__ src, int sx, int sy, int sz,
+                                                               uint8_t* __restrict__ dst, int dx, int dy, int dz) {
+    constexpr int kBox = kDims == 3 ? 8 : 4;
+    const unsigned t = blockIdx.x * 256u + threadIdx.x;  // the level's bytes fit 32 bits (the launch's)
+    if (t >= unsigned(dx) * unsigned(dy) * unsigned(dz) * unsigned(kChannels)) return;
+    const unsigned texel = t / kChannels, c = t - texel * kChannels, row = texel / unsigned(dx);
+    const int x = int(texel - row * unsigned(dx));
+    const unsigned uz = kDims == 3 ? row / unsigned(dy) : 0u;
+    const int z = int(uz), y = int(row - uz * unsigned(dy));
+    int sum = 0;
+#pragma unroll
+    for (int k = 0; k < kBox; ++k) {
+        const int xx = min(2 * x + (k & 1), sx - 1), yy = min(2 * y + ((k >> 1) & 1), sy - 1);
+        const int zz = kDims == 3 ? min(2 * z + ((k >> 2) & 1), sz - 1) : 0;
+        sum += src[(((long long)zz * sy + yy) * sx + xx) * kChannels + c];
+    }
+    dst[t] = uint8_t((sum + kBox / 2) / kBox);
+}
+
+// Up to kMipLevels mip steps in one launch.  A workgroup computes a tile of the first level (2^kTileLog texels
 // a side) from the source in memory, and, a tile's edge being even, its part of the next levels from
 // the one before in LDS.  Bound by launches: an edit's four chains (512^2, two of 128
 // and 32 a side) are 11 launches of 4.4 to 4.9 us; a launch per level made 28 of 1 to 4 us, and the edit
@@ -418,6 +439,22 @@ dim3 image_grid(int size, int channels) {
 }
 dim3 volume_grid(int nx, int ny, int nz) {
     return dim3(div_up(nx, kVolumeTileXY), div_up(ny, kVolumeTileXY), div_up(nz, kVolumeTileZ));
+}
+
+// Levels the next launch of a chain makes by tiles, or 0 for one level by bytes: tiles save launches (3.1 us
+// each), bytes are read and stored faster, and a thin level fills little of a tile.  us, level by level /
+// by tiles: one level of 512^2 3.6 / 3.6, three 9.6 / 3.8; three of 2048^2 (4,096 tiles) 9.8 / 7.5, of
+// 4096^2 17.1 / 21.5 and with four channels 39.3 / 35.8, of 1 x 2^20 texels of four bytes (32,768 tiles)
+// 10.5 / 60.9; three of 128^3 (512) 9.8 / 5.3, of 256^3 (4,096) 14.7 / 24.0; two of 64^3 with four channels
+// 6.7 / 7.5.  (Below 4 GiB no grid of tiles has more than 8,192 in y or z.)
+int mip_tile_levels(int dims, int channels, int dx, int dy, int dz, int remaining) {
+    const int edge = dims == 3 ? 8 : 16;
+    const bool full = dx >= edge && dy >= edge;
+    if ((long long)dx * dy * dz * channels > (1ll << 32) - 256) return std::min(kMipLevels, remaining);  // the bytes' index
+    if (dims == 2 && channels == 4 && full && std::max(dx, dy) <= 1 << 14) return std::min(kMipLevels, remaining);
+    const long long tiles = (long long)div_up(dx, edge) * div_up(dy, edge) * div_up(dz, dims == 3 ? edge : 1);
+    const int most = dims == 3 ? 1024 : full ? 8192 : remaining > 2 ? 4096 : 2048;
+    return tiles <= most && remaining >= (dims == 3 && channels > 2 ? 3 : 2) ? std::min(kMipLevels, remaining) : 0;
 }
 
 int validate_noise(const SkyhipNoiseCreateInfo* ci) {
@@ -574,26 +611,30 @@ extern "C" int skyhip_generate_mipmaps(SkyhipContext* ctx, uint8_t* texture, int
         return fail(SKYHIP_ERR_INVALID_SIZE, "bad texture size or level count");
     size_t off = 0;
     int sx = width, sy = height, sz = depth;
-    for (int l = 1; l < levels; l += kMipLevels) {
-        const int n = std::min(kMipLevels, levels - l), tile = dims == 3 ? 8 : 16;
-        const dim3 grid(div_up(std::max(sx / 2, 1), tile), div_up(std::max(sy / 2, 1), tile),
-                        dims == 3 ? div_up(std::max(sz / 2, 1), tile) : 1);
-        size_t src_bytes = size_t(sx) * sy * sz * channels;
-        auto launch = [&](auto c) {
-            constexpr int kC = decltype(c)::value;
-            if (dims == 3)
-                hipLaunchKernelGGL((downsample_kernel<3, kC>), grid, dim3(256), 0, ctx->stream, texture + off, sx, sy, sz,
-                                   texture + off + src_bytes, n);
+    for (int l = 1; l < levels;) {
+        const int dx = std::max(sx / 2, 1), dy = std::max(sy / 2, 1), dz = std::max(sz / 2, 1);
+        const int n = mip_tile_levels(dims, channels, dx, dy, dz, levels - l);
+        auto launch = [&](auto d, auto c) {
+            constexpr int kD = decltype(d)::value, kC = decltype(c)::value, kEdge = kD == 3 ? 8 : 16;
+            uint8_t *src = texture + off, *dst = src + size_t(sx) * sy * sz * kC;
+            if (n == 0)
+                hipLaunchKernelGGL((downsample_level_kernel<kD, kC>), dim3(div_up((long long)dx * dy * dz * kC, 256)),
+                                   dim3(256), 0, ctx->stream, src, sx, sy, sz, dst, dx, dy, dz);
             else
-                hipLaunchKernelGGL((downsample_kernel<2, kC>), grid, dim3(256), 0, ctx->stream, texture + off, sx, sy, sz,
-                                   texture + off + src_bytes, n);
+                hipLaunchKernelGGL((downsample_kernel<kD, kC>),
+                                   dim3(div_up(dx, kEdge), div_up(dy, kEdge), kD == 3 ? div_up(dz, kEdge) : 1), dim3(256),
+                                   0, ctx->stream, src, sx, sy, sz, dst, n);
         };
-        if (channels == 1) launch(std::integral_constant<int, 1>());
-        else if (channels == 2) launch(std::integral_constant<int, 2>());
-        else if (channels == 3) launch(std::integral_constant<int, 3>());
-        else launch(std::integral_constant<int, 4>());
+        auto channel = [&](auto d) {
+            if (channels == 1) launch(d, std::integral_constant<int, 1>());
+            else if (channels == 2) launch(d, std::integral_constant<int, 2>());
+            else if (channels == 3) launch(d, std::integral_constant<int, 3>());
+            else launch(d, std::integral_constant<int, 4>());
+        };
+        if (dims == 3) channel(std::integral_constant<int, 3>());
+        else channel(std::integral_constant<int, 2>());
         SKYHIP_LAUNCH_CHECK("downsample_kernel");
-        for (int k = 0; k < n; ++k) {
+        for (int k = 0; k < std::max(n, 1); ++k, ++l) {
             off += size_t(sx) * sy * sz * channels;
             sx = std::max(sx / 2, 1), sy = std::max(sy / 2, 1), sz = std::max(sz / 2, 1);
         }
