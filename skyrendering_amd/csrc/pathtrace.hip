@@ -1024,30 +1024,46 @@ constexpr int kRefillBlocksPerCu = 5;
 // body in every iteration.
 constexpr int kRefillMaxBrick = 4;
 
-// The tile of paths of a wave: the largest of 8 x 8, 8 x 4, .. 1 x 1 that makes three waves for every
-// SIMD.  ms per frame of the procedural cloud at 64 / 32 / 16 / 8 / 4 / 2 paths: 96 x 64 12.0 / 7.8 /
-// 5.4 / 4.2 / 3.4 / 2.9, 321 x 181 12.5 / 9.0 / 6.3 / 7.3, 640 x 360 14.3 / 15.3 / 15.4 / 18.9,
+// The tile of paths of a wave of the cooperative kernel: the largest of 8 x 8, 8 x 4, .. 1 x 1 that makes
+// three waves for every SIMD.  ms per frame of the procedural cloud at 64 / 32 / 16 / 8 / 4 / 2 paths: 96 x 64
+// 12.0 / 7.8 / 5.4 / 4.2 / 3.4 / 2.9, 321 x 181 12.5 / 9.0 / 6.3 / 7.3, 640 x 360 14.3 / 15.3 / 15.4 / 18.9,
 // 1280 x 720 33.5 / 38.8 / 48.4 / 67.0.
-template <int kMat>
-static void launch_coop(hipStream_t st, PtArgs a, int cu_count) {
+static void coop_tile(PtArgs& a, int cu_count) {
     const long long w = a.region[2] - a.region[0], h = a.region[3] - a.region[1], waves = 3ll * 4 * cu_count;
     a.coop_log_x = a.coop_log_y = 3;
     while (a.coop_log_x + a.coop_log_y > 0 &&
            (long long)div_up(w, 1 << a.coop_log_x) * div_up(h, 1 << a.coop_log_y) < waves)
         --(a.coop_log_x == a.coop_log_y ? a.coop_log_y : a.coop_log_x);
-    hipLaunchKernelGGL(path_trace_coop_kernel<kMat>, dim3(div_up(w, 1 << a.coop_log_x), div_up(h, 1 << a.coop_log_y)),
-                       dim3(64), 0, st, a);
+}
+
+// Whether a frame with one majorant is faster with a lane per path.  A constant medium's lookup costs less than
+// sharing it (us, a lane per path / cooperative: 321 x 181 182 / 229, 1920 x 1080 353 / 579 at 8
+// bounces); paths of one bounce over full waves end too early for idle lanes to matter (1920 x 1080:
+// procedural 2,466 / 3,054, Worley 3,119 / 3,832, FP16 grid 3,064 / 3,469; the costlier lookups of
+// the first material 7,196 / 6,713, the voxel texture 366 / 382 but 104 / 81 at 640 x 360; 32 bounces
+// 1280 x 720 37,500 / 31,300).
+static bool lane_per_path(const PtArgs& a) {
+    if (a.mat.kind == SKYHIP_MATERIAL_MINIMAL) return true;
+    return a.max_bounces == 1 && a.coop_log_x + a.coop_log_y == 6 && a.mat.kind != SKYHIP_MATERIAL_DEFAULT0 &&
+           a.mat.kind != SKYHIP_MATERIAL_VOXEL;
 }
 
 // Without a brick grid (one majorant): every material.
-static void launch_single_majorant(hipStream_t st, const PtArgs& a, int cu_count, bool count) {
-    const dim3 grid(div_up(a.region[2] - a.region[0], 8), div_up(a.region[3] - a.region[1], 8));
+static void launch_single_majorant(hipStream_t st, PtArgs a, int cu_count, bool count) {
+    coop_tile(a, cu_count);
+    const bool lanes = lane_per_path(a);
+    const int w = a.region[2] - a.region[0], h = a.region[3] - a.region[1];
     auto with = [&](auto kind) {
         constexpr int kMat = decltype(kind)::value;
         if (count)
-            hipLaunchKernelGGL((path_trace_kernel<kMat, false, true, false, false>), grid, dim3(64), 0, st, a);
-        else
-            launch_coop<kMat>(st, a, cu_count);
+            hipLaunchKernelGGL((path_trace_kernel<kMat, false, true, false, false>), dim3(div_up(w, 8), div_up(h, 8)),
+                               dim3(64), 0, st, a);
+        else if (lanes)
+            hipLaunchKernelGGL((path_trace_kernel<kMat, false, false, false, false>), dim3(div_up(w, 8), div_up(h, 8)),
+                               dim3(64), 0, st, a);
+        else if constexpr (kMat != SKYHIP_MATERIAL_MINIMAL)
+            hipLaunchKernelGGL(path_trace_coop_kernel<kMat>,
+                               dim3(div_up(w, 1 << a.coop_log_x), div_up(h, 1 << a.coop_log_y)), dim3(64), 0, st, a);
     };
     switch (a.mat.kind) {
         case SKYHIP_MATERIAL_DEFAULT0: return with(std::integral_constant<int, SKYHIP_MATERIAL_DEFAULT0>());
