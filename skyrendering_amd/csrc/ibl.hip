@@ -189,6 +189,12 @@ struct PrefilterLevels {
 };
 
 constexpr int kPrefilterWaves = 8;
+// Whether a level of width wl is made by samples, a wave to a texel and a lane to a sample, rather than by tiles
+// of 64 texels: where few texels leave CUs idle, a sample at a time is a chain of lookups (into the fine
+// levels of the environment cube, the mip following the level's own texels).  us of the whole pass by samples
+// up to a width of 4 / 8 / 16: 128^2 environment, 16^2 of 5 levels 7.8 / 4.7 / 4.7 (tiles alone 9.8), 32^2 of 5
+// 7.8 / 7.0 / 5.1, 128^2 of 5 10.1 / 10.1 / 10.7; 1024^2 environment, 32^2 of 5 20.4 / 15.8 / 8.3.
+__host__ __device__ inline bool prefilter_by_samples(int wl, int pw) { return wl <= 8 || pw <= 32; }
 struct PrefilterSample {
     float x, y, z;  // direction in the texel's frame; z is also the weight
     float blend;    // of level + 1
@@ -240,6 +246,35 @@ __device__ __forceinline__ void prefilter_add(const ushort4* __restrict__ level,
     sum = fma3(f3(w3), rgba16f_rgb(d), sum);
 }
 
+// The face of direction L and the position on it (cube_face_st, without its branches).
+__device__ __forceinline__ int prefilter_face(F3 L, float& cs, float& ct) {
+    const float ax = fabsf(L.x), ay = fabsf(L.y), az = fabsf(L.z);
+    const bool mx = ax >= ay && ax >= az, my = !mx && ay >= az;
+    const float major = mx ? L.x : my ? L.y : L.z;
+    const bool neg = !(major >= 0.0f);
+    const float sc0 = mx ? -L.z : L.x, tc0 = my ? L.z : -L.y;
+    const float sc = neg && !my ? -sc0 : sc0, tc = neg && my ? -tc0 : tc0;
+    const float ma = fabsf(major);
+    float inv = __builtin_amdgcn_rcpf(ma);
+    inv = fmaf(fmaf(-ma, inv, 1.0f), inv, inv);
+    cs = fmaf(0.5f * sc, inv, 0.5f), ct = fmaf(0.5f * tc, inv, 0.5f);
+    return (mx ? 0 : my ? 2 : 4) + (neg ? 1 : 0);
+}
+// Adds sample (x, y, z) of the frame (t0, t1, N) at level l0 + blend, l0 + 1 <= log_ew where blend > 0.
+__device__ __forceinline__ void prefilter_lookup(const ushort4* __restrict__ env, int log_ew, F3 t0, F3 t1, F3 N, float x,
+                                                 float y, float z, int l0, float blend, F3& sum) {
+    float cs, ct;
+    const int face = prefilter_face(fma3(t0, f3(x), fma3(t1, f3(y), N * z)), cs, ct);
+    // Level l starts at 8 (w^2 - w_l^2) texels.
+    const int log0 = log_ew - l0;
+    const ushort4* base = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * log0)));
+    prefilter_add(base, log0, face, cs, ct, z * (1.0f - blend), sum);
+    if (blend > 0.0f) {  // so there is a level l0 + 1
+        const ushort4* next = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * (log0 - 1))));
+        prefilter_add(next, log0 - 1, face, cs, ct, z * blend, sum);
+    }
+}
+
 __global__ __launch_bounds__(64 * kPrefilterWaves) void prefilter_kernel(const ushort4* __restrict__ env, int log_ew,
                                                                          float4* __restrict__ sh9_out,
                                                                          ushort4* __restrict__ out, int pw,
@@ -274,23 +309,40 @@ __global__ __launch_bounds__(64 * kPrefilterWaves) void prefilter_kernel(const u
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // The workgroup's texels: 8 x 8 of a face, or 64 in a row where a face is smaller.
-    const long long p = (long long)tile * 64 + lane;
-    const bool texel = p < 6ll * wl * wl;
-    const int face = int(p / (wl * wl)), q = int(p % (wl * wl));
-    const int per_row = wl >> 3;
-    const int x = wl >= 8 ? ((q >> 6) % per_row) * 8 + (q & 7) : q % wl;
-    const int y = wl >= 8 ? ((q >> 6) / per_row) * 8 + ((q >> 3) & 7) : q / wl;
-    const F3 N = cube_texel_dir(min(face, 5), x, y, wl);
+    const float a = roughness * roughness, inv_sa_texel = (6.0f * float(wl) * float(wl)) / (4.0f * kPiF);
+    if (prefilter_by_samples(wl, pw)) {  // a wave is a texel, a lane its sample
+        const int p = tile * kPrefilterWaves + wave;
+        if (p >= 6 * wl * wl) return;  // wave-uniform
+        const F3 N = cube_texel_dir(p / (wl * wl), p % wl, (p / wl) % wl, wl);
+        F3 t0, t1, sum = f3(0.0f);
+        onb_frame(N, t0, t1);
+        PrefilterSample s;
+        const uint32_t n = uint32_t(lv.samples[level]);
+        float weight = 0.0f;
+        if (uint32_t(lane) < n && prefilter_sample(uint32_t(lane), n, a * a, inv_sa_texel, elevels, s)) {
+            prefilter_lookup(env, log_ew, t0, t1, N, s.x, s.y, s.z, s.level, s.blend, sum);
+            weight = s.z;
+        }
+        for (int m = 32; m >= 1; m >>= 1) {
+            sum = sum + F3{__shfl_xor(sum.x, m, 64), __shfl_xor(sum.y, m, 64), __shfl_xor(sum.z, m, 64)};
+            weight += __shfl_xor(weight, m, 64);
+        }
+        if (lane == 0) dst[p] = to_rgba16f(sum * (1.0f / weight), 0.0f);
+        return;
+    }
+    // The workgroup's texels: 8 x 8 of a face.
+    const long long p = (long long)tile * 64;
+    const int face = int(p / (wl * wl)), q = int(p % (wl * wl)) >> 6, per_row = wl >> 3;
+    const int x = (q % per_row) * 8 + (lane & 7), y = (q / per_row) * 8 + (lane >> 3);
+    const F3 N = cube_texel_dir(face, x, y, wl);
     F3 t0, t1;
     onb_frame(N, t0, t1);
     if (wave == 0) {
-        const float a = roughness * roughness;
         const uint32_t n = uint32_t(lv.samples[level]);
         PrefilterSample s;
         const bool up =
             uint32_t(lane) < n &&
-            prefilter_sample(uint32_t(lane), n, a * a, (6.0f * float(wl) * float(wl)) / (4.0f * kPiF), elevels, s);
+            prefilter_sample(uint32_t(lane), n, a * a, inv_sa_texel, elevels, s);
         const uint64_t mask = __ballot(up);
         if (up) s_sample[__popcll(mask & ((1ull << lane) - 1))] = s;
         float weight = up ? s.z : 0.0f;
@@ -303,32 +355,13 @@ __global__ __launch_bounds__(64 * kPrefilterWaves) void prefilter_kernel(const u
 #pragma unroll 2
     for (int k = wave; k < count; k += kPrefilterWaves) {
         const PrefilterSample s = s_sample[k];
-        const F3 L = fma3(t0, f3(s.x), fma3(t1, f3(s.y), N * s.z));
-        const float ax = fabsf(L.x), ay = fabsf(L.y), az = fabsf(L.z);
-        const bool mx = ax >= ay && ax >= az, my = !mx && ay >= az;  // cube_face_st, without its branches
-        const float major = mx ? L.x : my ? L.y : L.z;
-        const bool neg = !(major >= 0.0f);
-        const float sc0 = mx ? -L.z : L.x, tc0 = my ? L.z : -L.y;
-        const float sc = neg && !my ? -sc0 : sc0, tc = neg && my ? -tc0 : tc0;
-        const float ma = fabsf(major);
-        float inv = __builtin_amdgcn_rcpf(ma);
-        inv = fmaf(fmaf(-ma, inv, 1.0f), inv, inv);
-        const float cs = fmaf(0.5f * sc, inv, 0.5f), ct = fmaf(0.5f * tc, inv, 0.5f);
-        const int cface = (mx ? 0 : my ? 2 : 4) + (neg ? 1 : 0);
         const int l0 = __builtin_amdgcn_readfirstlane(s.level);
         const float blend = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.blend)));
-        // Level l starts at 8 (w^2 - w_l^2) texels.
-        const int log0 = log_ew - l0;
-        const ushort4* base = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * log0)));
-        prefilter_add(base, log0, cface, cs, ct, s.z * (1.0f - blend), sum);
-        if (blend > 0.0f) {  // so there is a level l0 + 1
-            const ushort4* next = env + 8ll * ((1ll << (2 * log_ew)) - (1ll << (2 * (log0 - 1))));
-            prefilter_add(next, log0 - 1, cface, cs, ct, s.z * blend, sum);
-        }
+        prefilter_lookup(env, log_ew, t0, t1, N, s.x, s.y, s.z, l0, blend, sum);
     }
     s_sum[threadIdx.x] = sum;
     __syncthreads();
-    if (wave != 0 || !texel) return;
+    if (wave != 0) return;
 #pragma unroll
     for (int v = 1; v < kPrefilterWaves; ++v) sum = sum + s_sum[64 * v + lane];
     dst[(long long)face * wl * wl + y * wl + x] = to_rgba16f(sum * (1.0f / s_weight), 0.0f);
@@ -403,7 +436,7 @@ extern "C" int skyhip_ibl_precompute(SkyhipContext* ctx, const void* environment
         const float p = std::pow(lv.roughness[l], 0.3f);
         lv.samples[l] = std::min(std::max(int(uint32_t(1.0f * (1.0f - p) + 64.0f * p)), 1), 64);
         lv.block_start[l] = int(blocks);
-        blocks += div_up(6LL * wl * wl, lv.roughness[l] == 0.0f ? 64 * kPrefilterWaves : 64);
+        blocks += div_up(6LL * wl * wl, lv.roughness[l] == 0.0f ? 64 * kPrefilterWaves : prefilter_by_samples(wl, prefiltered_width) ? kPrefilterWaves : 64);
     }
     lv.block_start[roughness_count] = int(blocks);
     hipLaunchKernelGGL(prefilter_kernel, dim3(unsigned(kSh9Blocks + blocks)), dim3(64 * kPrefilterWaves), 0, ctx->stream,
