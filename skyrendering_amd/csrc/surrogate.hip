@@ -792,7 +792,7 @@ __global__ __launch_bounds__(256, 2) void sky_render_surrogate_kernel(const floa
 // Residual check: probes at the 4 quarter points of each 16 x 16 tile; a tile whose
 // largest |surrogate - plain| / max(plain, floor) exceeds the tolerance is flagged.  One
 // thread per probe: the 4 probes of a tile are 4 adjacent lanes, reduced with shuffles.  (For LUTs too
-// wide for sky_check_rows_kernel; four waves per SIMD as sky_radiance_kernel.)
+// wide for sky_check_rows_kernel and short marches; four waves per SIMD as sky_radiance_kernel.)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void sky_render_check_kernel(
     SkyRenderArgs a, int view_count) {
     const long long tiles_per_view = (long long)a.tiles_x * a.tiles_y;
@@ -898,6 +898,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     if (rows[row].ray.dist > 0.0f)
         L = (rayleigh_phase(nu) * Sr + mie_phase(A.g, nu) * Sm + A.ms_mask * Sx) * A.solar;
     a.out[(long long)view * a.width * a.height + (long long)y * a.width + x] = make_float4(L.x, L.y, L.z, 0.0f);
+}
+
+// The plain pass by pixels (sky_radiance_kernel's march), for marches too short to share: a tile evaluates 32
+// steps of its rows whatever their number.  us by pixels / by tiles, 8 views of 960 x 540: 1 step 49 / 98, 4
+// 97 / 134, 11 209 / 213, 12 226 / 224, 30 518 / 441; with the network and no tile flagged, the check by
+// probes / by rows, 1 step 187 / 191, 11 192.8 / 194.7.
+constexpr int kSharedSteps = 12;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void sky_render_pixels_kernel(SkyRenderArgs a,
+                                                                                                           int all_tiles) {
+    const int tile = blockIdx.x, view = blockIdx.y;
+    if (!all_tiles && a.flags[(long long)view * a.tiles_x * a.tiles_y + tile] == 0u) return;  // workgroup-uniform
+    const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+    const int x = tx * kTile + int(threadIdx.x & 15), y = ty * kTile + int(threadIdx.x >> 4);
+    if (x >= a.width || y >= a.height) return;
+    const F3 L = sky_radiance_q(a.luts, panorama_query(a.views[view], x, y, a.width, a.height));
+    a.out[(long long)view * a.width * a.height + (long long)y * a.width + x] = make_float4(L.x, L.y, L.z, 0.0f);
+}
+void launch_plain(hipStream_t st, const SkyRenderArgs& a, int view_count, int all_tiles) {
+    const dim3 grid(a.tiles_x * a.tiles_y, view_count);
+    if (row_step_count(a.luts.steps) < kSharedSteps)
+        hipLaunchKernelGGL(sky_render_pixels_kernel, grid, dim3(256), 0, st, a, all_tiles);
+    else
+        hipLaunchKernelGGL(sky_render_plain_kernel, grid, dim3(256), 0, st, a, all_tiles);
 }
 
 // ---------------------------------------------------------------------------
@@ -1272,7 +1295,7 @@ extern "C" int skyhip_sky_render_surrogate(SkyhipContext* ctx, int32_t network, 
     else
         hipLaunchKernelGGL(sky_render_surrogate_kernel<NetBF16SiLU>, dim3(blocks), dim3(256), 0, st, params, a,
                            view_count);
-    if (row_luts_fit(a.luts.tw, a.luts.mw)) {
+    if (row_luts_fit(a.luts.tw, a.luts.mw) && row_step_count(a.luts.steps) >= kSharedSteps) {
         const int parts = int(div_up(a.tiles_x, kCheckTiles));
         hipLaunchKernelGGL(sky_check_rows_kernel, dim3(a.tiles_y * parts, view_count), dim3(64 * kCheckWaves), 0, st, a,
                            parts);
@@ -1281,7 +1304,7 @@ extern "C" int skyhip_sky_render_surrogate(SkyhipContext* ctx, int32_t network, 
         hipLaunchKernelGGL(sky_render_check_kernel, dim3(unsigned((probes + 255) / 256)), dim3(256), 0, st, a,
                            view_count);
     }
-    hipLaunchKernelGGL(sky_render_plain_kernel, dim3(a.tiles_x * a.tiles_y, view_count), dim3(256), 0, st, a, 0);
+    launch_plain(st, a, view_count, 0);
     SKYHIP_LAUNCH_CHECK("sky render (surrogate)");
     return SKYHIP_OK;
 }
@@ -1294,8 +1317,7 @@ extern "C" int skyhip_sky_render_plain(SkyhipContext* ctx, const SkyhipSkyLuts* 
                              &dummy_counter, 1.0f, 1.0f, a));
     a.flags = nullptr;
     a.counters = nullptr;
-    hipLaunchKernelGGL(sky_render_plain_kernel, dim3(a.tiles_x * a.tiles_y, view_count), dim3(256), 0, ctx->stream, a,
-                       1);
+    launch_plain(ctx->stream, a, view_count, 1);
     SKYHIP_LAUNCH_CHECK("sky_render_plain_kernel");
     return SKYHIP_OK;
 }
