@@ -792,7 +792,7 @@ __global__ __launch_bounds__(256, 2) void sky_render_surrogate_kernel(const floa
 // Residual check: probes at the 4 quarter points of each 16 x 16 tile; a tile whose
 // largest |surrogate - plain| / max(plain, floor) exceeds the tolerance is flagged.  One
 // thread per probe: the 4 probes of a tile are 4 adjacent lanes, reduced with shuffles.  (For LUTs too
-// wide for sky_check_rows_kernel and short marches; four waves per SIMD as sky_radiance_kernel.)
+// wide for sky_check_rows_kernel, short marches and few probes; four waves per SIMD as sky_radiance_kernel.)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void sky_render_check_kernel(
     SkyRenderArgs a, int view_count) {
     const long long tiles_per_view = (long long)a.tiles_x * a.tiles_y;
@@ -942,11 +942,15 @@ __device__ __forceinline__ void panorama_scatter(const Atm& atm, const SkyLuts& 
                    lds, L, Tr);
 }
 
+// A row near the horizon reaches many columns of the LUTs at every step, and its wave blends them one step
+// after the other, which only many rows hide.  us with the network pass, by probes / by rows: 320 x 180
+// 34 / 61, 1920 x 1080 122 / 150, 4 of them 357 / 380, 8 (261,120 probes) 684 / 691, 16 1,349 / 1,320.
+constexpr long long kMinRowProbes = 1 << 18;
 constexpr int kCheckWaves = 4, kCheckRays = 2;
 constexpr int kCheckTiles = kCheckWaves * kCheckRays * 64 / 4;  // their probes are one march of every wave
 // The residual check of a tile row of view blockIdx.y, or of one of its `parts` of up to kCheckTiles tiles
-// (2,048 pixels; with the network pass an image of 16,384 x 16 takes 47.6 us, 143.6 with a row of tiles in
-// one workgroup, 67.6 with a thread per probe): the tiles' probes lie in two pixel rows.
+// (2,048 pixels; by rows an image of 16,384 x 16 took 47.6 us with the network pass, 143.6 with a row of tiles in
+// one workgroup): the tiles' probes lie in two pixel rows.
 // Four waves of two rays a lane take 1920 wide's 2 x 240 probes at once; 16 such views with the network
 // pass 1,364 us, 1,426 with every probe marching for itself (2 waves of four rays 1,367, of one 1,405).
 __global__ __launch_bounds__(64 * kCheckWaves) __attribute__((amdgpu_waves_per_eu(3))) void sky_check_rows_kernel(
@@ -1295,12 +1299,12 @@ extern "C" int skyhip_sky_render_surrogate(SkyhipContext* ctx, int32_t network, 
     else
         hipLaunchKernelGGL(sky_render_surrogate_kernel<NetBF16SiLU>, dim3(blocks), dim3(256), 0, st, params, a,
                            view_count);
-    if (row_luts_fit(a.luts.tw, a.luts.mw) && row_step_count(a.luts.steps) >= kSharedSteps) {
+    const long long probes = 4LL * a.tiles_x * a.tiles_y * view_count;
+    if (row_luts_fit(a.luts.tw, a.luts.mw) && row_step_count(a.luts.steps) >= kSharedSteps && probes >= kMinRowProbes) {
         const int parts = int(div_up(a.tiles_x, kCheckTiles));
         hipLaunchKernelGGL(sky_check_rows_kernel, dim3(a.tiles_y * parts, view_count), dim3(64 * kCheckWaves), 0, st, a,
                            parts);
     } else {
-        const long long probes = 4LL * a.tiles_x * a.tiles_y * view_count;
         hipLaunchKernelGGL(sky_render_check_kernel, dim3(unsigned((probes + 255) / 256)), dim3(256), 0, st, a,
                            view_count);
     }
