@@ -427,38 +427,50 @@ struct MsTotals {                // per polar angle: transmittance, multiple-sca
 // The zenith cosine of polar angle t (ms_ray's, for lanes 8 t .. 8 t + 7).
 __device__ __forceinline__ float ms_cos_theta(int t) { return 1.0f - 2.0f * ((0.5f + float(t)) / 8.0f); }
 
+// The march of one polar angle, by half a wave.
+struct MsMarch {
+    RowRay ray;
+    bool hit;
+    F3 tr, lf;  // so far
+};
+__device__ inline MsMarch ms_march(const AtmDev& A, int iy, int h, int theta) {
+    const float alt0 = (float(iy) / float(h - 1)) * A.thickness, r = alt0 + A.rb, mu = ms_cos_theta(theta);
+    const bool hit = ray_hits_ground(A, r, alt0, mu);
+    // mu_s at a step is a0 mu_s0 + a1 nu: r_mu_s0 stands for r alone.
+    return {RowRay{r, alt0, mu, hit ? distance_to_bottom(A, r, alt0, mu) : distance_to_top(A, r, alt0, mu), r, 0.0f}, hit,
+            f3(1.0f), f3(0.0f)};
+}
+// Steps [first, last) of its n, into row[0] onwards.
+__device__ inline void ms_march_steps(const AtmDev& A, MsMarch& m, int n, int first, int last, int tw, int th, MsStep* row) {
+    const float iso = 1.0f / (4.0f * kPiF), dx = m.ray.dist / A.ms_steps;
+    for (int f = first; f < last; f += kRowSteps) {
+        const RowStep s = row_step(A, m.ray, dx, n, f, tw, th, 2, m.tr);
+        const int j = f + int(threadIdx.x & 31);
+        const F3 ws = s.wr + s.wm;
+        F3 sum = j < n ? ws : f3(0.0f);
+        for (int off = 16; off >= 1; off >>= 1)
+            sum = sum + F3{__shfl_xor(sum.x, off, 32), __shfl_xor(sum.y, off, 32), __shfl_xor(sum.z, off, 32)};
+        m.lf += sum;
+        if (j < n) {
+            MsStep& d = row[j - first];
+            d.c[0] = make_float4(s.a0, s.a1, s.r2, s.h2q);
+            d.c[1] = make_float4(s.r, s.d_min, s.kx, s.fade_c);
+            d.c[2] = make_float4(ws.x * iso, ws.y * iso, ws.z * iso, s.fade_k);
+            d.c[3] = make_float4(s.ty, 0.0f, 0.0f, 0.0f);
+        }
+    }
+}
+__device__ __forceinline__ MsTotals ms_totals(const MsMarch& m) { return {m.tr, m.lf, m.ray.r, m.ray.dist, m.hit}; }
+
 // Fills `steps` (kMsThetas x n) and `totals` for the altitude of row iy: one (angle, step) per thread.
 // Every thread of the workgroup calls it; the caller synchronises.
 __device__ inline void ms_row_tables(const AtmDev& A, int iy, int h, int tw, int th, int n, MsStep* steps,
                                      MsTotals* totals) {
-    const float alt0 = (float(iy) / float(h - 1)) * A.thickness, r = alt0 + A.rb;
-    const float iso = 1.0f / (4.0f * kPiF);
     for (int e = threadIdx.x; e < kMsThetas * kRowSteps; e += blockDim.x) {  // half a wave per angle
         const int t = e / kRowSteps;
-        const float mu = ms_cos_theta(t);
-        const bool hit = ray_hits_ground(A, r, alt0, mu);
-        // mu_s at a step is a0 mu_s0 + a1 nu: r_mu_s0 stands for r alone.
-        const RowRay ray{r, alt0, mu, hit ? distance_to_bottom(A, r, alt0, mu) : distance_to_top(A, r, alt0, mu), r,
-                         0.0f};
-        const float dx = ray.dist / A.ms_steps;
-        F3 tr = f3(1.0f), lf = f3(0.0f);
-        for (int first = 0; first < n; first += kRowSteps) {
-            const RowStep s = row_step(A, ray, dx, n, first, tw, th, 2, tr);
-            const int j = first + (e & 31);
-            const F3 ws = s.wr + s.wm;
-            F3 sum = j < n ? ws : f3(0.0f);
-            for (int off = 16; off >= 1; off >>= 1)
-                sum = sum + F3{__shfl_xor(sum.x, off, 32), __shfl_xor(sum.y, off, 32), __shfl_xor(sum.z, off, 32)};
-            lf += sum;
-            if (j < n) {
-                MsStep& d = steps[t * n + j];
-                d.c[0] = make_float4(s.a0, s.a1, s.r2, s.h2q);
-                d.c[1] = make_float4(s.r, s.d_min, s.kx, s.fade_c);
-                d.c[2] = make_float4(ws.x * iso, ws.y * iso, ws.z * iso, s.fade_k);
-                d.c[3] = make_float4(s.ty, 0.0f, 0.0f, 0.0f);
-            }
-        }
-        if ((e & 31) == 0) totals[t] = {tr, lf, r, ray.dist, hit};
+        MsMarch m = ms_march(A, iy, h, t);
+        ms_march_steps(A, m, n, 0, n, tw, th, steps + t * n);
+        if ((e & 31) == 0) totals[t] = ms_totals(m);
     }
 }
 
