@@ -35,7 +35,8 @@ class LutSet:
         self.render_block = None
 
     def build(self, atmosphere: AtmosphereParameters, render: AtmosphereRenderParameters):
-        key = id(atmosphere)
+        # By value: a caller may change the object between frames, or drop it.
+        key = tuple(tuple(v) if isinstance(v, list) else v for v in vars(atmosphere).values())
         if key != self._atm_key:
             self.atm_block = atmosphere.buffer_data()
             self._atm_key = key
