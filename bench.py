@@ -42,23 +42,21 @@ HBM_PEAK_GBS = 8000.0
 # profiles/lut_batch_256x8.md): SQ_INSTS_VALU_FLOPS_FP32 + SQ_INSTS_VALU_FLOPS_FP32_TRANS count
 # operations per wave instruction (an FMA counts 2), so the lane operations are 64 times that,
 # scaled by the measured lane utilisation SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU), then
-# divided by the executed sample-steps (raymarch: 7.3665e9 over 35,111,907) or integrator steps
-# (LUT set, counted on the one-lane-per-texel kernels so that the split kernels' repeated ray
-# set-up is not counted as work: 1.0386e9 over 4,914,688; batch: 7.184e11 over 3,024,532,480)
-# of the same launches.  The LUT set's, the batch's and the environment's are the operations of the
-# texel-by-texel, sample-by-sample forms: the kernels share a row's steps and a level's samples since
-# and execute fewer, so their rates are equivalent ones.
+# divided by the sample-steps (raymarch: 7.3665e9 over 35,111,907) or integrator steps (LUT set:
+# 7.651e8 over 4,914,688; batch: 1.5757e11 over 3,024,532,480) of the same launches.  A step is one
+# ray's; the batch's rows and the multiple-scattering tables evaluate most of it once for many rays,
+# so their operations per step are few, and the figures are what is executed.
 RAYMARCH_KERNEL = "cloud_raymarch_kernel<5,false>"
 RAYMARCH_FP32_FLOP_PER_STEP = 209.8
-LUT_SET_FLOP_PER_STEP = 211.3
-BATCH_FLOP_PER_STEP = 237.5
+LUT_SET_FLOP_PER_STEP = 155.7
+BATCH_FLOP_PER_STEP = 52.1
 # The cloud shadow frame (map, two blur passes, froxel) and the environment update (cube, mips,
 # SH9, five prefiltered levels) of this bench's workloads: FP32 operations (the SQ counters as
 # above) and calibrated HBM bytes, summed over their launches (profiles/cloud_shadow_environment.md).
-SHADOW_FP32_FLOP_PER_FRAME = 4.472e8
-SHADOW_HBM_BYTES_PER_FRAME = 56.6e6
-ENV_FP32_FLOP_PER_UPDATE = 7.10e8
-ENV_HBM_BYTES_PER_UPDATE = 8.34e6
+SHADOW_FP32_FLOP_PER_FRAME = 4.657e8
+SHADOW_HBM_BYTES_PER_FRAME = 56.2e6
+ENV_FP32_FLOP_PER_UPDATE = 2.279e8
+ENV_HBM_BYTES_PER_UPDATE = 6.66e6
 
 # HBM traffic per launch, from `rocprofv3 --pmc FETCH_SIZE` and `--pmc WRITE_SIZE` runs of this
 # bench (KiB per dispatch), each divided by what the same counter reads per KiB moved by a
@@ -295,7 +293,7 @@ def bench_environment(ctx, reps=20):
                         "frac": round(ENV_FP32_FLOP_PER_UPDATE / (ms * 1e-3) / 1e12 / FP32_PEAK_TFLOPS, 4),
                         "traffic": int(ENV_HBM_BYTES_PER_UPDATE),
                         "traffic_gbs": round(ENV_HBM_BYTES_PER_UPDATE / (ms * 1e-3) / 1e9, 1),
-                        "note": "latency-bound chain of 3 launches (SH9 and the prefilter's five levels take 40 µs of it); "
+                        "note": "latency-bound chain of 3 launches (SH9 and the prefilter's five levels take half of it); "
                                 "FP32 operations and HBM bytes measured per update with rocprofv3 counters"}}
     import oracle
     sv_l, sv_t = rend.sky_view()
@@ -577,6 +575,8 @@ def bench_surrogate(ctx, epochs=2400, width=1920, height=1080, n_views=64, cpu_s
     out["lut_ms"] = round(timed(pano.render_lut), 3)
     out["lut_build_ms"] = round(timed(eatm.batch.launch), 3)
     out["speedup_vs_plain"] = round(out["plain_ms"] / out["surrogate_ms"], 3)
+    out["speedup_note"] = ("against render_plain's 16 x 16 tiles; by 64-column row pieces, which the library does not "
+                           "use, 8 views of 960 x 540 took 0.128 ms, the tiles 0.506, the network 0.346")
     samples = width * height * n_views
     achieved = samples * SURROGATE_FLOP_PER_SAMPLE / (out["network_pass_ms"] * 1e-3) / 1e12
     out["roofline"] = {"bound": "mfma", "unit": "TFLOP/s", "kernel": "sky_render_surrogate_kernel (+ probe check)",

@@ -1,9 +1,11 @@
 // Atmosphere LUT kernels for gfx950: transmittance, multiple scattering,
 // sky view and aerial perspective, plus their C-ABI entry points.
 //
-// Layout: every LUT is RGBA32F in GL texel order, one lane per texel (one
-// wave64 per texel for multiple scattering, whose 64 sphere directions map to
-// the 64 lanes), 256-lane workgroups, 1D grids over texels so stores coalesce.
+// Layout: every LUT is RGBA32F in GL texel order, neighbouring lanes at neighbouring texels so that
+// stores coalesce.  Transmittance is a lane per texel, four in the one-call set; multiple scattering a
+// wave64 per texel (its 64 sphere directions are the lanes), four waves in the set; the sky view a lane
+// per texel over its row's shared steps (sky_rows.h), or marching for itself with dither or wide LUTs,
+// two waves to 64 texels in the set; aerial perspective four waves to 64 froxels.
 #include "sky_rows.h"
 
 #include <algorithm>
@@ -310,7 +312,9 @@ int launch_sky_view(hipStream_t st, const SkyhipAtmosphereBufferData& b, const S
                     const float* T, int tw, int th, const float* MS, int mw, int mh, const uint16_t* bn, int bn_size,
                     float* L, float* Tr, int w, int h) {
     // Rows share their march unless the dither starts every texel's elsewhere, or the LUTs are wider
-    // than a wave's entries.  128 x 128, 30 steps: 12.7 us by rows, 31.6 texel by texel.
+    // than a wave's entries.  128 x 128, 30 steps: 12.7 us by rows, 31.6 texel by texel with the longer
+    // step and 18 with scatter_step (256 + 32 columns 13.1 against 257 + 32 18.3; 2048 x 1024 132 and
+    // 268).
     if (bn == nullptr && row_luts_fit(tw, mw)) {
         hipLaunchKernelGGL(sky_view_rows_kernel, dim3(div_up(w, 64), h), dim3(64), 0, st, b, r,
                            reinterpret_cast<const float4*>(T), tw, th, reinterpret_cast<const float4*>(MS), mw, mh,

@@ -144,6 +144,9 @@ __global__ __launch_bounds__(64 * kWaves) void batch_multiscattering_kernel(
 // every texel marching for itself; three rays per lane against six 2.9 / 4.3 ms (six leave two waves
 // a SIMD), runs of steps of one kind against a three-way branch per step 3.0 / 3.9 ms (the branch's
 // joins copy the sums), tiles of 4,096 texels against 1,024 2.8 / 3.0 ms (rows set up a lane each).
+// Workgroups of 256 take 45 KB of LDS, so three fit a CU (159 VGPRs); smaller ones reach four waves a SIMD
+// with 128 VGPRs and some spilled.  LUTs of more than 288 columns: 64 sets of 512 x 64 with 8 views each 1.93 ms,
+// 2.50 before rows, with cell-corner copies of both LUTs; of 256 x 64 0.97 / 2.38 ms.
 template <int kBlock>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void batch_sky_view_kernel(
     const SkyhipAtmosphereBufferData* __restrict__ atm, const SkyhipAtmosphereRenderBufferData* __restrict__ renders,

@@ -1,11 +1,11 @@
-// Per-texel bodies of the four atmosphere LUT passes, shared by the single-set
-// kernels (atmosphere.hip) and the batched builder (batch.hip), so a batch item
-// runs exactly the single-set arithmetic.
+// Per-texel bodies of the four atmosphere LUT passes, shared with sky_rows.h by the per-pass
+// kernels (atmosphere.hip) and the batched builder (batch.hip), so a batch item runs exactly the
+// per-pass arithmetic.
 //
 //   transmittance_texel   Atmosphere.glsl:71-88, :311-337 (FP32, or FP64 near the horizon)
 //   multiscattering_texel Atmosphere.glsl:344-438, one wave64 per texel
 //   sky_view_texel        AtmosphereRenderer.glsl:56-186
-//   aerial_ray            AtmosphereRenderer.glsl:191-243 (set-up; the integration is split over lanes)
+//   aerial_ray            AtmosphereRenderer.glsl:191-243 (set-up; the integration is split over waves)
 #pragma once
 
 #include "atmosphere_device.h"

@@ -841,8 +841,9 @@ __device__ __forceinline__ float panorama_nu(const PanoramaRow& r, int x, int w)
 // Plain pass: every pixel of flagged tiles (or of all tiles when all_tiles is set).  A workgroup is a
 // 16 x 16 tile; its 16 rows' steps are set up in LDS, 32 at a time, half a wave a row, and every
 // thread marches its pixel over its row's.  Bound by the texture addressing of the 8 texels a step
-// reads (12 bytes each).  8 views of 1920 x 1080: 1,722 us, 2,813 with every pixel evaluating its own
-// densities and exponentials.
+// reads (12 bytes each), and its 41 KB of LDS leave three workgroups to a CU.  8 views of 1920 x 1080:
+// 1,722 us, 2,813 with every pixel evaluating its own densities and exponentials.  (Whole row pieces of
+// 64 columns by row_scatter, not used here, took 0.128 ms for 8 views of 960 x 540, the tiles 0.506.)
 constexpr int kTile = 16;
 struct TileStep {
     float4 c[4];
