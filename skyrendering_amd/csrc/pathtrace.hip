@@ -793,7 +793,8 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
                                                  float t1, float& t) {
     bool on = track && a.sigma_t_max > 0.0f, hit = false;
     t = t0;
-    int it = 0, ahead = 4;  // draws ahead, doubled while flights go on (those past a collision are wasted)
+    int steps = kMaxTrackingSteps;  // left
+    int ahead = 4;  // draws ahead, doubled while flights go on (those past a collision are wasted)
     for (;;) {
         const unsigned long long m = __ballot(on);
         if (m == 0ull) return hit;
@@ -807,7 +808,7 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
                 } else {
                     const float sg = sigma_at<kMat>(a, o + d * t);
                     hit = rng.next() < sg * a.inv_sigma_t_max;
-                    on = !hit && ++it < kMaxTrackingSteps;
+                    on = !hit && --steps > 0;
                 }
             }
             continue;
@@ -835,8 +836,7 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
         const unsigned long long hits = __ballot(taken);
         if (on) {
             const unsigned long long mine = (hits >> (K * rank)) & (K == 64 ? ~0ull : (1ull << K) - 1ull);
-            const int left_steps = kMaxTrackingSteps - it;  // draws past the limit do not count
-            if (mine != 0ull && __builtin_ctzll(mine) < left_steps) {
+            if (mine != 0ull && __builtin_ctzll(mine) < steps) {  // draws past the limit do not count
                 const int j = K * rank + __builtin_ctzll(mine);
                 t = s.t[j];
                 rng.s = s.state[j];
@@ -844,12 +844,9 @@ __device__ __forceinline__ bool coop_delta_track(const PtArgs& a, CoopLds& s, bo
                 on = false;
             } else {
                 t = tt;
-                it += n;
-                on = !left;
-                if (n >= left_steps) {
-                    rng.s = s.state[K * rank + left_steps - 1];
-                    on = false;
-                }
+                if (n >= steps) rng.s = s.state[K * rank + steps - 1];
+                steps -= n;
+                on = !left && steps > 0;
             }
         }
     }
@@ -861,7 +858,7 @@ __device__ __forceinline__ float coop_ratio_track(const PtArgs& a, CoopLds& s, b
     float t = 0.0f, t1 = 0.0f, tr = 1.0f;
     if (track) region(a, o, d, t, t1);
     bool on = track && t < t1;
-    int it = 0;
+    int steps = kMaxTrackingSteps;
     for (;;) {
         const unsigned long long m = __ballot(on);
         if (m == 0ull) return clamp01(tr);
@@ -873,7 +870,7 @@ __device__ __forceinline__ float coop_ratio_track(const PtArgs& a, CoopLds& s, b
                     on = false;
                 } else {
                     tr *= 1.0f - fmaxf(0.0f, sigma_at<kMat>(a, o + d * t) * a.inv_sigma_t_max);
-                    on = ++it < kMaxTrackingSteps;
+                    on = --steps > 0;
                 }
             }
             continue;
@@ -895,10 +892,10 @@ __device__ __forceinline__ float coop_ratio_track(const PtArgs& a, CoopLds& s, b
         s.sigma[threadIdx.x] = coop_lookup<kMat>(a, s, tracking, K);
         wave_lds_fence();
         if (on) {
-            n = min(n, kMaxTrackingSteps - it);  // draws past the limit do not count
+            n = min(n, steps);  // draws past the limit do not count
             for (int j = 0; j < n; ++j) tr *= 1.0f - fmaxf(0.0f, s.sigma[K * rank + j] * a.inv_sigma_t_max);
-            it += n;
-            on = !left && it < kMaxTrackingSteps;
+            steps -= n;
+            on = !left && steps > 0;
         }
     }
 }
