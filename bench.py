@@ -68,8 +68,8 @@ FETCH_COUNTS_PER_KIB = 0.5
 WRITE_COUNTS_PER_KIB = 1.0
 PROFILED_KIB = {  # kernel: (FETCH_SIZE, WRITE_SIZE) in KiB per dispatch, mean over the profiled launches
     "cloud_raymarch_kernel<5,false>": (36040.0, 25686.0),
-    "path_trace_kernel<4,true,false,true,true>": (4.5146e6, 2.8026e4),
-    "path_trace_kernel<4,true,false,true,true> at 8^3 bricks": (3.4176e6, 2.8265e4),
+    "path_trace_kernel<4,true,false,true,true>": (4.567e6, 2.536e4),
+    "path_trace_kernel<4,true,false,true,true> at 8^3 bricks": (3.4605e6, 2.5465e4),
 }
 
 

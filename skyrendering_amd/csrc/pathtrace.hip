@@ -631,7 +631,7 @@ __device__ __forceinline__ float4 add_sample(const PtArgs& a, float u, float v, 
 // the tracking's fetch latency.  Measured on the 1024^2 brick-majorant workload at 16^3 (ms per frame,
 // one box): 5 waves 6.17-6.19, 6 waves 5.89-5.97, 7 waves (15 VGPRs spilled) 5.96-6.11, 8 waves (33)
 // 6.71-6.73; 6.33-6.37 with 5 waves while collisions and ground hits called the shadow ray's tracking
-// separately (lanes with either waited for the other's); over four clouds 1.02 to 1.14 times faster than that.
+// separately (lanes with either waited for the other's); over four clouds 1.01 to 1.14 times faster than that.
 // Every variant gives the same image.
 template <int kMat, bool kBricks, bool kCount, bool kCells, bool kFlat>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void path_trace_kernel(PtArgs a) {
